@@ -69,7 +69,8 @@ SL_FLOP_PER_PAIR = 28      # src/CPUKernels.cc:1008
 FAR32_TRAFFIC = {(3.0, 6.0): (2.0 * 389723.9 * 1024 + 52224.0 * 1024,
                               "profiles/k_far_groups_f32c_hbm_counters_512ves_p16.md")}
 FAR_KINDS = {"lds": 0, "scalar": 1, "scalar2": 2}
-FAR32_NAMES = {"lds": "k_far_f32c<SL>", "scalar": "k_far_groups_f32c", "scalar2": "k_far_groups_f32c2"}
+FAR32_NAMES = {"lds": "k_pairs_f32c<SL>", "scalar": "k_far_groups_f32c",
+               "scalar2": "k_far_groups_f32c"}
 DL_FLOP_PER_PAIR = 31      # src/PVFMMInterface.cc:365 (no Newton steps)
 
 
@@ -293,7 +294,7 @@ def bench_step(args):
             "flop_per_launch": flop, "pairs_per_launch": pairs,
             "two_density_pass_ms": (sum(s["ms_far2"] for s in learned_t)
                                     / max(1, sum(s["far2_calls"] for s in learned_t))),
-            "fp64_form": {"kernel": "k_far_f64<SL>" if args.far_kernel == "lds" else "k_far_groups_f64",
+            "fp64_form": {"kernel": "k_pairs_f64<SL>" if args.far_kernel == "lds" else "k_far_groups_f64",
                           "kernel_ms": far_ms_plain, "pairs_per_launch": pairs_plain,
                           "achieved": pairs_plain * SL_FLOP_PER_PAIR / (far_ms_plain * 1e-3) / 1e12,
                           "peak": PEAK_FP64_TFLOPS}}

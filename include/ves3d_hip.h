@@ -146,11 +146,10 @@ int ves3d_hip_set_gemm_tile(int tile);
 int ves3d_hip_valu_probe(int fp64, double *lane_fma_per_s);
 
 /* Selects the kernel of the far field between vesicles inside the implicit
- * step (StokesVelocity's PVFMMEval call, src/StokesVelocity.cc:481-485):
- * 0 = sources staged through LDS tiles, 1 = sources read through the scalar
- * cache (the default), 2 = as 1 with two targets per lane in the FP32 form.
- * All give the same sums up to rounding order.  No counterpart in the
- * reference. */
+ * step (StokesVelocity's PVFMMEval call, src/StokesVelocity.cc:481-485),
+ * where it has one source level: 0 = the kernels of the all-pairs entry
+ * points, 1 (the default) and 2 = the kernel of the source levels.  All give
+ * the same sums up to rounding order.  No counterpart in the reference. */
 int ves3d_hip_set_far_kernel(int kind);
 
 /* ---- direct Stokes sums ------------------------------------------------ */

@@ -151,6 +151,46 @@ def test_direct_eval_separate_targets(hip, orc):
     assert _relerr(out.cpu().numpy(), ref) < 1e-12
 
 
+@pytest.mark.parametrize("sl,dl", [(True, False), (False, True), (True, True)])
+@pytest.mark.parametrize("ns,nt,spg", [
+    (1, 1, 0), (31, 65, 0), (33, 64, 0), (256, 63, 0), (257, 1, 0), (3001, 700, 0),
+    (64, 64, 32), (2 * 257, 2 * 65, 257), (7 * 84, 7 * 40, 84), (1300, 132000, 0)])
+def test_direct_eval_split_edges(hip, orc, sl, dl, ns, nt, spg):
+    """Around the slices' edges: parts of 32 sources, tiles of 256, waves of
+    64 targets that span groups, shared and unshared target waves, a
+    coincident point in the last run, and targets with no partner at all.
+    FP64 sums of at most 3001 terms in another order: 1e-12 of the largest.
+    The mixed form rounds each term to 24 bits: 2e-5 on random clouds."""
+    rng = np.random.default_rng(ns + nt)
+    pos = rng.uniform(-1, 1, (ns, 3))
+    f, q = rng.uniform(-1, 1, (ns, 3)), rng.uniform(-1, 1, (ns, 6))
+    trg = rng.uniform(-1, 1, (nt, 3))
+    # keep random pairs apart (single terms would dominate the FP32 bound)
+    trg += 3.0 * np.sign(trg)
+    tpg = nt // (ns // spg) if spg else 0
+    if not spg:
+        trg[-1] = pos[-1]  # skipped: r = 0
+    a_sl, a_dl = (f if sl else None), (q if dl else None)
+    pick = np.unique(np.concatenate([np.arange(min(nt, 70)), [nt // 2, nt - 1]]))
+    ref = np.zeros((nt, 3))
+    if nt < 5000:
+        orc.orc_far_field(OL.p(pos), OL.p(a_sl), OL.p(a_dl), OL.cs(ns), OL.p(trg), OL.p(ref),
+                          OL.cs(nt), OL.cs(spg), OL.cs(tpg))
+        pick = np.arange(nt)
+    else:
+        sub, rs = np.ascontiguousarray(trg[pick]), np.zeros((pick.size, 3))
+        orc.orc_far_field(OL.p(pos), OL.p(a_sl), OL.p(a_dl), OL.cs(ns), OL.p(sub), OL.p(rs),
+                          OL.cs(pick.size), OL.cs(0), OL.cs(0))
+        ref[pick] = rs
+    for mixed, tol in ((False, 1e-12), (True, 2e-5)):
+        out = torch.full((nt, 3), np.nan, dtype=torch.float64, device="cuda")
+        K.direct_eval(_cuda(pos), _cuda(f) if sl else None, _cuda(q) if dl else None, _cuda(trg),
+                      out, spg, tpg, mixed=mixed)
+        got = out.cpu().numpy()
+        assert np.all(np.isfinite(got))
+        assert _relerr(got[pick], ref[pick]) < tol, (mixed, _relerr(got[pick], ref[pick]))
+
+
 def test_full_size_far_field_properties(hip, orc):
     """512 vesicles at p=16 (278,528 points): f32c vs f64 on every target,
     and f64 vs the oracle on a sample of 96 targets."""

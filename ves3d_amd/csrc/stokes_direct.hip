@@ -2,27 +2,33 @@
 //
 // Two kernel families:
 //
-//  1. k_far_*: the all-pairs / far-field sum that stands in for the FMM
-//     (StokesAlltoAll, src/CPUKernels.cc:966-1054, and the PVFMM pair kernels
-//     src/PVFMMInterface.cc:161-238, :284-369).  One target per lane, 256
-//     targets per workgroup; sources are staged through LDS in tiles of 256
-//     and read back as wave-wide broadcasts.  The source range is cut into
-//     `nsplit` slices; the slice index is the fastest-varying part of the
+//  1. k_pairs_* and k_far_groups_*: the all-pairs / far-field sum that stands
+//     in for the FMM (StokesAlltoAll, src/CPUKernels.cc:966-1054, and the
+//     PVFMM pair kernels src/PVFMMInterface.cc:161-238, :284-369).  One target
+//     per lane, 256 targets per workgroup.  Every lane of a wave meets the
+//     same source at the same time, so the sources are read with uniform
+//     addresses (s_load into SGPRs, which the VALU takes as operands): no LDS
+//     staging, no barriers.  The source range is cut into `nsplit` slices of
+//     whole groups or, where a slice per group would leave the chip idle, of
+//     parts of groups; the slice index is the fastest-varying part of the
 //     block index, so with nsplit a multiple of 8 every XCD (blocks are dealt
-//     round-robin over the 8 XCDs) streams only its own slice of sources
-//     through its L2.  Each slice writes an FP64 partial, and k_sum_slices adds
-//     the partials in a fixed order (deterministic, no atomics).
-//     The FP32 ("f32c") form stages each source tile relative to an FP64
-//     anchor (the tile's first point) and shifts the lane's target by the same
-//     anchor in FP64 before rounding, so coordinate differences keep FP32
-//     relative accuracy independent of the box size; pair terms are summed in
-//     FP32 over 64 sources and merged into an FP32 (hi, lo) TwoSum pair.
+//     round-robin over the 8 XCDs) streams only its own slices of sources
+//     through its L2.  Each slice writes an FP64 partial, and k_sum_slices
+//     adds the partials in a fixed order (deterministic, no atomics).
+//     The FP64 kernels read the caller's arrays as they lie.  The FP32
+//     ("f32c") form packs each source relative to an FP64 anchor near it and
+//     shifts the lane's target by the same anchor in FP64 before rounding, so
+//     coordinate differences keep FP32 relative accuracy independent of the
+//     box size; pair terms are summed in FP32 over 64 sources and merged into
+//     an FP32 (hi, lo) TwoSum pair.
 //
 //  2. k_vesicle_*: the per-vesicle Device<>::DirectStokes /
 //     DirectStokesDoubleLayer sums (src/CPUKernels.cc:8-118, :1059-1136) on
 //     AxisMajor [ves][xyz][stride] data; one wave per 64 targets of one
 //     vesicle, sources of that vesicle staged through LDS.
+#include <algorithm>
 #include <atomic>
+#include <type_traits>
 #include "common.hpp"
 #include "implicit.hpp"
 #include "runtime.hpp"
@@ -30,34 +36,9 @@
 namespace v3d {
 
 constexpr int FF_BLOCK = 256;
-constexpr int FF_TILE = 256;
-constexpr int FF_SUB = 64;  // FP32 form: TwoSum merge period (sources)
-
-struct __align__(16) SrcRec64 {
-  double x, y, z, _p0;
-  double fx, fy, fz, _p1;
-  double gx, gy, gz, _p2;
-  double nx, ny, nz, _p3;
-};
-struct __align__(16) SrcRec32 {
-  float x, y, z, _p0;
-  float fx, fy, fz, _p1;
-  float gx, gy, gz, _p2;
-  float nx, ny, nz, _p3;
-};
-
-// Source range of one slice: whole groups when grouped, else an even split.
-__device__ __forceinline__ void slice_range(long slice, int nsplit, long n_src,
-                                            long spg, long n_groups, long &g0,
-                                            long &g1) {
-  if (spg > 0) {
-    g0 = slice * n_groups / nsplit;
-    g1 = (slice + 1) * n_groups / nsplit;
-  } else {
-    g0 = 0;
-    g1 = 1;
-  }
-}
+constexpr int FF_TILE = 256;  // sources that share an anchor in k_pairs_f32c
+constexpr int FF_SUB = 64;    // FP32 form: TwoSum merge period (sources)
+constexpr int FF_PART = 32;   // fewest sources of a part of a group
 
 // 1/sqrt(x) for x > 0: the hardware estimate (v_rsq_f64, about 2^-20
 // relative) refined by one third-order step y (1 + e/2 + 3e^2/8),
@@ -68,273 +49,517 @@ __device__ __forceinline__ double rsqrt_pair(double x) {
   const double e = fma(y * -x, y, 1.0);
   return fma(y * e, fma(e, 0.375, 0.5), y);
 }
+__device__ __forceinline__ float rsqrt_pair(float x) { return __frsqrt_rn(x); }
 
-// GUARD: drop pairs with r^2 <= eps2.  Without it a coincident pair gives
-// NaN; the far field between vesicles runs without it (distinct vesicles'
-// surfaces are disjoint, so every pair is at a positive distance).
-template <bool SL, bool DL, bool GUARD>
-__global__ __launch_bounds__(FF_BLOCK) void k_far_f64(
-    const double *__restrict__ spos, const double *__restrict__ sld,
-    const double *__restrict__ dld, long n_src, const double *__restrict__ tpos,
-    long n_trg, long spg, long tpg, long n_groups, int nsplit, double eps2,
-    double csl, double cdl, double *__restrict__ part) {
-  __shared__ SrcRec64 sh[FF_TILE];
-  const long slice = blockIdx.x % nsplit;
-  const long tb = blockIdx.x / nsplit;
-  const long t = tb * FF_BLOCK + threadIdx.x;
-  const bool tvalid = t < n_trg;
-  double tx = 0, ty = 0, tz = 0;
-  if (tvalid) {
-    tx = tpos[3 * t];
-    ty = tpos[3 * t + 1];
-    tz = tpos[3 * t + 2];
-  }
-  const bool grouped = spg > 0 && tpg > 0;
-  const long my_g = (grouped && tvalid) ? t / tpg : -1;
-  const long tfirst = tb * FF_BLOCK;
-  const long tlast = min(tfirst + FF_BLOCK, n_trg) - 1;
-  // the group holding all the block's targets (or -1), divided once
-  const long own_b = (grouped && tfirst / tpg == tlast / tpg) ? tfirst / tpg : -1;
+// The r^2 bias that removes a target's own group from a sum without making
+// control flow divergent.  FP32: 1/sqrt(inf) = 0 and every term is an exact
+// zero.  FP64: infinity would turn the refinement step into a NaN; with 1e200
+// an own-group source adds 1e-100 |f|, nothing at 53 bits.
+constexpr double kOwnGroupBias64 = 1e200;
+constexpr float kOwnGroupBias = __builtin_inff();
 
-  double Sx = 0, Sy = 0, Sz = 0, Qx = 0, Qy = 0, Qz = 0;
-  long g0, g1;
-  slice_range(slice, nsplit, n_src, grouped ? spg : 0, n_groups, g0, g1);
-  for (long g = g0; g < g1; ++g) {
-    long sb, se;
-    if (grouped) {
-      if (g == own_b) continue;  // block-uniform skip
-      sb = g * spg;
-      se = sb + spg;
-    } else {
-      sb = slice * n_src / nsplit;
-      se = (slice + 1) * n_src / nsplit;
-    }
-    const bool lane_on = tvalid && (my_g != g);
-    for (long c0 = sb; c0 < se; c0 += FF_TILE) {
-      const int cnt = (int)min((long)FF_TILE, se - c0);
-      __syncthreads();
-      for (int i = threadIdx.x; i < cnt; i += FF_BLOCK) {
-        const long s = c0 + i;
-        SrcRec64 r;
-        r.x = spos[3 * s];
-        r.y = spos[3 * s + 1];
-        r.z = spos[3 * s + 2];
-        if (SL) {
-          r.fx = sld[3 * s];
-          r.fy = sld[3 * s + 1];
-          r.fz = sld[3 * s + 2];
-        }
-        if (DL) {
-          r.gx = dld[6 * s];
-          r.gy = dld[6 * s + 1];
-          r.gz = dld[6 * s + 2];
-          r.nx = dld[6 * s + 3];
-          r.ny = dld[6 * s + 4];
-          r.nz = dld[6 * s + 5];
-        }
-        sh[i] = r;
-      }
-      __syncthreads();
-      if (lane_on) {
-#pragma unroll 4
-        for (int j = 0; j < cnt; ++j) {
-          const double dx = tx - sh[j].x, dy = ty - sh[j].y, dz = tz - sh[j].z;
-          const double r2 = dx * dx + dy * dy + dz * dz;
-          // unconditional rsqrt + select: no per-pair branch in the loop
-          const double rq = rsqrt_pair(r2);
-          const double ri = GUARD ? ((r2 > eps2) ? rq : 0.0) : rq;
-          const double ri2 = ri * ri;
-          if (SL) {
-            const double ip =
-                (sh[j].fx * dx + sh[j].fy * dy + sh[j].fz * dz) * ri2;
-            Sx += ri * (sh[j].fx + dx * ip);
-            Sy += ri * (sh[j].fy + dy * ip);
-            Sz += ri * (sh[j].fz + dz * ip);
-          }
-          if (DL) {
-            const double p = (sh[j].nx * dx + sh[j].ny * dy + sh[j].nz * dz) *
-                             (sh[j].gx * dx + sh[j].gy * dy + sh[j].gz * dz) *
-                             (ri2 * ri2 * ri);
-            Qx += dx * p;
-            Qy += dy * p;
-            Qz += dz * p;
-          }
-        }
-      }
-    }
-  }
-  if (tvalid) {
-    double *o = part + (slice * n_trg + t) * 3;
-    o[0] = csl * Sx + cdl * Qx;
-    o[1] = csl * Sy + cdl * Qy;
-    o[2] = csl * Sz + cdl * Qz;
-  }
+// Slices over parts of groups: unit u = (group u / nsub, part u % nsub), and
+// slice k holds units k per .. (k + 1) per - 1 (the last slice what is left).
+// share (1 or 4): waves of a workgroup that take the same targets, each a
+// slice of its own, and add their sums in LDS.
+struct SliceMap {
+  unsigned units, per, nsub, share;
+};
+struct Slice {
+  unsigned u, u1;  // units
+  unsigned g, j;   // group and part of unit u
+};
+__device__ __forceinline__ Slice slice_of(const SliceMap &m, unsigned block_slice) {
+  const unsigned wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const unsigned k = m.share == 1 ? block_slice : block_slice * m.share + wv;
+  Slice s;
+  s.u = min(k * m.per, m.units);
+  s.u1 = min(s.u + m.per, m.units);
+  s.g = s.u / m.nsub;
+  s.j = s.u % m.nsub;
+  return s;
+}
+// a / b with the short 32-bit division wherever the operands allow it
+__device__ __forceinline__ long quot(long a, long b) {
+  return ((a | b) >> 32) ? a / b : (long)((unsigned)a / (unsigned)b);
 }
 
-template <bool SL, bool DL, bool GUARD>
-__global__ __launch_bounds__(FF_BLOCK) void k_far_f32c(
-    const double *__restrict__ spos, const double *__restrict__ sld,
-    const double *__restrict__ dld, long n_src, const double *__restrict__ tpos,
-    long n_trg, long spg, long tpg, long n_groups, int nsplit, float eps2,
-    double csl, double cdl, double *__restrict__ part) {
-  __shared__ SrcRec32 sh[FF_TILE];
-  const long slice = blockIdx.x % nsplit;
-  const long tb = blockIdx.x / nsplit;
-  const long t = tb * FF_BLOCK + threadIdx.x;
-  const bool tvalid = t < n_trg;
-  double tx = 0, ty = 0, tz = 0;
-  if (tvalid) {
-    tx = tpos[3 * t];
-    ty = tpos[3 * t + 1];
-    tz = tpos[3 * t + 2];
+// The targets of a wave: 64 consecutive ones, one per lane.  A lane past the
+// last target computes for the last one and stores nothing, so that control
+// flow inside the source loops stays uniform.
+struct WaveTargets {
+  long row;    // wave index over the targets
+  bool live;   // the wave has a target
+  long t, tc;  // the lane's target, clamped to the last one
+  long group;  // the lane's group (grouped sums)
+  long own;    // the group that holds all the wave's targets, or -1
+};
+__device__ __forceinline__ WaveTargets wave_targets(long tb, unsigned share, long n_trg, long tpg) {
+  const long wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  WaveTargets w;
+  w.row = share == 1 ? tb * (FF_BLOCK / 64) + wv : tb;
+  const long first = w.row * 64, last = min(first + 64, n_trg) - 1;
+  w.live = first < n_trg;
+  w.t = first + (threadIdx.x & 63);
+  w.tc = min(w.t, n_trg - 1);
+  w.group = w.own = -1;
+  if (tpg > 0 && w.live) {
+    const long gf = quot(first, tpg);
+    w.own = gf == quot(last, tpg) ? gf : -1;
+    w.group = w.own >= 0 ? gf : quot(w.tc, tpg);
   }
-  const bool grouped = spg > 0 && tpg > 0;
-  const long my_g = (grouped && tvalid) ? t / tpg : -1;
-  const long tfirst = tb * FF_BLOCK;
-  const long tlast = min(tfirst + FF_BLOCK, n_trg) - 1;
-  // the group holding all the block's targets (or -1), divided once
-  const long own_b = (grouped && tfirst / tpg == tlast / tpg) ? tfirst / tpg : -1;
+  return w;
+}
 
-  // (hi, lo) compensated running sums
-  float Sh[3] = {0, 0, 0}, Sl[3] = {0, 0, 0};
-  float Qh[3] = {0, 0, 0}, Ql[3] = {0, 0, 0};
-  long g0, g1;
-  slice_range(slice, nsplit, n_src, grouped ? spg : 0, n_groups, g0, g1);
-  for (long g = g0; g < g1; ++g) {
-    long sb, se;
-    if (grouped) {
-      if (g == own_b) continue;
-      sb = g * spg;
-      se = sb + spg;
-    } else {
-      sb = slice * n_src / nsplit;
-      se = (slice + 1) * n_src / nsplit;
-    }
-    const bool lane_on = tvalid && (my_g != g);
-    for (long c0 = sb; c0 < se; c0 += FF_TILE) {
-      const int cnt = (int)min((long)FF_TILE, se - c0);
-      __syncthreads();
-      const double ax = spos[3 * c0], ay = spos[3 * c0 + 1], az = spos[3 * c0 + 2];
-      for (int i = threadIdx.x; i < cnt; i += FF_BLOCK) {
-        const long s = c0 + i;
-        SrcRec32 r;
-        r.x = (float)(spos[3 * s] - ax);
-        r.y = (float)(spos[3 * s + 1] - ay);
-        r.z = (float)(spos[3 * s + 2] - az);
-        if (SL) {
-          r.fx = (float)sld[3 * s];
-          r.fy = (float)sld[3 * s + 1];
-          r.fz = (float)sld[3 * s + 2];
-        }
-        if (DL) {
-          r.gx = (float)dld[6 * s];
-          r.gy = (float)dld[6 * s + 1];
-          r.gz = (float)dld[6 * s + 2];
-          r.nx = (float)dld[6 * s + 3];
-          r.ny = (float)dld[6 * s + 4];
-          r.nz = (float)dld[6 * s + 5];
-        }
-        sh[i] = r;
-      }
-      __syncthreads();
-      if (lane_on) {
-        const float lx = (float)(tx - ax), ly = (float)(ty - ay), lz = (float)(tz - az);
-        for (int j0 = 0; j0 < cnt; j0 += FF_SUB) {
-          const int j1 = min(cnt, j0 + FF_SUB);
-          float sx = 0, sy = 0, sz = 0, qx = 0, qy = 0, qz = 0;
-#pragma unroll 4
-          for (int j = j0; j < j1; ++j) {
-            const float dx = lx - sh[j].x, dy = ly - sh[j].y, dz = lz - sh[j].z;
-            const float r2 = dx * dx + dy * dy + dz * dz;
-            const float rq = __frsqrt_rn(r2);
-            const float ri = GUARD ? ((r2 > eps2) ? rq : 0.0f) : rq;
-            const float ri2 = ri * ri;
-            if (SL) {
-              const float ip = (sh[j].fx * dx + sh[j].fy * dy + sh[j].fz * dz) * ri2;
-              sx += ri * (sh[j].fx + dx * ip);
-              sy += ri * (sh[j].fy + dy * ip);
-              sz += ri * (sh[j].fz + dz * ip);
-            }
-            if (DL) {
-              const float p = (sh[j].nx * dx + sh[j].ny * dy + sh[j].nz * dz) *
-                              (sh[j].gx * dx + sh[j].gy * dy + sh[j].gz * dz) *
-                              (ri2 * ri2 * ri);
-              qx += dx * p;
-              qy += dy * p;
-              qz += dz * p;
-            }
-          }
-          float s_, e_;
-          if (SL) {
-            two_sum(Sh[0], sx, s_, e_); Sh[0] = s_; Sl[0] += e_;
-            two_sum(Sh[1], sy, s_, e_); Sh[1] = s_; Sl[1] += e_;
-            two_sum(Sh[2], sz, s_, e_); Sh[2] = s_; Sl[2] += e_;
-          }
-          if (DL) {
-            two_sum(Qh[0], qx, s_, e_); Qh[0] = s_; Ql[0] += e_;
-            two_sum(Qh[1], qy, s_, e_); Qh[1] = s_; Ql[1] += e_;
-            two_sum(Qh[2], qz, s_, e_); Qh[2] = s_; Ql[2] += e_;
-          }
-        }
-      }
-    }
-  }
-  if (tvalid) {
-    double *o = part + (slice * n_trg + t) * 3;
+// Writes the wave's sums (N per target) to o[N t ..]: where the workgroup's
+// waves share their targets, those of all four added in wave order.
+template <int N>
+__device__ __forceinline__ void store_sums(const WaveTargets &w, unsigned share, long n_trg,
+                                           const double (&v)[N], double *__restrict__ o) {
+  double s[N];
 #pragma unroll
-    for (int c = 0; c < 3; ++c)
-      o[c] = csl * ((double)Sh[c] + (double)Sl[c]) + cdl * ((double)Qh[c] + (double)Ql[c]);
+  for (int c = 0; c < N; ++c) s[c] = v[c];
+  if (share > 1) {
+    __shared__ double red[FF_BLOCK / 64 - 1][N][64];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    if (wv > 0) {
+#pragma unroll
+      for (int c = 0; c < N; ++c) red[wv - 1][c][lane] = s[c];
+    }
+    __syncthreads();
+    if (wv > 0) return;
+#pragma unroll
+    for (int k = 0; k < FF_BLOCK / 64 - 1; ++k)
+#pragma unroll
+      for (int c = 0; c < N; ++c) s[c] += red[k][c][lane];
+  }
+  if (w.t < n_trg) {
+#pragma unroll
+    for (int c = 0; c < N; ++c) o[3 * w.t + c] = s[c];
   }
 }
 
-__global__ void k_sum_slices(const double *__restrict__ part, int nsplit, long n,
-                             double *__restrict__ out) {
+// One pair's contribution: f / r + (f.d) d / r^3 and k (n.d)(g.d) d / r^5,
+// with ri = 1 / r, f at `f`, (g, n) at `q`.  With both layers the terms along
+// d share one coefficient.
+template <bool SL, bool DL, typename T>
+__device__ __forceinline__ void add_pair(T dx, T dy, T dz, T ri, const T *__restrict__ f,
+                                         const T *__restrict__ q, T k, T (&S)[3]) {
+  const T ri2 = ri * ri;
+  if constexpr (!DL) {
+    const T ip = (f[0] * dx + f[1] * dy + f[2] * dz) * ri2;
+    S[0] = fma(ri, fma(dx, ip, f[0]), S[0]);
+    S[1] = fma(ri, fma(dy, ip, f[1]), S[1]);
+    S[2] = fma(ri, fma(dz, ip, f[2]), S[2]);
+  } else {
+    const T t = (q[3] * dx + q[4] * dy + q[5] * dz) * (q[0] * dx + q[1] * dy + q[2] * dz) * ri2;
+    if constexpr (SL) {
+      const T w = fma(k, t, f[0] * dx + f[1] * dy + f[2] * dz) * (ri * ri2);
+      S[0] = fma(dx, w, fma(ri, f[0], S[0]));
+      S[1] = fma(dy, w, fma(ri, f[1], S[1]));
+      S[2] = fma(dz, w, fma(ri, f[2], S[2]));
+    } else {
+      const T w = t * (ri * ri2);
+      S[0] = fma(dx, w, S[0]);
+      S[1] = fma(dy, w, S[1]);
+      S[2] = fma(dz, w, S[2]);
+    }
+  }
+}
+
+// r^2 >= 0 ordered as an unsigned integer (FP64: by its high word).
+__device__ __forceinline__ unsigned order_key(double x) { return (unsigned)__double2hiint(x); }
+__device__ __forceinline__ unsigned order_key(float x) { return __float_as_uint(x); }
+
+// GUARD: pairs with r^2 <= eps2 contribute nothing.  Such pairs are rare (a
+// point meeting itself), so runs of FF_RUN sources are summed without a test
+// while the smallest r^2 is kept (half an integer instruction per pair); a
+// wave that met one repeats the run with a selection per pair.
+constexpr int FF_RUN = 32;
+
+// n consecutive FP64 sources (positions p, densities f, (g, n) at q) at one
+// target, U at a time.
+template <int U, bool SL, bool DL, bool GUARD>
+__device__ __forceinline__ void add_sources64(double tx, double ty, double tz, double bias, int n,
+                                              const double *__restrict__ p,
+                                              const double *__restrict__ f,
+                                              const double *__restrict__ q, double k, double eps2,
+                                              double (&S)[3]) {
+  unsigned m = ~0u;
+  auto block = [&](int i, auto uc, bool select) {
+    constexpr int V = decltype(uc)::value;
+    double dx[V], dy[V], dz[V], r2[V];
+#pragma unroll
+    for (int u = 0; u < V; ++u) {
+      const double *__restrict__ x = p + (i + u) * 3;
+      dx[u] = tx - x[0];
+      dy[u] = ty - x[1];
+      dz[u] = tz - x[2];
+      r2[u] = fma(dz[u], dz[u], fma(dy[u], dy[u], fma(dx[u], dx[u], bias)));
+    }
+    if (GUARD && !select) {
+#pragma unroll
+      for (int u = 0; u < V; ++u) m = min(m, order_key(r2[u]));
+    }
+#pragma unroll
+    for (int u = 0; u < V; ++u) {
+      double ri = rsqrt_pair(r2[u]);
+      if (GUARD && select) ri = r2[u] > eps2 ? ri : 0.0;
+      add_pair<SL, DL>(dx[u], dy[u], dz[u], ri, f + (i + u) * 3, q + (i + u) * 6, k, S);
+    }
+  };
+  using One = std::integral_constant<int, 1>;
+  const int run = GUARD ? FF_RUN : n;
+  for (int i0 = 0; i0 < n; i0 += run) {
+    const int i1 = min(n, i0 + run);
+    const double S0[3] = {S[0], S[1], S[2]};
+    m = ~0u;
+    int i = i0;
+    for (; i + U <= i1; i += U) block(i, std::integral_constant<int, U>(), false);
+    for (; i < i1; ++i) block(i, One(), false);
+    if (GUARD && __any(m <= order_key(eps2))) {
+#pragma unroll
+      for (int c = 0; c < 3; ++c) S[c] = S0[c];
+#pragma unroll 1
+      for (i = i0; i < i1; ++i) block(i, One(), true);
+    }
+  }
+}
+
+// One step of U pairs' arithmetic, kept together by the scheduler: a SIMD
+// issues runs of one independent FP32 instruction faster than the same
+// instructions pair by pair (18 instructions per single-layer pair: 62 against
+// 71 cycles measured on registers alone, whatever file the operands are in).
+template <int U, typename F>
+__device__ __forceinline__ void stage(F f) {
+#pragma unroll
+  for (int u = 0; u < U; ++u) f(u);
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// U consecutive FP32 records at one target (lx, ly, lz): NS single-layer
+// densities, into S (and T), and with DL the double layer, into S:
+// (x, y, z[, f[, h]][, g, n]).  KEY: m keeps the smallest r^2.
+template <int U, int NS, bool DL, bool KEY>
+__device__ __forceinline__ void add_block32(const float *__restrict__ rec, float lx, float ly,
+                                            float lz, float bias, float k, float (&S)[3],
+                                            float (&T)[3], unsigned &m) {
+  constexpr int R = 3 + 3 * NS + (DL ? 6 : 0);
+  static_assert(!DL || NS <= 1, "one density beside a double layer");
+  float s[U * R];
+#pragma unroll
+  for (int i = 0; i < U * R; ++i) s[i] = rec[i];
+  float d[U][3], ri[U], t[U];
+  stage<U>([&](int u) { d[u][0] = lx - s[u * R]; });
+  stage<U>([&](int u) { d[u][1] = ly - s[u * R + 1]; });
+  stage<U>([&](int u) { d[u][2] = lz - s[u * R + 2]; });
+  stage<U>([&](int u) { ri[u] = fmaf(d[u][0], d[u][0], bias); });
+  stage<U>([&](int u) { ri[u] = fmaf(d[u][1], d[u][1], ri[u]); });
+  stage<U>([&](int u) { ri[u] = fmaf(d[u][2], d[u][2], ri[u]); });
+  if constexpr (KEY) stage<U>([&](int u) { m = min(m, order_key(ri[u])); });
+  stage<U>([&](int u) { ri[u] = rsqrt_pair(ri[u]); });
+  auto dot = [&](float (&o)[U], int c) {  // record entries c .. c + 2 times d
+    stage<U>([&](int u) { o[u] = s[u * R + c] * d[u][0]; });
+    stage<U>([&](int u) { o[u] = fmaf(s[u * R + c + 1], d[u][1], o[u]); });
+    stage<U>([&](int u) { o[u] = fmaf(s[u * R + c + 2], d[u][2], o[u]); });
+  };
+  if constexpr (!DL) {
+#pragma unroll
+    for (int e = 0; e < NS; ++e) {
+      const int c0 = 3 + 3 * e;
+      float (&Z)[3] = e ? T : S;
+      float a[U][3];
+      dot(t, c0);
+      stage<U>([&](int u) { t[u] *= ri[u]; });
+      stage<U>([&](int u) { t[u] *= ri[u]; });
+#pragma unroll
+      for (int c = 0; c < 3; ++c)
+        stage<U>([&](int u) { a[u][c] = fmaf(d[u][c], t[u], s[u * R + c0 + c]); });
+      stage<U>([&](int u) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) Z[c] = fmaf(ri[u], a[u][c], Z[c]);
+      });
+    }
+  } else {
+    float w[U], q[U];
+    dot(t, R - 3);
+    dot(w, R - 6);
+    stage<U>([&](int u) { q[u] = ri[u] * ri[u]; });
+    stage<U>([&](int u) { t[u] *= w[u]; });
+    stage<U>([&](int u) { t[u] *= q[u]; });
+    stage<U>([&](int u) { q[u] *= ri[u]; });
+    if constexpr (NS == 1) {
+      dot(w, 3);
+      stage<U>([&](int u) { t[u] = fmaf(k, t[u], w[u]); });
+      stage<U>([&](int u) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) S[c] = fmaf(ri[u], s[u * R + 3 + c], S[c]);
+      });
+    }
+    stage<U>([&](int u) { t[u] *= q[u]; });
+    stage<U>([&](int u) {
+#pragma unroll
+      for (int c = 0; c < 3; ++c) S[c] = fmaf(d[u][c], t[u], S[c]);
+    });
+  }
+}
+
+// FP64 sums of n_groups groups of spg sources (ungrouped: one group, tpg = 0),
+// part j of a group its sources j plen .. (j + 1) plen - 1.
+// Bound: FP64 VALU issue, 23 instructions per single-layer pair, 33 with both
+// layers (4.0-4.5 cycles each on a SIMD, 16 for v_rsq_f64).  Measured with
+// both layers between 320 vesicles of 544 points (3.0e10 pairs): 32.9 ms;
+// sources staged through LDS as 128-byte records, read back as broadcasts,
+// took 42.9 ms.
+template <bool SL, bool DL, bool GUARD>
+__global__ __launch_bounds__(FF_BLOCK) void k_pairs_f64(
+    const double *__restrict__ spos, const double *__restrict__ sld,
+    const double *__restrict__ dld, long spg, const double *__restrict__ tpos, long n_trg, long tpg,
+    SliceMap map, long plen, unsigned nsplit, double eps2, double scale, double ratio,
+    double *__restrict__ part) {
+  const unsigned slice = blockIdx.x % nsplit;
+  const WaveTargets w = wave_targets(blockIdx.x / nsplit, map.share, n_trg, tpg);
+  if (!w.live) return;
+  const double tx = tpos[3 * w.tc], ty = tpos[3 * w.tc + 1], tz = tpos[3 * w.tc + 2];
+  double S[3] = {0, 0, 0};
+  Slice k = slice_of(map, slice);
+  constexpr int U = DL ? 2 : 4;
+  while (k.u < k.u1) {
+    // the slice's parts of group k.g, in one run
+    const unsigned take = min(map.nsub - k.j, k.u1 - k.u);
+    const long g = k.g, r0 = k.j * plen, n = min(take * plen, spg - r0), s0 = g * spg + r0;
+    if (g != w.own) {  // wave-uniform skip
+      const double bias = w.group == g ? kOwnGroupBias64 : 0.0;
+      const double *__restrict__ p = spos + 3 * s0;
+      const double *__restrict__ f = SL ? sld + 3 * s0 : p;
+      const double *__restrict__ q = DL ? dld + 6 * s0 : p;
+      for (long i = 0; i < n; i += 1 << 24)
+        add_sources64<U, SL, DL, GUARD>(tx, ty, tz, bias, (int)min(n - i, 1L << 24), p + 3 * i,
+                                        f + 3 * i, q + 6 * i, ratio, eps2, S);
+    }
+    k.u += take;
+    k.j = 0;
+    ++k.g;
+  }
+  const double v[3] = {scale * S[0], scale * S[1], scale * S[2]};
+  store_sums(w, map.share, n_trg, v, part + (long)slice * n_trg * 3);
+}
+
+// FP32 partial sums merged into a TwoSum (hi, lo) pair.
+struct Acc32 {
+  float h[3], l[3];
+};
+__device__ __forceinline__ void acc_merge(Acc32 &a, const float (&x)[3]) {
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    float s_, e_;
+    two_sum(a.h[c], x[c], s_, e_);
+    a.h[c] = s_;
+    a.l[c] += e_;
+  }
+}
+
+// FP32 records (x, y, z[, f][, g, n]) relative to the anchor of their tile of
+// FF_TILE sources (the tile's first point; tiles restart with every group).
+template <bool SL, bool DL>
+__global__ void k_pack_pairs32(const double *__restrict__ spos, const double *__restrict__ sld,
+                               const double *__restrict__ dld, long n, long spg,
+                               float *__restrict__ rec) {
+  constexpr int R = 3 + (SL ? 3 : 0) + (DL ? 6 : 0);
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  double s = 0;
-  for (int k = 0; k < nsplit; ++k) s += part[(long)k * n + i];
-  out[i] = s;
-}
-
-// Number of source slices: a multiple of 8 (one per XCD), raised until the
-// grid holds at least ~16 waves per SIMD of the 256-CU part.
-static int choose_nsplit(long n_trg, long n_src, long n_groups) {
-  const long tblocks = (n_trg + FF_BLOCK - 1) / FF_BLOCK;
-  int ns = 8;
-  while (ns < 64 && tblocks * ns * (FF_BLOCK / 64) < 16 * 1024) ns *= 2;
-  long cap = n_groups > 0 ? n_groups : (n_src + FF_TILE - 1) / FF_TILE;
-  if (cap < 1) cap = 1;
-  if (ns > cap) ns = (int)cap;
-  return ns;
-}
-
-template <bool F32, bool SL, bool DL>
-static void launch_far(dim3 grid, hipStream_t st, const double *spos,
-                       const double *sld, const double *dld, long n_src,
-                       const double *tpos, long n_trg, long sp, long tp,
-                       long n_groups, int ns, double eps2, double csl,
-                       double cdl, double *part, bool guard) {
-  if (F32) {
-    if (guard)
-      k_far_f32c<SL, DL, true><<<grid, FF_BLOCK, 0, st>>>(spos, sld, dld, n_src, tpos, n_trg, sp, tp,
-                                                          n_groups, ns, (float)eps2, csl, cdl, part);
-    else
-      k_far_f32c<SL, DL, false><<<grid, FF_BLOCK, 0, st>>>(spos, sld, dld, n_src, tpos, n_trg, sp, tp,
-                                                           n_groups, ns, (float)eps2, csl, cdl, part);
-  } else {
-    if (guard)
-      k_far_f64<SL, DL, true><<<grid, FF_BLOCK, 0, st>>>(spos, sld, dld, n_src, tpos, n_trg, sp, tp,
-                                                         n_groups, ns, eps2, csl, cdl, part);
-    else
-      k_far_f64<SL, DL, false><<<grid, FF_BLOCK, 0, st>>>(spos, sld, dld, n_src, tpos, n_trg, sp, tp,
-                                                          n_groups, ns, eps2, csl, cdl, part);
+  const long g0 = spg > 0 ? quot(i, spg) * spg : 0;
+  const double *a = spos + 3 * (g0 + (i - g0) / FF_TILE * FF_TILE);
+  float *r = rec + i * R;
+#pragma unroll
+  for (int c = 0; c < 3; ++c) r[c] = (float)(spos[3 * i + c] - a[c]);
+  if (SL) {
+#pragma unroll
+    for (int c = 0; c < 3; ++c) r[3 + c] = (float)sld[3 * i + c];
   }
+  if (DL) {
+#pragma unroll
+    for (int c = 0; c < 6; ++c) r[R - 6 + c] = (float)dld[6 * i + c];
+  }
+}
+
+// The FP32 form over such records: cell c is tile c % ntile of group
+// c / ntile (ungrouped: one group of n_src sources), cut into nsub parts of
+// plen sources.  Bound: FP32 VALU issue, 18 instructions per single-layer
+// pair and 28 with both layers, 3.5 cycles each on average.  Measured, single
+// layer from 59,803 sources to 7,001 targets: 214 us with its packing and
+// sum (217 us from LDS tiles).
+template <bool SL, bool DL, bool GUARD>
+__global__ __launch_bounds__(FF_BLOCK, DL ? 8 : (GUARD ? 6 : 7)) void k_pairs_f32c(
+    const float *__restrict__ rec, const double *__restrict__ spos, long spg, unsigned ntile,
+    const double *__restrict__ tpos, long n_trg, long tpg, SliceMap map, int plen, unsigned nsplit,
+    float eps2, double scale, float ratio, double *__restrict__ part) {
+  constexpr int R = 3 + (SL ? 3 : 0) + (DL ? 6 : 0), U = DL ? 4 : 8;
+  constexpr int FO = 3, QO = R - 6;
+  const unsigned slice = blockIdx.x % nsplit;
+  const WaveTargets w = wave_targets(blockIdx.x / nsplit, map.share, n_trg, tpg);
+  if (!w.live) return;
+  const double tx = tpos[3 * w.tc], ty = tpos[3 * w.tc + 1], tz = tpos[3 * w.tc + 2];
+  Acc32 A = {{0, 0, 0}, {0, 0, 0}};
+  Slice k = slice_of(map, slice);
+  unsigned tile = k.g % ntile;
+  long g = k.g / ntile;
+  while (k.u < k.u1) {
+    // the slice's parts of cell k.g, in one run
+    const unsigned take = min(map.nsub - k.j, k.u1 - k.u);
+    if (g != w.own) {  // wave-uniform skip
+      const long c0 = g * spg + (long)tile * FF_TILE;
+      const int cnt = (int)min((long)FF_TILE, spg - (long)tile * FF_TILE);
+      const int r0 = (int)k.j * plen, r1 = min(cnt, r0 + (int)take * plen);
+      const float bias = w.group == g ? kOwnGroupBias : 0.0f;
+      const double *a = spos + 3 * c0;
+      const float lx = (float)(tx - a[0]), ly = (float)(ty - a[1]), lz = (float)(tz - a[2]);
+      for (int i0 = r0; i0 < r1; i0 += FF_SUB) {
+        const float *__restrict__ r = rec + (c0 + i0) * R;
+        const int n = min(FF_SUB, r1 - i0);
+        float S[3] = {0, 0, 0};
+        constexpr int run = GUARD ? FF_RUN : FF_SUB;
+        for (int k0 = 0; k0 < n; k0 += run) {
+          const int k1 = min(n, k0 + run);
+          const float S0[3] = {S[0], S[1], S[2]};
+          unsigned m = ~0u;
+          int i = k0;
+          for (; i + U <= k1; i += U)
+            add_block32<U, SL ? 1 : 0, DL, GUARD>(r + i * R, lx, ly, lz, bias, ratio, S, S, m);
+          for (; i < k1; ++i)
+            add_block32<1, SL ? 1 : 0, DL, GUARD>(r + i * R, lx, ly, lz, bias, ratio, S, S, m);
+          if (GUARD && __any(m <= order_key(eps2))) {
+#pragma unroll
+            for (int c = 0; c < 3; ++c) S[c] = S0[c];
+#pragma unroll 1
+            for (i = k0; i < k1; ++i) {
+              const float *__restrict__ s = r + i * R;
+              const float dx = lx - s[0], dy = ly - s[1], dz = lz - s[2];
+              const float r2 = fmaf(dz, dz, fmaf(dy, dy, fmaf(dx, dx, bias)));
+              add_pair<SL, DL>(dx, dy, dz, r2 > eps2 ? rsqrt_pair(r2) : 0.0f, s + FO, s + QO,
+                               ratio, S);
+            }
+          }
+        }
+        acc_merge(A, S);
+      }
+    }
+    k.u += take;
+    k.j = 0;
+    if (++tile == ntile) {
+      tile = 0;
+      ++g;
+    }
+  }
+  double v[3];
+#pragma unroll
+  for (int c = 0; c < 3; ++c) v[c] = scale * ((double)A.h[c] + (double)A.l[c]);
+  store_sums(w, map.share, n_trg, v, part + (long)slice * n_trg * 3);
+}
+
+// out[i] = the sum of the slices' partials: G threads per output add every
+// G-th slice, and their sums are added in order.
+template <int G>
+__global__ __launch_bounds__(256) void k_sum_slices(const double *__restrict__ part, int nsplit,
+                                                    long n, double *__restrict__ out) {
+  constexpr int W = 256 / G;
+  __shared__ double sh[G][W];
+  const int c = threadIdx.x % W, q = threadIdx.x / W;
+  const long i = (long)blockIdx.x * W + c;
+  double s = 0;
+  if (i < n) {
+#pragma unroll 4
+    for (int k = q; k < nsplit; k += G) s += part[(long)k * n + i];
+  }
+  sh[q][c] = s;
+  __syncthreads();
+  if (q == 0 && i < n) {
+    for (int k = 1; k < G; ++k) s += sh[k][c];
+    out[i] = s;
+  }
+}
+static int sum_slices(const double *part, int nsplit, long n, double *out, hipStream_t st) {
+  // few slices: one coalesced 512-byte read per wave; many (few targets): 16
+  // threads share an output's chain of loads
+  if (nsplit >= 64)
+    k_sum_slices<16><<<cdiv(n, 16), 256, 0, st>>>(part, nsplit, n, out);
+  else
+    k_sum_slices<4><<<cdiv(n, 64), 256, 0, st>>>(part, nsplit, n, out);
+  return launch_status();
+}
+
+// How the sources are cut.  A wave's life must be short against the launch,
+// or its last round leaves SIMDs idle: 32 waves per SIMD of the 256-CU part
+// (32 * 1024), as long as a slice keeps 128 sources (the partial sums are 48
+// bytes of traffic per slice and target); else 16 per SIMD in slices of at
+// least FF_PART sources.  Where the targets alone give less than 2048 waves,
+// the waves of a workgroup share their targets, which quarters the partial
+// sums; 1024 slices bound them where the targets are few.  Otherwise the
+// slices come in multiples of 8, one per XCD.  Parts of groups even out the
+// slices (about eight units each) unless there are many groups per slice.
+// Measured: the far field of two vesicles (624 targets, 2404 sources) 10 us,
+// 348 us with whole groups per slice; 2400 points to themselves 14.5 us with
+// the sum, 22.7 us in slices of 256 sources.
+struct Split {
+  int nsplit;
+  SliceMap map;
+};
+static Split choose_split(long n_trg, long n_groups, long spg, long max_slices = 1024) {
+  const long waves = (n_trg + 63) / 64, total = n_groups * spg;
+  const unsigned share = waves < 2048 ? 4 : 1;
+  const long w16 = (16 * 1024 + waves - 1) / waves, w32 = 2 * w16;
+  long want = total / 128 >= w16 ? std::min(w32, total / 128) : std::min(w16, total / FF_PART);
+  if (share == 1) want = std::max(8L, (want + 7) / 8 * 8);
+  want = std::max(1L, std::min(want, max_slices * share));
+  const long finest = (spg + FF_PART - 1) / FF_PART;
+  const long nsub = n_groups >= 8 * want ? 1 : std::min((8 * want + n_groups - 1) / n_groups, finest);
+  const long units = n_groups * nsub;
+  const long per = std::max(1L, (units + want - 1) / want);
+  const long slices = (units + per - 1) / per;
+  Split s;
+  s.nsplit = (int)((slices + share - 1) / share);
+  s.map = SliceMap{(unsigned)units, (unsigned)per, (unsigned)nsub, share};
+  return s;
+}
+// Workgroups of a launch over n_trg targets.
+static dim3 split_grid(const Split &s, long n_trg) {
+  const long waves = (n_trg + 63) / 64;
+  const long tblocks = s.map.share == 1 ? (waves + FF_BLOCK / 64 - 1) / (FF_BLOCK / 64) : waves;
+  return dim3((unsigned)(tblocks * s.nsplit));
+}
+// Part length of a group of cnt sources cut into nsub parts, a multiple of q.
+static long part_length(long cnt, unsigned nsub, long q) {
+  const long l = (cnt + nsub - 1) / nsub;
+  return std::max(q, (l + q - 1) / q * q);
+}
+
+template <bool SL, bool DL, bool GUARD>
+static int launch_pairs64(dim3 grid, hipStream_t st, const double *spos, const double *sld,
+                          const double *dld, long spg, const double *tpos, long n_trg, long tpg,
+                          const Split &sp, double eps2, double csl, double cdl, double *part) {
+  k_pairs_f64<SL, DL, GUARD><<<grid, FF_BLOCK, 0, st>>>(
+      spos, sld, dld, spg, tpos, n_trg, tpg, sp.map, part_length(spg, sp.map.nsub, 4),
+      (unsigned)sp.nsplit, eps2, SL ? csl : cdl, SL ? cdl / csl : 1.0, part);
+  return launch_status();
+}
+template <bool SL, bool DL, bool GUARD>
+static int launch_pairs32(dim3 grid, hipStream_t st, const double *spos, const double *sld,
+                          const double *dld, long n_src, long spg, unsigned ntile,
+                          const double *tpos, long n_trg, long tpg, const Split &sp, double eps2,
+                          double csl, double cdl, double *part, float *rec) {
+  k_pack_pairs32<SL, DL><<<cdiv(n_src, 256), 256, 0, st>>>(spos, sld, dld, n_src,
+                                                           tpg > 0 ? spg : 0, rec);
+  V3D_CHECK(launch_status());
+  k_pairs_f32c<SL, DL, GUARD><<<grid, FF_BLOCK, 0, st>>>(
+      rec, spos, spg, ntile, tpos, n_trg, tpg, sp.map, (int)part_length(std::min(spg, (long)FF_TILE), sp.map.nsub, 8),
+      (unsigned)sp.nsplit, (float)eps2, SL ? csl : cdl, (float)(SL ? cdl / csl : 1.0), part);
+  return launch_status();
 }
 
 // Shared driver of the all-pairs and far-field entry points.
 // part_fixed (optional): caller-provided scratch of part_cap bytes for the
 // per-slice partial sums instead of the library's workspace; the slice count
-// is then lowered until the partials fit.
+// is then held to what fits.
 template <bool F32>
 static int far_eval(const double *spos, const double *sld, const double *dld,
                     size_t n_src, const double *tpos, double *tvel, size_t n_trg,
@@ -349,490 +574,243 @@ static int far_eval(const double *spos, const double *sld, const double *dld,
   }
   if (!spos) return VES3D_INVALID_PARAMETER;
   const bool grouped = spg > 0 && tpg > 0;
-  long n_groups = 0;
-  if (grouped) {
-    if (n_src % spg || n_trg % tpg || n_src / spg != n_trg / tpg)
-      return VES3D_INVALID_PARAMETER;
-    n_groups = (long)(n_src / spg);
-  }
-  int ns = choose_nsplit((long)n_trg, (long)n_src, n_groups);
-  double *part = nullptr;
+  if (grouped && (n_src % spg || n_trg % tpg || n_src / spg != n_trg / tpg))
+    return VES3D_INVALID_PARAMETER;
+  const long n_groups = grouped ? (long)(n_src / spg) : 1;
+  const long sp = grouped ? (long)spg : (long)n_src, tp = grouped ? (long)tpg : 0;
+  const size_t per_slice = n_trg * 3 * sizeof(double);
+  long max_slices = 1024;
   if (part_fixed) {
-    const size_t per_slice = n_trg * 3 * sizeof(double);
     if (per_slice > part_cap) return VES3D_INVALID_PARAMETER;
-    while ((size_t)ns * per_slice > part_cap) ns = ns > 8 ? ns / 2 : ns - 1;
-    part = part_fixed;
-  } else {
-    part = (double *)workspace(kWsFarPartial, (size_t)ns * n_trg * 3 * sizeof(double));
+    max_slices = std::min(max_slices, (long)(part_cap / per_slice));
   }
+  const unsigned ntile = (unsigned)((sp + FF_TILE - 1) / FF_TILE);
+  const Split split = F32 ? choose_split((long)n_trg, n_groups * ntile, std::min(sp, (long)FF_TILE),
+                                         max_slices)
+                          : choose_split((long)n_trg, n_groups, sp, max_slices);
+  double *part =
+      part_fixed ? part_fixed : (double *)workspace(kWsFarPartial, split.nsplit * per_slice);
   if (!part) return VES3D_MEMORY_ERROR;
-  const long tblocks = ((long)n_trg + FF_BLOCK - 1) / FF_BLOCK;
-  const dim3 grid((unsigned)(tblocks * ns));
-  const long sp = grouped ? (long)spg : 0, tp = grouped ? (long)tpg : 0;
-  if (sld && dld)
-    launch_far<F32, true, true>(grid, st, spos, sld, dld, n_src, tpos, n_trg, sp, tp, n_groups, ns, eps2, csl, cdl, part, guard);
-  else if (sld)
-    launch_far<F32, true, false>(grid, st, spos, sld, dld, n_src, tpos, n_trg, sp, tp, n_groups, ns, eps2, csl, cdl, part, guard);
-  else
-    launch_far<F32, false, true>(grid, st, spos, sld, dld, n_src, tpos, n_trg, sp, tp, n_groups, ns, eps2, csl, cdl, part, guard);
-  V3D_CHECK(launch_status());
-  const long n = (long)n_trg * 3;
-  k_sum_slices<<<cdiv(n, 256), 256, 0, st>>>(part, ns, n, tvel);
-  return launch_status();
+  const size_t rec_n = 3 + (sld ? 3 : 0) + (dld ? 6 : 0);
+  float *rec = F32 ? (float *)workspace(kWsFarRecords, n_src * rec_n * sizeof(float)) : nullptr;
+  if (F32 && !rec) return VES3D_MEMORY_ERROR;
+  const dim3 grid = split_grid(split, (long)n_trg);
+#define V3D_PAIRS(SL, DL, G)                                                                     \
+  V3D_CHECK(F32 ? (launch_pairs32<SL, DL, G>(grid, st, spos, sld, dld, (long)n_src, sp, ntile,   \
+                                             tpos, (long)n_trg, tp, split, eps2, csl, cdl, part, \
+                                             rec))                                               \
+                : (launch_pairs64<SL, DL, G>(grid, st, spos, sld, dld, sp, tpos, (long)n_trg,    \
+                                             tp, split, eps2, csl, cdl, part)))
+  if (sld && dld) {
+    if (guard) V3D_PAIRS(true, true, true);
+    else V3D_PAIRS(true, true, false);
+  } else if (sld) {
+    if (guard) V3D_PAIRS(true, false, true);
+    else V3D_PAIRS(true, false, false);
+  } else {
+    if (guard) V3D_PAIRS(false, true, true);
+    else V3D_PAIRS(false, true, false);
+  }
+#undef V3D_PAIRS
+  return sum_slices(part, split.nsplit, (long)n_trg * 3, tvel, st);
 }
 
 // ---------------------------------------------------------------------------
-// Far field between groups with the sources read through the scalar cache.
-// Every lane of a wave uses the same source at the same time, so the source
-// records are loaded with uniform addresses (s_load into SGPRs, which the
-// VALU reads as operands): no LDS staging, no barriers, and the per-pair
-// instruction stream is the arithmetic alone.  Records are packed once per
-// call; the FP32 form stores each source relative to its group's first point
-// (the group anchor, FP64), and the lane shifts its target by the same anchor
-// in FP64 before rounding, as the LDS form does per tile.
-struct __align__(16) FarRec64 {
-  double x, y, z, fx, fy, fz, _p0, _p1;
+// Far field between groups, with several source levels.  Every group
+// (vesicle) carries its fine sources (the upsampled surface) and, optionally,
+// coarser ones: level 1 the surface at its own order with its own quadrature
+// weights, level 2 a lower order still.  flags[w][g] names the level wave w
+// (targets 64 w .. 64 w + 63) reads group g at: level l where every target of
+// the wave is at least kappa_l times g's radius from g's centre, so that the
+// coarser quadrature is as accurate as the fine one there (null: the fine
+// level everywhere; the flags never name an absent level).  The level, the
+// record base and the count are wave-uniform (SGPRs).  A wave whose targets
+// all belong to group g skips g.
+constexpr int kMaxLevels = 3;
+struct LevelSizes {
+  int cnt[kMaxLevels];   // sources per group
+  int plen[kMaxLevels];  // sources per part of a group
 };
-struct __align__(16) FarRec32 {
-  float x, y, z, fx, fy, fz, _p0, _p1;
+// The wave's level flags, 64 groups at a time in one register across the
+// lanes: a flag in the source loop is then a v_readlane, not a load that
+// everything after it waits for.
+struct WaveFlags {
+  const unsigned char *row;  // null: level 0 everywhere
+  unsigned n_groups, base;
+  int v;
+  __device__ __forceinline__ void load(unsigned g) {
+    base = g;
+    const unsigned i = g + (threadIdx.x & 63);
+    v = i < n_groups ? row[i] : 0;
+  }
+  __device__ __forceinline__ int level(unsigned g) {
+    if (!row) return 0;
+    if (g - base >= 64) load(g);
+    return __builtin_amdgcn_readlane(v, (int)(g - base));
+  }
 };
-
-__global__ void k_pack_far64(const double *__restrict__ spos, const double *__restrict__ sld,
-                             long n, FarRec64 *__restrict__ rec) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  FarRec64 r;
-  r.x = spos[3 * i];
-  r.y = spos[3 * i + 1];
-  r.z = spos[3 * i + 2];
-  r.fx = sld[3 * i];
-  r.fy = sld[3 * i + 1];
-  r.fz = sld[3 * i + 2];
-  r._p0 = r._p1 = 0.0;
-  rec[i] = r;
-}
-// FP32 records relative to the group's anchor anc[3 (i / spg) apg] (the
-// first fine source of the group, for both levels).
-__global__ void k_pack_far32(const double *__restrict__ spos, const double *__restrict__ sld,
-                             long n, long spg, const double *__restrict__ anc, long apg,
-                             FarRec32 *__restrict__ rec) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const double *a = anc + 3 * (i / spg) * apg;
-  FarRec32 r;
-  r.x = (float)(spos[3 * i] - a[0]);
-  r.y = (float)(spos[3 * i + 1] - a[1]);
-  r.z = (float)(spos[3 * i + 2] - a[2]);
-  r.fx = (float)sld[3 * i];
-  r.fy = (float)sld[3 * i + 1];
-  r.fz = (float)sld[3 * i + 2];
-  r._p0 = r._p1 = 0.0f;
-  rec[i] = r;
+__device__ __forceinline__ WaveFlags wave_flags(const unsigned char *flags, long row,
+                                                unsigned n_groups, unsigned g0) {
+  WaveFlags f{flags ? flags + row * n_groups : nullptr, n_groups, 0, 0};
+  if (flags) f.load(g0);
+  return f;
 }
 
-// The r^2 bias that removes a target's own group from the FP64 sums (see
-// kOwnGroupBias below): about 1e-15 |f| per own-group source.
-constexpr double kOwnGroupBias64 = 1e30;
-
-// Multi-level sources.  Every group (vesicle) carries its fine sources (spg
-// records: the upsampled surface) and, optionally, coarser ones: level 1
-// the surface at its own order with its own quadrature weights, level 2 a
-// lower order still.  flags[w][g] names the level wave w (targets 64 w ..
-// 64 w + 63) reads group g at: level l where every target of the wave is at
-// least kappa_l times g's radius from g's centre, so that the coarser
-// quadrature is as accurate as the fine one there.  The level, the record
-// base and the count are wave-uniform (SGPRs), so the source loop keeps its
-// scalar addressing.  A wave whose targets all belong to group g skips g.
-struct WaveSpan {
-  long row, first, last;  // flag row (clamped to the last wave), first and last target
-  long own;               // the group that holds all the wave's targets, or -1
-};
-// The divisions run once per wave here, not once per group in the source
-// loops (a 64-bit division is a long scalar sequence).
-__device__ __forceinline__ WaveSpan wave_span(long tb, long n_trg, long tpg) {
-  const long wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const long w = tb * (FF_BLOCK / 64) + wv;
-  const long n_waves = (n_trg + 63) / 64;
-  WaveSpan r;
-  r.row = w < n_waves ? w : n_waves - 1;
-  r.first = w * 64;
-  r.last = min(r.first + 64, n_trg) - 1;
-  const long gf = r.first / tpg, gl = r.last / tpg;
-  r.own = gf == gl ? gf : -1;
-  return r;
+template <int ND>
+__device__ __forceinline__ void store_pass(const WaveTargets &w, unsigned share, unsigned slice,
+                                           long n_trg, const double (&v)[3 * ND], double *part1,
+                                           double *part2) {
+  const long o = (long)slice * n_trg * 3;
+  const double a[3] = {v[0], v[1], v[2]};
+  store_sums(w, share, n_trg, a, part1 + o);
+  if constexpr (ND == 2) {
+    const double b[3] = {v[3], v[4], v[5]};
+    if (share > 1) __syncthreads();  // the first sums have left LDS
+    store_sums(w, share, n_trg, b, part2 + o);
+  }
 }
 
-// The source levels of the far field between groups: level 0 the fine
-// records (spg per group), levels 1 and 2 coarser ones (cnt[l] per group,
-// 0: absent); flags[w][g] names the level wave w reads group g at (null:
-// level 0 everywhere).  The flags never name an absent level.
-template <typename Rec>
-struct FarLevels {
-  const Rec *rec[3];
-  long cnt[3];
+// FP64 levels: point-major positions and densities as they lie.  ND: number
+// of densities on the same sources (the step's right-hand side and its first
+// matvec): the pair geometry (d, r^2, 1/r, 1/r^2) is computed once and serves
+// both Stokeslet sums.
+struct FarLevels64 {
+  const double *pos[kMaxLevels], *den[2][kMaxLevels];
+  LevelSizes n;
   const unsigned char *flags;
-  __device__ __forceinline__ int level(long row, long n_groups, long g) const {
-    return flags ? (int)flags[row * n_groups + g] : 0;
-  }
 };
-
+template <int ND>
 __global__ __launch_bounds__(FF_BLOCK) void k_far_groups_f64(
-    const FarLevels<FarRec64> L, long spg, long n_groups, const double *__restrict__ tpos,
-    long n_trg, long tpg, int nsplit, double csl, double *__restrict__ part) {
-  const long slice = blockIdx.x % nsplit;
-  const long tb = blockIdx.x / nsplit;
-  const long t = tb * FF_BLOCK + threadIdx.x;
-  const bool tvalid = t < n_trg;
-  // lanes past the last target compute for it and store nothing, and a
-  // target's own group enters through an r^2 bias, so the source loop's
-  // control flow is uniform (its addressing stays scalar)
-  const long tc = tvalid ? t : n_trg - 1;
-  const double tx = tpos[3 * tc], ty = tpos[3 * tc + 1], tz = tpos[3 * tc + 2];
-  const long my_g = tc / tpg;
-  const WaveSpan ws = wave_span(tb, n_trg, tpg);
-  double Sx = 0, Sy = 0, Sz = 0;
-  long g0, g1;
-  slice_range(slice, nsplit, 0, spg, n_groups, g0, g1);
-  for (long g = g0; g < g1; ++g) {
-    if (g == ws.own) continue;  // wave-uniform skip
-    const double bias = my_g == g ? kOwnGroupBias64 : 0.0;
-    const int lv = L.level(ws.row, n_groups, g);
-    const FarRec64 *__restrict__ r = L.rec[lv] + g * L.cnt[lv];
-    const int ns = (int)L.cnt[lv];
-#pragma unroll 4
-    for (int j = 0; j < ns; ++j) {
-      const FarRec64 s = r[j];
-      const double dx = tx - s.x, dy = ty - s.y, dz = tz - s.z;
-      const double r2 = fma(dz, dz, fma(dy, dy, fma(dx, dx, bias)));
-      const double ri = rsqrt_pair(r2);
-      const double ri2 = ri * ri;
-      const double ip = (s.fx * dx + s.fy * dy + s.fz * dz) * ri2;
-      Sx += ri * (s.fx + dx * ip);
-      Sy += ri * (s.fy + dy * ip);
-      Sz += ri * (s.fz + dz * ip);
-    }
-  }
-  if (tvalid) {
-    double *o = part + (slice * n_trg + t) * 3;
-    o[0] = csl * Sx;
-    o[1] = csl * Sy;
-    o[2] = csl * Sz;
-  }
-}
-
-// FP32 partial sums merged into a TwoSum (hi, lo) pair, and the r^2 bias that
-// removes a target's own group: each own-group source then adds about
-// 1e-15 |f| (the coincident one included, without a NaN), far below FP32
-// resolution of the sum.
-struct Acc32 {
-  float h[3], l[3];
-};
-__device__ __forceinline__ void acc_merge(Acc32 &a, float x, float y, float z) {
-  float s_, e_;
-  two_sum(a.h[0], x, s_, e_); a.h[0] = s_; a.l[0] += e_;
-  two_sum(a.h[1], y, s_, e_); a.h[1] = s_; a.l[1] += e_;
-  two_sum(a.h[2], z, s_, e_); a.h[2] = s_; a.l[2] += e_;
-}
-constexpr float kOwnGroupBias = 1e30f;
-
-__global__ __launch_bounds__(FF_BLOCK) void k_far_groups_f32c(
-    const FarLevels<FarRec32> L, const double *__restrict__ spos, long spg, long n_groups,
-    const double *__restrict__ tpos, long n_trg, long tpg, int nsplit, double csl,
-    double *__restrict__ part) {
-  const long slice = blockIdx.x % nsplit;
-  const long tb = blockIdx.x / nsplit;
-  const long t = tb * FF_BLOCK + threadIdx.x;
-  const bool tvalid = t < n_trg;
-  // a lane past the last target computes for the last one and stores nothing,
-  // so that control flow inside the group loop stays uniform
-  const long tc = tvalid ? t : n_trg - 1;
-  const double tx = tpos[3 * tc], ty = tpos[3 * tc + 1], tz = tpos[3 * tc + 2];
-  const long my_g = tc / tpg;
-  const WaveSpan ws = wave_span(tb, n_trg, tpg);
-  Acc32 S = {{0, 0, 0}, {0, 0, 0}};
-  long g0, g1;
-  slice_range(slice, nsplit, 0, spg, n_groups, g0, g1);
-  for (long g = g0; g < g1; ++g) {
-    if (g == ws.own) continue;  // wave-uniform skip
-    // a target's own group is not skipped lane by lane (that would make the
-    // loop below divergent): its r^2 carries kOwnGroupBias instead
-    const float bias = my_g == g ? kOwnGroupBias : 0.0f;
-    const double *a = spos + 3 * g * spg;  // the group's anchor (every level)
-    const float lx = (float)(tx - a[0]), ly = (float)(ty - a[1]), lz = (float)(tz - a[2]);
-    const int lv = L.level(ws.row, n_groups, g);
-    const FarRec32 *__restrict__ r = L.rec[lv] + g * L.cnt[lv];
-    const long cnt = L.cnt[lv];
-    auto chunk = [&](const FarRec32 *__restrict__ rr, int n, float &sx, float &sy,
-                     float &sz) {
-      auto pair = [&](const FarRec32 &src) {
-        const float dx = lx - src.x, dy = ly - src.y, dz = lz - src.z;
-        const float r2 = fmaf(dz, dz, fmaf(dy, dy, fmaf(dx, dx, bias)));
-        const float ri = __frsqrt_rn(r2);
-        const float ri2 = ri * ri;
-        const float ip = (src.fx * dx + src.fy * dy + src.fz * dz) * ri2;
-        sx += ri * (src.fx + dx * ip);
-        sy += ri * (src.fy + dy * ip);
-        sz += ri * (src.fz + dz * ip);
-      };
-      if (n == FF_SUB) {
-#pragma unroll 8
-        for (int j = 0; j < FF_SUB; ++j) pair(rr[j]);
-      } else {
-        for (int j = 0; j < n; ++j) pair(rr[j]);
-      }
-    };
-    for (long j0 = 0; j0 < cnt; j0 += FF_SUB) {
-      float sx = 0, sy = 0, sz = 0;
-      chunk(r + j0, (int)min((long)FF_SUB, cnt - j0), sx, sy, sz);
-      acc_merge(S, sx, sy, sz);
-    }
-  }
-  if (tvalid) {
-    double *o = part + (slice * n_trg + t) * 3;
-#pragma unroll
-    for (int c = 0; c < 3; ++c) o[c] = csl * ((double)S.h[c] + (double)S.l[c]);
-  }
-}
-
-// Two targets per lane (t and t + FF_BLOCK): each source record loaded
-// through the scalar cache serves two pairs.  A target must not see its own
-// group's sources; instead of a lane-divergent skip (which would move the
-// source addressing out of SGPRs), its r^2 carries a bias of 1e30 for that
-// group, folded into the fma chain at no cost: each such source then adds
-// about 1e-15 |f| (including the coincident one, without a NaN), some 1e-14
-// of the sum and far below FP32 resolution.
-
-__global__ __launch_bounds__(FF_BLOCK) void k_far_groups_f32c2(
-    const FarRec32 *__restrict__ rec, const double *__restrict__ spos, long spg, long n_groups,
-    const double *__restrict__ tpos, long n_trg, long tpg, int nsplit, double csl,
-    double *__restrict__ part) {
-  const long slice = blockIdx.x % nsplit;
-  const long tb = blockIdx.x / nsplit;
-  const long ta = tb * (2 * FF_BLOCK) + threadIdx.x, tbb = ta + FF_BLOCK;
-  const bool va = ta < n_trg, vb = tbb < n_trg;
-  const long ca = va ? ta : n_trg - 1, cb = vb ? tbb : n_trg - 1;
-  const double Ax = tpos[3 * ca], Ay = tpos[3 * ca + 1], Az = tpos[3 * ca + 2];
-  const double Bx = tpos[3 * cb], By = tpos[3 * cb + 1], Bz = tpos[3 * cb + 2];
-  const long ga = ca / tpg, gbb = cb / tpg;
-  const long tfirst = tb * (2 * FF_BLOCK);
-  const long tlast = min(tfirst + 2 * FF_BLOCK, n_trg) - 1;
-  const long own_b = tfirst / tpg == tlast / tpg ? tfirst / tpg : -1;
-  Acc32 A = {{0, 0, 0}, {0, 0, 0}}, B = {{0, 0, 0}, {0, 0, 0}};
-  long g0, g1;
-  slice_range(slice, nsplit, 0, spg, n_groups, g0, g1);
-  for (long g = g0; g < g1; ++g) {
-    if (g == own_b) continue;  // block-uniform skip
-    const double *a = spos + 3 * g * spg;
-    const float ax = (float)(Ax - a[0]), ay = (float)(Ay - a[1]), az = (float)(Az - a[2]);
-    const float bx = (float)(Bx - a[0]), by = (float)(By - a[1]), bz = (float)(Bz - a[2]);
-    const FarRec32 *__restrict__ r = rec + g * spg;
-    const float bias_a = ga == g ? kOwnGroupBias : 0.0f;
-    const float bias_b = gbb == g ? kOwnGroupBias : 0.0f;
-    for (long j0 = 0; j0 < spg; j0 += FF_SUB) {
-      const long j1 = min(spg, j0 + FF_SUB);
-      float ux = 0, uy = 0, uz = 0, vx = 0, vy = 0, vz = 0;
-#pragma unroll 4
-      for (long j = j0; j < j1; ++j) {
-        const FarRec32 s = r[j];
-        {
-          const float dx = ax - s.x, dy = ay - s.y, dz = az - s.z;
-          const float r2 = fmaf(dx, dx, fmaf(dy, dy, fmaf(dz, dz, bias_a)));
-          const float ri = __frsqrt_rn(r2);
-          const float ri2 = ri * ri;
-          const float ip = (s.fx * dx + s.fy * dy + s.fz * dz) * ri2;
-          ux += ri * (s.fx + dx * ip);
-          uy += ri * (s.fy + dy * ip);
-          uz += ri * (s.fz + dz * ip);
-        }
-        {
-          const float dx = bx - s.x, dy = by - s.y, dz = bz - s.z;
-          const float r2 = fmaf(dx, dx, fmaf(dy, dy, fmaf(dz, dz, bias_b)));
-          const float ri = __frsqrt_rn(r2);
-          const float ri2 = ri * ri;
-          const float ip = (s.fx * dx + s.fy * dy + s.fz * dz) * ri2;
-          vx += ri * (s.fx + dx * ip);
-          vy += ri * (s.fy + dy * ip);
-          vz += ri * (s.fz + dz * ip);
-        }
-      }
-      acc_merge(A, ux, uy, uz);
-      acc_merge(B, vx, vy, vz);
-    }
-  }
-  if (va) {
-    double *o = part + (slice * n_trg + ta) * 3;
-#pragma unroll
-    for (int c = 0; c < 3; ++c) o[c] = csl * ((double)A.h[c] + (double)A.l[c]);
-  }
-  if (vb) {
-    double *o = part + (slice * n_trg + tbb) * 3;
-#pragma unroll
-    for (int c = 0; c < 3; ++c) o[c] = csl * ((double)B.h[c] + (double)B.l[c]);
-  }
-}
-
-// Two densities on the same sources and targets in one pass (the step's
-// right-hand side and the solver's first matvec): the pair geometry (d, r^2,
-// 1/r, 1/r^2) is computed once and serves both Stokeslet sums.
-struct __align__(16) FarRec32x2 {
-  float x, y, z, ax, ay, az, bx, by, bz, _p0, _p1, _p2;
-};
-struct __align__(16) FarRec64x2 {
-  double x, y, z, ax, ay, az, bx, by, bz, _p0, _p1, _p2;
-};
-
-__global__ void k_pack_far32x2(const double *__restrict__ spos, const double *__restrict__ s1,
-                               const double *__restrict__ s2, long n, long spg,
-                               const double *__restrict__ anc, long apg,
-                               FarRec32x2 *__restrict__ rec) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const double *a = anc + 3 * (i / spg) * apg;
-  FarRec32x2 r;
-  r.x = (float)(spos[3 * i] - a[0]);
-  r.y = (float)(spos[3 * i + 1] - a[1]);
-  r.z = (float)(spos[3 * i + 2] - a[2]);
-  r.ax = (float)s1[3 * i];
-  r.ay = (float)s1[3 * i + 1];
-  r.az = (float)s1[3 * i + 2];
-  r.bx = (float)s2[3 * i];
-  r.by = (float)s2[3 * i + 1];
-  r.bz = (float)s2[3 * i + 2];
-  r._p0 = r._p1 = r._p2 = 0.0f;
-  rec[i] = r;
-}
-__global__ void k_pack_far64x2(const double *__restrict__ spos, const double *__restrict__ s1,
-                               const double *__restrict__ s2, long n,
-                               FarRec64x2 *__restrict__ rec) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  FarRec64x2 r;
-  r.x = spos[3 * i];
-  r.y = spos[3 * i + 1];
-  r.z = spos[3 * i + 2];
-  r.ax = s1[3 * i];
-  r.ay = s1[3 * i + 1];
-  r.az = s1[3 * i + 2];
-  r.bx = s2[3 * i];
-  r.by = s2[3 * i + 1];
-  r.bz = s2[3 * i + 2];
-  r._p0 = r._p1 = r._p2 = 0.0;
-  rec[i] = r;
-}
-
-__global__ __launch_bounds__(FF_BLOCK) void k_far_groups_f32c_x2(
-    const FarLevels<FarRec32x2> L, const double *__restrict__ spos, long spg, long n_groups,
-    const double *__restrict__ tpos, long n_trg, long tpg, int nsplit, double csl,
-    double *__restrict__ part1, double *__restrict__ part2) {
-  const long slice = blockIdx.x % nsplit;
-  const long tb = blockIdx.x / nsplit;
-  const long t = tb * FF_BLOCK + threadIdx.x;
-  const bool tvalid = t < n_trg;
-  const long tc = tvalid ? t : n_trg - 1;  // uniform control flow, as k_far_groups_f32c
-  const double tx = tpos[3 * tc], ty = tpos[3 * tc + 1], tz = tpos[3 * tc + 2];
-  const long my_g = tc / tpg;
-  const WaveSpan ws = wave_span(tb, n_trg, tpg);
-  Acc32 A = {{0, 0, 0}, {0, 0, 0}}, B = {{0, 0, 0}, {0, 0, 0}};
-  long g0, g1;
-  slice_range(slice, nsplit, 0, spg, n_groups, g0, g1);
-  for (long g = g0; g < g1; ++g) {
-    if (g == ws.own) continue;  // wave-uniform skip
-    const float bias = my_g == g ? kOwnGroupBias : 0.0f;
-    const double *a = spos + 3 * g * spg;
-    const float lx = (float)(tx - a[0]), ly = (float)(ty - a[1]), lz = (float)(tz - a[2]);
-    const int lv = L.level(ws.row, n_groups, g);
-    const FarRec32x2 *__restrict__ r = L.rec[lv] + g * L.cnt[lv];
-    const long n = L.cnt[lv];
-    for (long j0 = 0; j0 < n; j0 += FF_SUB) {
-      const int cnt = (int)min((long)FF_SUB, n - j0);
-      const FarRec32x2 *__restrict__ rr = r + j0;
-      float ux = 0, uy = 0, uz = 0, vx = 0, vy = 0, vz = 0;
-      auto pair = [&](const FarRec32x2 &src) {
-        const float dx = lx - src.x, dy = ly - src.y, dz = lz - src.z;
-        const float r2 = fmaf(dz, dz, fmaf(dy, dy, fmaf(dx, dx, bias)));
-        const float ri = __frsqrt_rn(r2);
-        const float ri2 = ri * ri;
-        const float ip = (src.ax * dx + src.ay * dy + src.az * dz) * ri2;
-        ux += ri * (src.ax + dx * ip);
-        uy += ri * (src.ay + dy * ip);
-        uz += ri * (src.az + dz * ip);
-        const float iq = (src.bx * dx + src.by * dy + src.bz * dz) * ri2;
-        vx += ri * (src.bx + dx * iq);
-        vy += ri * (src.by + dy * iq);
-        vz += ri * (src.bz + dz * iq);
-      };
-      if (cnt == FF_SUB) {
-#pragma unroll 4
-        for (int j = 0; j < FF_SUB; ++j) pair(rr[j]);
-      } else {
-        for (int j = 0; j < cnt; ++j) pair(rr[j]);
-      }
-      acc_merge(A, ux, uy, uz);
-      acc_merge(B, vx, vy, vz);
-    }
-  }
-  if (tvalid) {
-    double *o1 = part1 + (slice * n_trg + t) * 3, *o2 = part2 + (slice * n_trg + t) * 3;
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-      o1[c] = csl * ((double)A.h[c] + (double)A.l[c]);
-      o2[c] = csl * ((double)B.h[c] + (double)B.l[c]);
-    }
-  }
-}
-
-__global__ __launch_bounds__(FF_BLOCK) void k_far_groups_f64_x2(
-    const FarLevels<FarRec64x2> L, long spg, long n_groups, const double *__restrict__ tpos,
-    long n_trg, long tpg, int nsplit, double csl, double *__restrict__ part1,
+    const FarLevels64 L, unsigned n_groups, const double *__restrict__ tpos, long n_trg, long tpg,
+    SliceMap map, unsigned nsplit, double csl, double *__restrict__ part1,
     double *__restrict__ part2) {
-  const long slice = blockIdx.x % nsplit;
-  const long tb = blockIdx.x / nsplit;
-  const long t = tb * FF_BLOCK + threadIdx.x;
-  const bool tvalid = t < n_trg;
-  const long tc = tvalid ? t : n_trg - 1;  // uniform control flow, as k_far_groups_f64
-  const double tx = tpos[3 * tc], ty = tpos[3 * tc + 1], tz = tpos[3 * tc + 2];
-  const long my_g = tc / tpg;
-  const WaveSpan ws = wave_span(tb, n_trg, tpg);
-  double Sx = 0, Sy = 0, Sz = 0, Tx = 0, Ty = 0, Tz = 0;
-  long g0, g1;
-  slice_range(slice, nsplit, 0, spg, n_groups, g0, g1);
-  for (long g = g0; g < g1; ++g) {
-    if (g == ws.own) continue;  // wave-uniform skip
-    const double bias = my_g == g ? kOwnGroupBias64 : 0.0;
-    const int lv = L.level(ws.row, n_groups, g);
-    const FarRec64x2 *__restrict__ r = L.rec[lv] + g * L.cnt[lv];
-    const int ns = (int)L.cnt[lv];
-#pragma unroll 2
-    for (int j = 0; j < ns; ++j) {
-      const FarRec64x2 s = r[j];
-      const double dx = tx - s.x, dy = ty - s.y, dz = tz - s.z;
-      const double r2 = fma(dz, dz, fma(dy, dy, fma(dx, dx, bias)));
-      const double ri = rsqrt_pair(r2);
-      const double ri2 = ri * ri;
-      const double ip = (s.ax * dx + s.ay * dy + s.az * dz) * ri2;
-      Sx += ri * (s.ax + dx * ip);
-      Sy += ri * (s.ay + dy * ip);
-      Sz += ri * (s.az + dz * ip);
-      const double iq = (s.bx * dx + s.by * dy + s.bz * dz) * ri2;
-      Tx += ri * (s.bx + dx * iq);
-      Ty += ri * (s.by + dy * iq);
-      Tz += ri * (s.bz + dz * iq);
+  const unsigned slice = blockIdx.x % nsplit;
+  const WaveTargets w = wave_targets(blockIdx.x / nsplit, map.share, n_trg, tpg);
+  if (!w.live) return;
+  const double tx = tpos[3 * w.tc], ty = tpos[3 * w.tc + 1], tz = tpos[3 * w.tc + 2];
+  const int own = (int)w.own, group = (int)w.group;
+  double S[ND][3] = {};
+  Slice k = slice_of(map, slice);
+  WaveFlags fl = wave_flags(L.flags, w.row, n_groups, k.g);
+  while (k.u < k.u1) {
+    const unsigned take = min(map.nsub - k.j, k.u1 - k.u);
+    const int g = (int)k.g;
+    if (g != own) {  // wave-uniform skip
+      const double bias = group == g ? kOwnGroupBias64 : 0.0;
+      const int lv = fl.level(g);
+      const int cnt = L.n.cnt[lv], r0 = (int)k.j * L.n.plen[lv];
+      const int n = min((int)take * L.n.plen[lv], cnt - r0);
+      const long s0 = 3 * ((long)g * cnt + r0);
+      const double *__restrict__ p = L.pos[lv] + s0;
+      const double *__restrict__ f = L.den[0][lv] + s0;
+      const double *__restrict__ h = L.den[ND - 1][lv] + s0;
+      auto block = [&](int i, auto uc) {
+        constexpr int U = decltype(uc)::value;
+#pragma unroll
+        for (int k = 0; k < U; ++k) {
+          const int e = 3 * (i + k);
+          const double dx = tx - p[e], dy = ty - p[e + 1], dz = tz - p[e + 2];
+          const double ri = rsqrt_pair(fma(dz, dz, fma(dy, dy, fma(dx, dx, bias))));
+          add_pair<true, false>(dx, dy, dz, ri, f + e, f, 0.0, S[0]);
+          if constexpr (ND == 2) add_pair<true, false>(dx, dy, dz, ri, h + e, h, 0.0, S[1]);
+        }
+      };
+      constexpr int U = ND == 2 ? 2 : 4;
+      int i = 0;
+      for (; i + U <= n; i += U) block(i, std::integral_constant<int, U>());
+      for (; i < n; ++i) block(i, std::integral_constant<int, 1>());
     }
+    k.u += take;
+    k.j = 0;
+    ++k.g;
   }
-  if (tvalid) {
-    double *o1 = part1 + (slice * n_trg + t) * 3, *o2 = part2 + (slice * n_trg + t) * 3;
-    o1[0] = csl * Sx;
-    o1[1] = csl * Sy;
-    o1[2] = csl * Sz;
-    o2[0] = csl * Tx;
-    o2[1] = csl * Ty;
-    o2[2] = csl * Tz;
-  }
+  double v[3 * ND];
+#pragma unroll
+  for (int c = 0; c < 3 * ND; ++c) v[c] = csl * S[c / 3][c % 3];
+  store_pass<ND>(w, map.share, slice, n_trg, v, part1, part2);
 }
 
-// 0: LDS-staged source tiles (k_far_*), 1: scalar-cache source records
-// (k_far_groups_*), 2: as 1 with two targets per lane in the FP32 form;
-// selects the far field between groups.
+// FP32 levels: records (x, y, z, f[, h]) of 3 + 3 ND floats, relative to the
+// group's anchor (its first fine source, for every level).  Measured, three
+// levels of 512 vesicles at p = 16 (3.3e10 pairs): 13.5 ms with one density
+// (15.1 ms with the pairs one after the other in program order, a flag load
+// per group and the counts' remainders one source at a time); 65 VGPRs would
+// cost the eighth wave per SIMD.
+struct FarLevels32 {
+  const float *rec[kMaxLevels];
+  LevelSizes n;
+  const unsigned char *flags;
+};
+template <int ND>
+__global__ void k_pack_far32(const double *__restrict__ spos, const double *__restrict__ s1,
+                             const double *__restrict__ s2, long n, long spg,
+                             const double *__restrict__ anc, long apg, float *__restrict__ rec) {
+  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const double *a = anc + 3 * quot(i, spg) * apg;
+  float *r = rec + i * (3 + 3 * ND);
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    r[c] = (float)(spos[3 * i + c] - a[c]);
+    r[3 + c] = (float)s1[3 * i + c];
+    if constexpr (ND == 2) r[6 + c] = (float)s2[3 * i + c];
+  }
+}
+template <int ND>
+__global__ __launch_bounds__(FF_BLOCK, 8) void k_far_groups_f32c(
+    const FarLevels32 L, const double *__restrict__ spos, unsigned n_groups,
+    const double *__restrict__ tpos, long n_trg, long tpg, SliceMap map, unsigned nsplit,
+    double csl, double *__restrict__ part1, double *__restrict__ part2) {
+  constexpr int R = 3 + 3 * ND;
+  const unsigned slice = blockIdx.x % nsplit;
+  const WaveTargets w = wave_targets(blockIdx.x / nsplit, map.share, n_trg, tpg);
+  if (!w.live) return;
+  const double tx = tpos[3 * w.tc], ty = tpos[3 * w.tc + 1], tz = tpos[3 * w.tc + 2];
+  const int own = (int)w.own, group = (int)w.group;
+  Acc32 A = {{0, 0, 0}, {0, 0, 0}}, B = {{0, 0, 0}, {0, 0, 0}};
+  Slice k = slice_of(map, slice);
+  WaveFlags fl = wave_flags(L.flags, w.row, n_groups, k.g);
+  while (k.u < k.u1) {
+    const unsigned take = min(map.nsub - k.j, k.u1 - k.u);
+    const int g = (int)k.g;
+    if (g != own) {  // wave-uniform skip
+      const float bias = group == g ? kOwnGroupBias : 0.0f;
+      const double *a = spos + 3 * (long)g * L.n.cnt[0];  // the group's anchor
+      const float lx = (float)(tx - a[0]), ly = (float)(ty - a[1]), lz = (float)(tz - a[2]);
+      const int lv = fl.level(g);
+      const int cnt = L.n.cnt[lv], r0 = (int)k.j * L.n.plen[lv];
+      const int r1 = min(cnt, r0 + (int)take * L.n.plen[lv]);
+      const float *__restrict__ r = L.rec[lv] + (long)g * cnt * R;
+      for (int i0 = r0; i0 < r1; i0 += FF_SUB) {
+        const float *__restrict__ rr = r + (long)i0 * R;
+        const int n = min(FF_SUB, r1 - i0);
+        float S[3] = {0, 0, 0}, T[3] = {0, 0, 0};
+        constexpr int U = ND == 2 ? 4 : 8;
+        unsigned m = 0;
+        int i = 0;
+        for (; i + U <= n; i += U)
+          add_block32<U, ND, false, false>(rr + i * R, lx, ly, lz, bias, 0.0f, S, T, m);
+        for (; i < n; ++i)
+          add_block32<1, ND, false, false>(rr + i * R, lx, ly, lz, bias, 0.0f, S, T, m);
+        acc_merge(A, S);
+        if constexpr (ND == 2) acc_merge(B, T);
+      }
+    }
+    k.u += take;
+    k.j = 0;
+    ++k.g;
+  }
+  double v[3 * ND];
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    v[c] = csl * ((double)A.h[c] + (double)A.l[c]);
+    if constexpr (ND == 2) v[3 + c] = csl * ((double)B.h[c] + (double)B.l[c]);
+  }
+  store_pass<ND>(w, map.share, slice, n_trg, v, part1, part2);
+}
+
+// 0: the all-pairs entry points' kernels (k_pairs_*), otherwise
+// k_far_groups_*; selects the far field between groups without coarser levels.
 static std::atomic<int> g_far_kind{1};
 
 // ---------------------------------------------------------------------------
@@ -1066,82 +1044,103 @@ int far_coarse_flags(const double *spos, size_t n_src, size_t spg, const double 
   return launch_status();
 }
 
+// Packed FP32 records of every level (ND densities), or null on failure.
+template <int ND>
+static int pack_levels32(const double *spos, const double *s1, const double *s2, long n_src,
+                         long spg, const FarCoarse *c, long n_groups, hipStream_t st,
+                         FarLevels32 *L) {
+  constexpr size_t rsz = (3 + 3 * ND) * sizeof(float);
+  const long n_c = c ? (long)c->cpg * n_groups : 0, n_c2 = c ? (long)c->cpg2 * n_groups : 0;
+  float *rec = (float *)workspace(kWsFarRecords, n_src * rsz);
+  float *crec = n_c ? (float *)workspace(kWsFarCoarse, n_c * rsz) : nullptr;
+  float *crec2 = n_c2 ? (float *)workspace(kWsFarCoarse2, n_c2 * rsz) : nullptr;
+  if (!rec || (n_c && !crec) || (n_c2 && !crec2)) return VES3D_MEMORY_ERROR;
+  k_pack_far32<ND><<<cdiv(n_src, 256), 256, 0, st>>>(spos, s1, s2, n_src, spg, spos, spg, rec);
+  V3D_CHECK(launch_status());
+  if (n_c) {
+    k_pack_far32<ND><<<cdiv(n_c, 256), 256, 0, st>>>(c->pos, c->den1, c->den2, n_c, (long)c->cpg,
+                                                     spos, spg, crec);
+    V3D_CHECK(launch_status());
+  }
+  if (n_c2) {
+    k_pack_far32<ND><<<cdiv(n_c2, 256), 256, 0, st>>>(c->pos2, c->l2den1, c->l2den2, n_c2,
+                                                      (long)c->cpg2, spos, spg, crec2);
+    V3D_CHECK(launch_status());
+  }
+  L->rec[0] = rec;
+  L->rec[1] = crec;
+  L->rec[2] = crec2;
+  return VES3D_SUCCESS;
+}
+
+// ND densities s1 (and s2) on the same sources, one pass.
+template <int ND>
+static int far_groups(bool f32c, const double *spos, const double *s1, const double *s2,
+                      size_t n_src, const double *tpos, double *tvel1, double *tvel2,
+                      size_t n_trg, size_t spg, size_t tpg, hipStream_t st,
+                      const FarCoarse *coarse) {
+  if (n_trg == 0) return VES3D_SUCCESS;
+  if (!spos || !s1 || !tpos || !tvel1 || (ND == 2 && (!s2 || !tvel2)))
+    return VES3D_INVALID_PARAMETER;
+  if (n_src % spg || n_trg % tpg || n_src / spg != n_trg / tpg) return VES3D_INVALID_PARAMETER;
+  if (coarse && !coarse_valid(*coarse, ND == 2)) return VES3D_INVALID_PARAMETER;
+  const double csl = 1.0 / (8.0 * kPi);
+  const long n_groups = (long)(n_src / spg);
+  if (n_groups > 0x7fffffffL || spg > 0x7fffffffUL) return VES3D_INVALID_PARAMETER;
+  const Split split = choose_split((long)n_trg, n_groups, (long)spg);
+  const size_t per_pass = (size_t)split.nsplit * n_trg * 3;
+  double *part = (double *)workspace(kWsFarPartial, ND * per_pass * sizeof(double));
+  if (!part) return VES3D_MEMORY_ERROR;
+  double *part2 = part + (ND - 1) * per_pass;
+  LevelSizes n;
+  const long cnt[kMaxLevels] = {(long)spg, coarse ? (long)coarse->cpg : 0,
+                                coarse ? (long)coarse->cpg2 : 0};
+  for (int l = 0; l < kMaxLevels; ++l) {
+    n.cnt[l] = (int)cnt[l];
+    n.plen[l] = (int)part_length(cnt[l], split.map.nsub, f32c ? 8 : 4);
+  }
+  const unsigned char *flags = coarse ? coarse->flags : nullptr;
+  const dim3 grid = split_grid(split, (long)n_trg);
+  if (f32c) {
+    FarLevels32 L{};
+    V3D_CHECK(pack_levels32<ND>(spos, s1, s2, (long)n_src, (long)spg, coarse, n_groups, st, &L));
+    L.n = n;
+    L.flags = flags;
+    k_far_groups_f32c<ND><<<grid, FF_BLOCK, 0, st>>>(L, spos, (unsigned)n_groups, tpos, (long)n_trg,
+                                                     (long)tpg, split.map, (unsigned)split.nsplit,
+                                                     csl, part, part2);
+  } else {
+    FarLevels64 L{};
+    L.pos[0] = spos;
+    L.den[0][0] = s1;
+    L.den[1][0] = s2;
+    if (coarse) {
+      L.pos[1] = coarse->pos;
+      L.den[0][1] = coarse->den1;
+      L.den[1][1] = coarse->den2;
+      L.pos[2] = coarse->pos2;
+      L.den[0][2] = coarse->l2den1;
+      L.den[1][2] = coarse->l2den2;
+    }
+    L.n = n;
+    L.flags = flags;
+    k_far_groups_f64<ND><<<grid, FF_BLOCK, 0, st>>>(L, (unsigned)n_groups, tpos, (long)n_trg,
+                                                    (long)tpg, split.map, (unsigned)split.nsplit,
+                                                    csl, part, part2);
+  }
+  V3D_CHECK(launch_status());
+  V3D_CHECK(sum_slices(part, split.nsplit, (long)n_trg * 3, tvel1, st));
+  return ND == 2 ? sum_slices(part2, split.nsplit, (long)n_trg * 3, tvel2, st) : VES3D_SUCCESS;
+}
+
 int far_field_between_groups(bool f32c, const double *spos, const double *sld, size_t n_src,
                              const double *tpos, double *tvel, size_t n_trg, size_t spg,
                              size_t tpg, hipStream_t st, const FarCoarse *coarse) {
   if (spg == 0 || tpg == 0) return VES3D_INVALID_PARAMETER;
-  const double csl = 1.0 / (8.0 * kPi), cdl = 3.0 / (4.0 * kPi);
-  if (!coarse && g_far_kind.load() == 0) {
-    if (f32c)
-      return far_eval<true>(spos, sld, nullptr, n_src, tpos, tvel, n_trg, spg, tpg, 0.0, csl, cdl, st, false);
-    return far_eval<false>(spos, sld, nullptr, n_src, tpos, tvel, n_trg, spg, tpg, 0.0, csl, cdl, st, false);
-  }
-  if (n_trg == 0) return VES3D_SUCCESS;
-  if (!spos || !sld || !tpos || !tvel) return VES3D_INVALID_PARAMETER;
-  if (n_src % spg || n_trg % tpg || n_src / spg != n_trg / tpg) return VES3D_INVALID_PARAMETER;
-  if (coarse && !coarse_valid(*coarse, false)) return VES3D_INVALID_PARAMETER;
-  const long n_groups = (long)(n_src / spg);
-  const int ns = choose_nsplit((long)n_trg, (long)n_src, n_groups);
-  const size_t rsz = f32c ? sizeof(FarRec32) : sizeof(FarRec64);
-  double *part = (double *)workspace(kWsFarPartial, (size_t)ns * n_trg * 3 * sizeof(double));
-  void *rec = workspace(kWsFarRecords, n_src * rsz);
-  const long cpg = coarse ? (long)coarse->cpg : 0, n_c = cpg * n_groups;
-  const long cpg2 = coarse ? (long)coarse->cpg2 : 0, n_c2 = cpg2 * n_groups;
-  void *crec = coarse ? workspace(kWsFarCoarse, n_c * rsz) : nullptr;
-  void *crec2 = cpg2 ? workspace(kWsFarCoarse2, n_c2 * rsz) : nullptr;
-  if (!part || !rec || (coarse && !crec) || (cpg2 && !crec2)) return VES3D_MEMORY_ERROR;
-  const unsigned char *cflag = coarse ? coarse->flags : nullptr;
-  const long tblocks = ((long)n_trg + FF_BLOCK - 1) / FF_BLOCK;
-  const dim3 grid((unsigned)(tblocks * ns));
-  if (f32c) {
-    k_pack_far32<<<cdiv((long)n_src, 256), 256, 0, st>>>(spos, sld, (long)n_src, (long)spg, spos,
-                                                          (long)spg, (FarRec32 *)rec);
-    V3D_CHECK(launch_status());
-    if (coarse) {
-      k_pack_far32<<<cdiv(n_c, 256), 256, 0, st>>>(coarse->pos, coarse->den1, n_c, cpg, spos,
-                                                    (long)spg, (FarRec32 *)crec);
-      V3D_CHECK(launch_status());
-    }
-    if (cpg2) {
-      k_pack_far32<<<cdiv(n_c2, 256), 256, 0, st>>>(coarse->pos2, coarse->l2den1, n_c2, cpg2,
-                                                     spos, (long)spg, (FarRec32 *)crec2);
-      V3D_CHECK(launch_status());
-    }
-    if (!coarse && g_far_kind.load() == 2) {
-      const long tb2 = ((long)n_trg + 2 * FF_BLOCK - 1) / (2 * FF_BLOCK);
-      k_far_groups_f32c2<<<dim3((unsigned)(tb2 * ns)), FF_BLOCK, 0, st>>>(
-          (const FarRec32 *)rec, spos, (long)spg, n_groups, tpos, (long)n_trg, (long)tpg, ns, csl,
-          part);
-    } else {
-      const FarLevels<FarRec32> L{
-          {(const FarRec32 *)rec, (const FarRec32 *)crec, (const FarRec32 *)crec2},
-          {(long)spg, cpg, cpg2}, cflag};
-      k_far_groups_f32c<<<grid, FF_BLOCK, 0, st>>>(L, spos, (long)spg, n_groups, tpos,
-                                                   (long)n_trg, (long)tpg, ns, csl, part);
-    }
-  } else {
-    k_pack_far64<<<cdiv((long)n_src, 256), 256, 0, st>>>(spos, sld, (long)n_src, (FarRec64 *)rec);
-    V3D_CHECK(launch_status());
-    if (coarse) {
-      k_pack_far64<<<cdiv(n_c, 256), 256, 0, st>>>(coarse->pos, coarse->den1, n_c,
-                                                    (FarRec64 *)crec);
-      V3D_CHECK(launch_status());
-    }
-    if (cpg2) {
-      k_pack_far64<<<cdiv(n_c2, 256), 256, 0, st>>>(coarse->pos2, coarse->l2den1, n_c2,
-                                                     (FarRec64 *)crec2);
-      V3D_CHECK(launch_status());
-    }
-    const FarLevels<FarRec64> L{
-        {(const FarRec64 *)rec, (const FarRec64 *)crec, (const FarRec64 *)crec2},
-        {(long)spg, cpg, cpg2}, cflag};
-    k_far_groups_f64<<<grid, FF_BLOCK, 0, st>>>(L, (long)spg, n_groups, tpos, (long)n_trg,
-                                                (long)tpg, ns, csl, part);
-  }
-  V3D_CHECK(launch_status());
-  const long n = (long)n_trg * 3;
-  k_sum_slices<<<cdiv(n, 256), 256, 0, st>>>(part, ns, n, tvel);
-  return launch_status();
+  if (!coarse && g_far_kind.load() == 0)
+    return far_field_sl_dl(f32c, spos, sld, nullptr, n_src, tpos, tvel, n_trg, spg, tpg, false, st);
+  return far_groups<1>(f32c, spos, sld, nullptr, n_src, tpos, tvel, nullptr, n_trg, spg, tpg, st,
+                       coarse);
 }
 
 int far_field_between_groups2(bool f32c, const double *spos, const double *sld1,
@@ -1149,77 +1148,12 @@ int far_field_between_groups2(bool f32c, const double *spos, const double *sld1,
                               double *tvel2, size_t n_trg, size_t spg, size_t tpg,
                               hipStream_t st, const FarCoarse *coarse) {
   if (spg == 0 || tpg == 0) return VES3D_INVALID_PARAMETER;
-  if (!coarse && g_far_kind.load() != 1) {  // the other kernels evaluate one density at a time
+  if (!coarse && g_far_kind.load() == 0) {  // one density at a time
     V3D_CHECK(far_field_between_groups(f32c, spos, sld1, n_src, tpos, tvel1, n_trg, spg, tpg, st));
     return far_field_between_groups(f32c, spos, sld2, n_src, tpos, tvel2, n_trg, spg, tpg, st);
   }
-  if (n_trg == 0) return VES3D_SUCCESS;
-  if (!spos || !sld1 || !sld2 || !tpos || !tvel1 || !tvel2) return VES3D_INVALID_PARAMETER;
-  if (n_src % spg || n_trg % tpg || n_src / spg != n_trg / tpg) return VES3D_INVALID_PARAMETER;
-  if (coarse && !coarse_valid(*coarse, true)) return VES3D_INVALID_PARAMETER;
-  const double csl = 1.0 / (8.0 * kPi);
-  const long n_groups = (long)(n_src / spg);
-  const int ns = choose_nsplit((long)n_trg, (long)n_src, n_groups);
-  const size_t rsz = f32c ? sizeof(FarRec32x2) : sizeof(FarRec64x2);
-  double *part = (double *)workspace(kWsFarPartial, (size_t)2 * ns * n_trg * 3 * sizeof(double));
-  void *rec = workspace(kWsFarRecords, n_src * rsz);
-  const long cpg = coarse ? (long)coarse->cpg : 0, n_c = cpg * n_groups;
-  const long cpg2 = coarse ? (long)coarse->cpg2 : 0, n_c2 = cpg2 * n_groups;
-  void *crec = coarse ? workspace(kWsFarCoarse, n_c * rsz) : nullptr;
-  void *crec2 = cpg2 ? workspace(kWsFarCoarse2, n_c2 * rsz) : nullptr;
-  if (!part || !rec || (coarse && !crec) || (cpg2 && !crec2)) return VES3D_MEMORY_ERROR;
-  const unsigned char *cflag = coarse ? coarse->flags : nullptr;
-  double *part2 = part + (size_t)ns * n_trg * 3;
-  const long tblocks = ((long)n_trg + FF_BLOCK - 1) / FF_BLOCK;
-  const dim3 grid((unsigned)(tblocks * ns));
-  if (f32c) {
-    k_pack_far32x2<<<cdiv((long)n_src, 256), 256, 0, st>>>(spos, sld1, sld2, (long)n_src,
-                                                            (long)spg, spos, (long)spg,
-                                                            (FarRec32x2 *)rec);
-    V3D_CHECK(launch_status());
-    if (coarse) {
-      k_pack_far32x2<<<cdiv(n_c, 256), 256, 0, st>>>(coarse->pos, coarse->den1, coarse->den2,
-                                                      n_c, cpg, spos, (long)spg,
-                                                      (FarRec32x2 *)crec);
-      V3D_CHECK(launch_status());
-    }
-    if (cpg2) {
-      k_pack_far32x2<<<cdiv(n_c2, 256), 256, 0, st>>>(coarse->pos2, coarse->l2den1,
-                                                       coarse->l2den2, n_c2, cpg2, spos,
-                                                       (long)spg, (FarRec32x2 *)crec2);
-      V3D_CHECK(launch_status());
-    }
-    const FarLevels<FarRec32x2> L{
-        {(const FarRec32x2 *)rec, (const FarRec32x2 *)crec, (const FarRec32x2 *)crec2},
-        {(long)spg, cpg, cpg2}, cflag};
-    k_far_groups_f32c_x2<<<grid, FF_BLOCK, 0, st>>>(L, spos, (long)spg, n_groups, tpos,
-                                                    (long)n_trg, (long)tpg, ns, csl, part, part2);
-  } else {
-    k_pack_far64x2<<<cdiv((long)n_src, 256), 256, 0, st>>>(spos, sld1, sld2, (long)n_src,
-                                                            (FarRec64x2 *)rec);
-    V3D_CHECK(launch_status());
-    if (coarse) {
-      k_pack_far64x2<<<cdiv(n_c, 256), 256, 0, st>>>(coarse->pos, coarse->den1, coarse->den2,
-                                                      n_c, (FarRec64x2 *)crec);
-      V3D_CHECK(launch_status());
-    }
-    if (cpg2) {
-      k_pack_far64x2<<<cdiv(n_c2, 256), 256, 0, st>>>(coarse->pos2, coarse->l2den1,
-                                                       coarse->l2den2, n_c2, (FarRec64x2 *)crec2);
-      V3D_CHECK(launch_status());
-    }
-    const FarLevels<FarRec64x2> L{
-        {(const FarRec64x2 *)rec, (const FarRec64x2 *)crec, (const FarRec64x2 *)crec2},
-        {(long)spg, cpg, cpg2}, cflag};
-    k_far_groups_f64_x2<<<grid, FF_BLOCK, 0, st>>>(L, (long)spg, n_groups, tpos, (long)n_trg,
-                                                   (long)tpg, ns, csl, part, part2);
-  }
-  V3D_CHECK(launch_status());
-  const long n = (long)n_trg * 3;
-  k_sum_slices<<<cdiv(n, 256), 256, 0, st>>>(part, ns, n, tvel1);
-  V3D_CHECK(launch_status());
-  k_sum_slices<<<cdiv(n, 256), 256, 0, st>>>(part2, ns, n, tvel2);
-  return launch_status();
+  return far_groups<2>(f32c, spos, sld1, sld2, n_src, tpos, tvel1, tvel2, n_trg, spg, tpg, st,
+                       coarse);
 }
 
 }  // namespace v3d
