@@ -69,21 +69,57 @@ __global__ __launch_bounds__(256) void k_diff_loss(const float *__restrict__ Y,
   __syncthreads();
   if (threadIdx.x == 0) part[blockIdx.x] = sh[0] + sh[1] + sh[2] + sh[3];
 }
-__global__ void k_sum_parts(const double *part, int n, double scale, double *out) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
-    double s = 0;
-    for (int i = 0; i < n; ++i) s += part[i];
-    out[0] = s * scale;
-  }
+// The sum of v over a workgroup of 256 (in thread 0), in a fixed order.
+__device__ __forceinline__ double block_sum(double v) {
+  __shared__ double sh[4];
+  v = wave_sum(v);
+  __syncthreads();
+  if (threadIdx.x % 64 == 0) sh[threadIdx.x / 64] = v;
+  __syncthreads();
+  return sh[0] + sh[1] + sh[2] + sh[3];
+}
+// Latency-bound: one workgroup over at most 4096 partials (4 us; one thread
+// adding them in turn took 218 us).
+__global__ __launch_bounds__(256) void k_sum_parts(const double *__restrict__ part, int n,
+                                                   double scale, double *out) {
+  double s = 0;
+  for (int i = threadIdx.x; i < n; i += 256) s += part[i];
+  s = block_sum(s);
+  if (threadIdx.x == 0) out[0] = s * scale;
 }
 __global__ void k_gelu_back(float *dH, const float *__restrict__ A, long n) {
   GL(i, n) dH[i] *= gelu_g(A[i]);
 }
-__global__ void k_colsum(const float *__restrict__ D, long B, int w, float *g) {
-  GL(c, (long)w) {
-    float s = 0;
-    for (long r = 0; r < B; ++r) s += D[r * w + c];
-    g[c] = s;
+// Bias gradients: the column sums of the three layers' output gradients
+// D_l [B][w_l] in one launch.  Latency-bound (5 MB at a batch of 1024): a
+// workgroup takes 32 columns, 32 threads down each in steps of 32 rows, so
+// that the reads are 128-byte runs and every column has 32 chains of loads in
+// flight; the 32 partial sums are added in FP64 in order.  One thread per
+// column took 227 us per layer, 0.7 ms of a 1.2 ms minibatch.
+struct BiasGrads {
+  const float *D[3];
+  float *g[3];
+  int w[3];
+};
+__global__ __launch_bounds__(1024) void k_bias_grads(const BiasGrads a, long B) {
+  __shared__ float sh[32][33];
+  const int c = threadIdx.x & 31, q = threadIdx.x >> 5;
+  int l = 0, blk = blockIdx.x;
+  while (blk >= (a.w[l] + 31) / 32) blk -= (a.w[l++] + 31) / 32;
+  const int w = a.w[l], col = blk * 32 + c;
+  float s = 0;
+  if (col < w) {
+    const float *__restrict__ D = a.D[l] + col;
+#pragma unroll 8
+    for (long r = q; r < B; r += 32) s += D[r * w];
+  }
+  sh[q][c] = s;
+  __syncthreads();
+  if (q == 0 && col < w) {
+    double t = 0;
+#pragma unroll
+    for (int k = 0; k < 32; ++k) t += (double)sh[k][c];
+    a.g[l][col] = (float)t;
   }
 }
 // ---- BF16 activations on MFMA
@@ -254,16 +290,20 @@ __global__ __launch_bounds__(256) void k_sq_sums(const float *__restrict__ Y,
     part[2 * blockIdx.x + 1] = sh[1][0] + sh[1][1] + sh[1][2] + sh[1][3];
   }
 }
-// acc[0..1] += sums of the nb partial pairs (one thread, fixed order)
-__global__ void k_acc_pairs(const double *part, int nb, double *acc) {
-  if (blockIdx.x != 0 || threadIdx.x != 0) return;
+// acc[0..1] += sums of the nb partial pairs (one workgroup, fixed order)
+__global__ __launch_bounds__(256) void k_acc_pairs(const double *__restrict__ part, int nb,
+                                                   double *acc) {
   double a = 0, b = 0;
-  for (int k = 0; k < nb; ++k) {
+  for (int k = threadIdx.x; k < nb; k += 256) {
     a += part[2 * k];
     b += part[2 * k + 1];
   }
-  acc[0] += a;
-  acc[1] += b;
+  a = block_sum(a);
+  b = block_sum(b);
+  if (threadIdx.x == 0) {
+    acc[0] += a;
+    acc[1] += b;
+  }
 }
 // Adam (Kingma & Ba 2015, Algorithm 1) with decoupled weight decay wd
 // (Loshchilov & Hutter 2019): P -= lr (m_hat / (sqrt(v_hat) + eps) + wd P)
@@ -551,6 +591,12 @@ int LearnedPC::forward(const float *Z, long B, float *Y, hipStream_t st) {
   return launch_status();
 }
 
+int LearnedPC::bias_grads(long B, hipStream_t st) {
+  const BiasGrads a{{dY_, dA2_, dA1_}, {G_ + ob3_, G_ + ob2_, G_ + ob1_}, {nin_, width_, width_}};
+  k_bias_grads<<<cdiv(nin_, 32) + 2 * cdiv(width_, 32), 1024, 0, st>>>(a, B);
+  return launch_status();
+}
+
 int LearnedPC::loss_grad(const float *Z, const float *T, long B, double *loss_host,
                          hipStream_t st) {
   V3D_CHECK(forward(Z, B, Y_, st));
@@ -559,7 +605,7 @@ int LearnedPC::loss_grad(const float *Z, const float *T, long B, double *loss_ho
   const int nb = (int)std::min<long>(4096, std::max<long>(1, (tot + 255) / 256));
   k_diff_loss<<<nb, 256, 0, st>>>(Y_, T, tot, 1.0f / (float)tot, dY_, lossbuf_);
   V3D_CHECK(launch_status());
-  k_sum_parts<<<1, 64, 0, st>>>(lossbuf_, nb, 0.5 / (double)tot, lossbuf_ + 4100);
+  k_sum_parts<<<1, 256, 0, st>>>(lossbuf_, nb, 0.5 / (double)tot, lossbuf_ + 4100);
   V3D_CHECK(launch_status());
   if (act_ == 1) {
     // BF16 operands of every product, FP32 gradients and bias sums
@@ -568,20 +614,15 @@ int LearnedPC::loss_grad(const float *Z, const float *T, long B, double *loss_ho
     k_to_bf16<<<gb(tot), 256, 0, st>>>(dY_, tot, dYh_);
     V3D_CHECK(launch_status());
     V3D_CHECK((gemm_bf16<false, false>(n, w, Bi, dYh_, n, H2h_, w, G_ + oW3_, w, st)));
-    k_colsum<<<gb(n), 256, 0, st>>>(dY_, B, n, G_ + ob3_);
-    V3D_CHECK(launch_status());
     V3D_CHECK((gemm_bf16<true, false>(Bi, w, n, dYh_, n, W3h, w, dA2_, w, st)));
     k_gelu_back_bf<<<gb(B * w), 256, 0, st>>>(dA2_, A2_, B * w, dA2h_);
     V3D_CHECK(launch_status());
     V3D_CHECK((gemm_bf16<false, false>(w, w, Bi, dA2h_, w, H1h_, w, G_ + oW2_, w, st)));
-    k_colsum<<<gb(w), 256, 0, st>>>(dA2_, B, w, G_ + ob2_);
-    V3D_CHECK(launch_status());
     V3D_CHECK((gemm_bf16<true, false>(Bi, w, w, dA2h_, w, W2h, w, dA1_, w, st)));
     k_gelu_back_bf<<<gb(B * w), 256, 0, st>>>(dA1_, A1_, B * w, dA1h_);
     V3D_CHECK(launch_status());
     V3D_CHECK((gemm_bf16<false, false>(w, n, Bi, dA1h_, w, Zh_, n, G_ + oW1_, n, st)));
-    k_colsum<<<gb(w), 256, 0, st>>>(dA1_, B, w, G_ + ob1_);
-    V3D_CHECK(launch_status());
+    V3D_CHECK(bias_grads(B, st));
     if (loss_host) {
       V3D_HIP(hipMemcpyAsync(loss_host, lossbuf_ + 4100, sizeof(double), hipMemcpyDeviceToHost,
                              st));
@@ -591,22 +632,17 @@ int LearnedPC::loss_grad(const float *Z, const float *T, long B, double *loss_ho
   }
   // layer 3
   V3D_CHECK(gemm(n, w, (int)B, dY_, 1, n, H2_, w, 1, G_ + oW3_, st));  // dY^T H2
-  k_colsum<<<gb(n), 256, 0, st>>>(dY_, B, n, G_ + ob3_);
-  V3D_CHECK(launch_status());
   V3D_CHECK(gemm((int)B, w, n, dY_, n, 1, P_ + oW3_, w, 1, dA2_, st));  // dY W3
   k_gelu_back<<<gb(B * w), 256, 0, st>>>(dA2_, A2_, B * w);
   V3D_CHECK(launch_status());
   // layer 2
   V3D_CHECK(gemm(w, w, (int)B, dA2_, 1, w, H1_, w, 1, G_ + oW2_, st));
-  k_colsum<<<gb(w), 256, 0, st>>>(dA2_, B, w, G_ + ob2_);
-  V3D_CHECK(launch_status());
   V3D_CHECK(gemm((int)B, w, w, dA2_, w, 1, P_ + oW2_, w, 1, dA1_, st));
   k_gelu_back<<<gb(B * w), 256, 0, st>>>(dA1_, A1_, B * w);
   V3D_CHECK(launch_status());
   // layer 1
   V3D_CHECK(gemm(w, n, (int)B, dA1_, 1, w, Z, n, 1, G_ + oW1_, st));
-  k_colsum<<<gb(w), 256, 0, st>>>(dA1_, B, w, G_ + ob1_);
-  V3D_CHECK(launch_status());
+  V3D_CHECK(bias_grads(B, st));
   if (loss_host) {
     V3D_HIP(hipMemcpyAsync(loss_host, lossbuf_ + 4100, sizeof(double), hipMemcpyDeviceToHost, st));
     V3D_HIP(hipStreamSynchronize(st));
@@ -644,7 +680,7 @@ int LearnedPC::subset_loss(const int *idx, long m, double *loss_host, double *ta
     const int nb = (int)std::min<long>(kEvalParts, std::max<long>(1, (tot + 255) / 256));
     k_sq_sums<<<nb, 256, 0, st>>>(Y_, Tb_, tot, part);
     V3D_CHECK(launch_status());
-    k_acc_pairs<<<1, 64, 0, st>>>(part, nb, acc);
+    k_acc_pairs<<<1, 256, 0, st>>>(part, nb, acc);
     V3D_CHECK(launch_status());
   }
   double h[2];

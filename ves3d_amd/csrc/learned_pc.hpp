@@ -82,6 +82,7 @@ class LearnedPC {
  private:
   int ensure_batch(long B);
   int refresh_bf16(hipStream_t st);
+  int bias_grads(long B, hipStream_t st);
   int gemm(int M, int N, int K, const float *A, long ars, long acs, const float *Bm, long brs,
            long bcs, float *C, hipStream_t st);
 
