@@ -124,126 +124,203 @@ __global__ __launch_bounds__(1024) void k_bias_grads(const BiasGrads a, long B) 
 }
 // ---- BF16 activations on MFMA
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-// y = bf16(x), round to nearest even
-__global__ void k_to_bf16(const float *__restrict__ x, long n, __bf16 *y) {
-  GL(i, n) y[i] = (__bf16)x[i];
+// Every product of the network has its contracted index contiguous in both
+// operands, C[m][n] = sum_k A[m lda + k] B[n ldb + k]: what a product reads
+// transposed is written transposed by its producer (HT below, and W2^T, W3^T
+// beside the weights), with rows of ldt = B rounded up to 8, zero past B.
+
+// Y[r][c] = bf16(X[r][c]) (round to nearest even) and its transpose
+// YT[c][r] (ldt >= rows, zeros past them); either may be null.  One 32 x 32
+// tile per workgroup.
+struct ToBf16 {
+  const float *X;
+  __bf16 *Y, *YT;
+  int rows, cols, ldt;
+};
+__device__ __forceinline__ void store_transposed(const __bf16 (&sh)[32][34], int r0, int c0,
+                                                 int cols, int ldt, __bf16 *__restrict__ YT) {
+  const int c = threadIdx.x >> 3, r = (threadIdx.x & 7) * 4;
+  if (c0 + c >= cols || r0 + r >= ldt) return;
+  const bf16x4 v = {sh[r][c], sh[r + 1][c], sh[r + 2][c], sh[r + 3][c]};
+  *(bf16x4 *)(YT + (long)(c0 + c) * ldt + r0 + r) = v;
 }
-// A += b (FP32, kept for the backward pass); H = bf16(gelu(A))
-__global__ void k_bias_gelu_bf(float *A, const float *__restrict__ b, long B, int w, __bf16 *H) {
-  GL(i, B * w) {
-    const float a = A[i] + b[i % w];
-    A[i] = a;
-    H[i] = (__bf16)gelu_f(a);
+__global__ __launch_bounds__(256) void k_to_bf16(const ToBf16 a0, const ToBf16 a1,
+                                                 const ToBf16 a2) {
+  __shared__ __bf16 sh[32][34];
+  const ToBf16 a = blockIdx.y == 0 ? a0 : (blockIdx.y == 1 ? a1 : a2);
+  const int ct = (a.cols + 31) / 32;
+  const int r0 = (int)(blockIdx.x / ct) * 32, c0 = (int)(blockIdx.x % ct) * 32;
+  if (r0 >= a.rows) return;
+  const int r = r0 + (threadIdx.x >> 3), c = c0 + (threadIdx.x & 7) * 4;
+  bf16x4 v = {};
+  if (r < a.rows && c < a.cols) {  // cols is a multiple of 4
+    const float *x = a.X + (long)r * a.cols + c;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] = (__bf16)x[u];
+    if (a.Y) *(bf16x4 *)(a.Y + (long)r * a.cols + c) = v;
   }
-}
-// dA *= gelu'(A) (FP32, for the bias gradient); dAh = bf16(dA)
-__global__ void k_gelu_back_bf(float *dA, const float *__restrict__ A, long n, __bf16 *dAh) {
-  GL(i, n) {
-    const float g = dA[i] * gelu_g(A[i]);
-    dA[i] = g;
-    dAh[i] = (__bf16)g;
-  }
+  if (!a.YT) return;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) sh[threadIdx.x >> 3][(threadIdx.x & 7) * 4 + u] = v[u];
+  __syncthreads();
+  store_transposed(sh, r0, c0, a.cols, a.ldt, a.YT);
 }
 
-// C[M][N] (FP32, row stride ldc) = sum_k A(m, k) B(k, n) with BF16 operands
-// on v_mfma_f32_16x16x32_bf16 and FP32 accumulation.
-//   A(m, k) = A[m lda + k] (AK: k contiguous) or A[k lda + m];
-//   B(k, n) = B[n ldb + k] (BK: k contiguous) or B[k ldb + n].
-// A workgroup of 4 waves computes a 64 x 64 tile, each wave 32 x 32 as 2 x 2
-// MFMA tiles, over K slabs of 32 staged through LDS with k contiguous, so
-// that a lane's 8 operands are one 16-byte LDS read: lane l supplies row
-// (l % 16) of A and column (l % 16) of B at the slab's k = 8 (l / 16) .. +7,
-// the same k for both operands (the sum does not depend on which k the
-// instruction assigns to which register, only on A and B agreeing), and
-// holds results of rows 4 (l / 16) + r, column l % 16 (r = 0..3).  Global
-// loads are 16-byte vectors along the contiguous direction; the host
-// requires that extent and the leading dimension to be multiples of 8 and
-// both bases 16-byte aligned, so a vector is either whole in range or whole
-// out of it (then zero).
-constexpr int kBT = 64, kBK = 32, kBPad = 8;
-template <bool AK, bool BK>
+// What becomes of the product's tile (FP32 sums v):
+enum GemmOut {
+  kOutStore,    // C = v
+  kOutBias,     // C = v + bias
+  kOutGelu,     // a = v + bias (to C if given); H = bf16(gelu(a)), HT its transpose
+  kOutGeluOdd,  // H[m] = bf16(gelu(v + bias)), H[M + m] = bf16(gelu(-v + bias))
+  kOutOdd,      // A holds 2 M rows: C = ((v + bias) - (v' + bias)) / 2, v' of row M + m
+  kOutLoss,     // d = v + bias - T; C = d / n, H = bf16(C), HT; part = sum d^2 of the tile
+  kOutBack      // C = v gelu'(P), H = bf16(C), HT (P the pre-activations)
+};
+struct GemmEpi {
+  float *C = nullptr;
+  const float *bias = nullptr, *P = nullptr, *T = nullptr;
+  __bf16 *H = nullptr, *HT = nullptr;
+  double *part = nullptr;
+  float invn = 0.0f;
+  int ldt = 0;
+};
+
+// A workgroup computes a 32 x 32 tile; its four waves take every fourth slab
+// of 32 k and add their sums through LDS in wave order.  The operands go
+// straight from memory to the MFMA registers: lane l supplies row l % 16 of
+// each 16-row strip at k = 8 (l / 16) .. + 7 of the slab, one 16-byte load
+// (the same k for both operands, so the k order inside the instruction does
+// not matter), and holds results of rows 4 (l / 16) + r, column l % 16.
+// Bound: latency.  The products of a minibatch are 0.1-0.6 GFLOP, under a
+// microsecond of matrix work, so what counts is one workgroup per CU and all
+// its loads in flight at once: 64 x 64 tiles through LDS, one slab after the
+// other, took 12-32 us per product, this form 4-8 us at a batch of 1024.
+// Rows past M or N are clamped to the last one and not stored.  The host
+// requires K, lda and ldb multiples of 8 and 16-byte aligned bases, so a
+// vector is whole in range or whole out of it (then zero).
+template <GemmOut OUT>
 __global__ __launch_bounds__(256) void k_gemm_bf16(int M, int N, int K,
                                                    const __bf16 *__restrict__ A, long lda,
                                                    const __bf16 *__restrict__ B, long ldb,
-                                                   float *__restrict__ C, long ldc) {
-  __shared__ __attribute__((aligned(16))) __bf16 As[kBT][kBK + kBPad];
-  __shared__ __attribute__((aligned(16))) __bf16 Bs[kBT][kBK + kBPad];
+                                                   const GemmEpi e) {
+  constexpr int NS = OUT == kOutOdd ? 2 : 1;  // tiles of A that meet the same tile of B
+  __shared__ float red[4][NS][32][33];
+  __shared__ __bf16 sh[32][34];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const long m0 = (long)blockIdx.y * kBT, n0 = (long)blockIdx.x * kBT;
-  const int wm = (w >> 1) * 32, wn = (w & 1) * 32;
   const int li = lane & 15, lg = lane >> 4;
-  f32x4 acc[2][2];
+  const int m0 = blockIdx.x * 32, n0 = blockIdx.y * 32;
+  const __bf16 *pa[NS][2], *pb[2];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < 2; ++i) {
+    const long m = min(m0 + 16 * i + li, M - 1), n = min(n0 + 16 * i + li, N - 1);
 #pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const bf16x8 zero8 = {};
-  for (int k0 = 0; k0 < K; k0 += kBK) {
-    // one 8-vector of each operand per thread: 64 x 32 = 256 vectors
-    if constexpr (AK) {
-      const int m = tid >> 2, kk = (tid & 3) * 8;
-      const long gm = m0 + m, gk = k0 + kk;
-      const bf16x8 v = (gm < M && gk < K) ? *(const bf16x8 *)(A + gm * lda + gk) : zero8;
-      *(bf16x8 *)&As[m][kk] = v;
-    } else {
-      const int kk = tid >> 3, mm = (tid & 7) * 8;
-      const long gm = m0 + mm, gk = k0 + kk;
-      const bf16x8 v = (gm < M && gk < K) ? *(const bf16x8 *)(A + gk * lda + gm) : zero8;
+    for (int h = 0; h < NS; ++h) pa[h][i] = A + (m + (long)h * M) * lda + 8 * lg;
+    pb[i] = B + n * ldb + 8 * lg;
+  }
+  f32x4 acc[NS][2][2] = {};
+  auto slab = [&](int k0, bool whole) {
+    bf16x8 a[NS][2], b[2];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) As[mm + u][kk] = v[u];
+    for (int i = 0; i < 2; ++i) {
+      const bool in = whole || k0 + 8 * lg < K;
+#pragma unroll
+      for (int h = 0; h < NS; ++h) a[h][i] = in ? *(const bf16x8 *)(pa[h][i] + k0) : bf16x8{};
+      b[i] = in ? *(const bf16x8 *)(pb[i] + k0) : bf16x8{};
     }
-    if constexpr (BK) {
-      const int n = tid >> 2, kk = (tid & 3) * 8;
-      const long gn = n0 + n, gk = k0 + kk;
-      const bf16x8 v = (gn < N && gk < K) ? *(const bf16x8 *)(B + gn * ldb + gk) : zero8;
-      *(bf16x8 *)&Bs[n][kk] = v;
-    } else {
-      const int kk = tid >> 3, nn = (tid & 7) * 8;
-      const long gn = n0 + nn, gk = k0 + kk;
-      const bf16x8 v = (gn < N && gk < K) ? *(const bf16x8 *)(B + gk * ldb + gn) : zero8;
 #pragma unroll
-      for (int u = 0; u < 8; ++u) Bs[nn + u][kk] = v[u];
-    }
-    __syncthreads();
-    bf16x8 a[2], b[2];
+    for (int h = 0; h < NS; ++h)
 #pragma unroll
-    for (int i = 0; i < 2; ++i) a[i] = *(const bf16x8 *)&As[wm + 16 * i + li][8 * lg];
+      for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) b[j] = *(const bf16x8 *)&Bs[wn + 16 * j + li][8 * lg];
+        for (int j = 0; j < 2; ++j)
+          acc[h][i][j] =
+              __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[h][i], b[j], acc[h][i][j], 0, 0, 0);
+  };
+  int k0 = 32 * w;
+  for (; k0 + 3 * 128 + 32 <= K; k0 += 4 * 128) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) slab(k0 + 128 * u, true);
+  }
+  for (; k0 + 32 <= K; k0 += 128) slab(k0, true);
+  if (k0 < K) slab(k0, false);
+#pragma unroll
+  for (int h = 0; h < NS; ++h)
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
       for (int j = 0; j < 2; ++j)
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
-    __syncthreads();
+#pragma unroll
+        for (int r = 0; r < 4; ++r) red[w][h][16 * i + 4 * lg + r][16 * j + li] = acc[h][i][j][r];
+  __syncthreads();
+  // four consecutive columns of one row per thread
+  const int tr = tid >> 3, tc = (tid & 7) * 4;
+  const int m = m0 + tr, n = n0 + tc;
+  const bool row = m < M;
+  const long o = (long)m * N + n;
+  double d2 = 0;
+  bf16x4 hv = {};
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    float v[NS];
+#pragma unroll
+    for (int h = 0; h < NS; ++h)
+      v[h] = ((red[0][h][tr][tc + u] + red[1][h][tr][tc + u]) + red[2][h][tr][tc + u]) +
+             red[3][h][tr][tc + u];
+    if (!row || n + u >= N) continue;
+    if constexpr (OUT == kOutStore) {
+      e.C[o + u] = v[0];
+    } else if constexpr (OUT == kOutBias) {
+      e.C[o + u] = v[0] + e.bias[n + u];
+    } else if constexpr (OUT == kOutGelu) {
+      const float a = v[0] + e.bias[n + u];
+      if (e.C) e.C[o + u] = a;
+      hv[u] = (__bf16)gelu_f(a);
+    } else if constexpr (OUT == kOutGeluOdd) {
+      e.H[o + u] = (__bf16)gelu_f(v[0] + e.bias[n + u]);
+      e.H[(long)M * N + o + u] = (__bf16)gelu_f(-v[0] + e.bias[n + u]);
+    } else if constexpr (OUT == kOutOdd) {
+      e.C[o + u] = 0.5f * ((v[0] + e.bias[n + u]) - (v[NS - 1] + e.bias[n + u]));
+    } else if constexpr (OUT == kOutLoss) {
+      const float d = v[0] + e.bias[n + u] - e.T[o + u];
+      e.C[o + u] = d * e.invn;
+      hv[u] = (__bf16)(d * e.invn);
+      d2 += (double)d * d;
+    } else {
+      const float g = v[0] * gelu_g(e.P[o + u]);
+      e.C[o + u] = g;
+      hv[u] = (__bf16)g;
+    }
   }
+  if constexpr (OUT == kOutGelu || OUT == kOutLoss || OUT == kOutBack) {
+    if (e.H && row && n < N) *(bf16x4 *)(e.H + o) = hv;  // N is a multiple of 8
+    if (e.HT) {
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const long gm = m0 + wm + 16 * i + 4 * lg + r, gn = n0 + wn + 16 * j + li;
-        if (gm < M && gn < N) C[gm * ldc + gn] = acc[i][j][r];
-      }
+      for (int u = 0; u < 4; ++u) sh[tr][tc + u] = hv[u];
+      __syncthreads();
+      store_transposed(sh, m0, n0, N, e.ldt, e.HT);
+    }
+  }
+  if constexpr (OUT == kOutLoss) {
+    d2 = block_sum(d2);
+    if (tid == 0) e.part[(long)blockIdx.y * gridDim.x + blockIdx.x] = d2;
+  }
 }
 
-template <bool AK, bool BK>
-int gemm_bf16(int M, int N, int K, const __bf16 *A, long lda, const __bf16 *B, long ldb, float *C,
-              long ldc, hipStream_t st) {
-  if (M < 1 || N < 1 || K < 1) return VES3D_INVALID_PARAMETER;
-  if ((AK ? K : M) % 8 || lda % 8 || (BK ? K : N) % 8 || ldb % 8) return VES3D_INVALID_PARAMETER;
+template <GemmOut OUT>
+int gemm_bf16(long M, int N, long K, const __bf16 *A, long lda, const __bf16 *B, long ldb,
+              const GemmEpi &e, hipStream_t st) {
+  if (M < 1 || N < 1 || K < 1 || K > 0x7fffff00L) return VES3D_INVALID_PARAMETER;
+  if (K % 8 || N % 8 || lda % 8 || ldb % 8) return VES3D_INVALID_PARAMETER;
   if (((uintptr_t)A | (uintptr_t)B) & 15) return VES3D_INVALID_PARAMETER;
-  const long gy = (M + kBT - 1) / kBT;
-  if (gy > 65535) return VES3D_INVALID_PARAMETER;
-  dim3 grid((unsigned)((N + kBT - 1) / kBT), (unsigned)gy);
-  k_gemm_bf16<AK, BK><<<grid, 256, 0, st>>>(M, N, K, A, lda, B, ldb, C, ldc);
+  const unsigned gy = cdiv(N, 32);
+  if (M > 0x7fffff00L || gy > 65535) return VES3D_INVALID_PARAMETER;
+  k_gemm_bf16<OUT><<<dim3(cdiv(M, 32), gy), 256, 0, st>>>((int)M, N, (int)K, A, lda, B, ldb, e);
   return launch_status();
 }
 
-// Adam (Kingma & Ba 2015, Algorithm 1)
 // out = -in
 __global__ void k_negate(const float *__restrict__ in, long n, float *out) {
   GL(i, n) out[i] = -in[i];
@@ -370,14 +447,15 @@ __device__ __forceinline__ double to_canonical(const double *__restrict__ y, lon
   return z;
 }
 
+template <typename T>
 __global__ void k_gather_rows(const double *__restrict__ y, long nv, int nc,
                               const int2 *__restrict__ cinfo, const double *__restrict__ scale,
-                              const double *__restrict__ frames, float *Z) {
+                              const double *__restrict__ frames, T *Z) {
   const int nin = 4 * nc;
   GL(i, nv * nin) {
     const long v = i / nin;
     const int j = (int)(i % nin);
-    Z[i] = (float)(to_canonical(y, v, j, nv, nc, cinfo, frames) / scale[v]);
+    Z[i] = (T)(float)(to_canonical(y, v, j, nv, nc, cinfo, frames) / scale[v]);
   }
 }
 // The correction skips the tension coefficients of degree > tcut: the
@@ -440,8 +518,9 @@ LearnedPC::~LearnedPC() {
   if (perm_) (void)hipFree(perm_);
   if (vidx_) (void)hipFree(vidx_);
   if (Pbest_) (void)hipFree(Pbest_);
-  for (__bf16 *p : {Wh_, Zh_, H1h_, H2h_, dYh_, dA2h_, dA1h_})
+  for (__bf16 *p : {Wh_, Zh_, H1h_, H2h_, dYh_, dA2h_, trh_})
     if (p) (void)hipFree(p);
+  if (part_) (void)hipFree(part_);
   for (auto &kv : descs_) (void)hipFree(kv.second);
 }
 
@@ -449,7 +528,8 @@ int LearnedPC::set_activations(int mode) {
   if (mode != 0 && mode != 1) return VES3D_INVALID_PARAMETER;
   if (mode == 1 && (nin_ % 8 || width_ % 8)) return VES3D_INVALID_PARAMETER;
   if (mode == 1 && !Wh_) {
-    const long nw = (long)width_ * nin_ * 2 + (long)width_ * width_;
+    // [W1 | W2 | W3 | W2^T | W3^T]
+    const long nw = (long)width_ * nin_ * 3 + 2L * width_ * width_;
     if (hipMalloc(&Wh_, sizeof(__bf16) * nw) != hipSuccess) return VES3D_MEMORY_ERROR;
   }
   act_ = mode;
@@ -463,12 +543,12 @@ int LearnedPC::set_activations(int mode) {
 
 int LearnedPC::refresh_bf16(hipStream_t st) {
   if (!wdirty_) return VES3D_SUCCESS;
-  const long w = width_, n = nin_;
-  k_to_bf16<<<gb(w * n), 256, 0, st>>>(P_ + oW1_, w * n, Wh_);
-  V3D_CHECK(launch_status());
-  k_to_bf16<<<gb(w * w), 256, 0, st>>>(P_ + oW2_, w * w, Wh_ + w * n);
-  V3D_CHECK(launch_status());
-  k_to_bf16<<<gb(n * w), 256, 0, st>>>(P_ + oW3_, n * w, Wh_ + w * n + w * w);
+  const int w = width_, n = nin_;
+  const long wn = (long)w * n, ww = (long)w * w;
+  const ToBf16 a1{P_ + oW1_, Wh_, nullptr, w, n, 0};
+  const ToBf16 a2{P_ + oW2_, Wh_ + wn, Wh_ + 2 * wn + ww, w, w, w};
+  const ToBf16 a3{P_ + oW3_, Wh_ + wn + ww, Wh_ + 2 * wn + 2 * ww, n, w, n};
+  k_to_bf16<<<dim3(cdiv(w, 32) * std::max(cdiv(w, 32), cdiv(n, 32)), 3), 256, 0, st>>>(a1, a2, a3);
   V3D_CHECK(launch_status());
   wdirty_ = false;
   return VES3D_SUCCESS;
@@ -521,14 +601,24 @@ int LearnedPC::ensure_batch(long B) {
   for (float **p : nb)
     if (hipMalloc(p, sizeof(float) * B * n) != hipSuccess) return VES3D_MEMORY_ERROR;
   if (hipMalloc(&scale_, sizeof(double) * B) != hipSuccess) return VES3D_MEMORY_ERROR;
-  for (__bf16 *p : {Zh_, H1h_, H2h_, dYh_, dA2h_, dA1h_})
+  for (__bf16 *p : {Zh_, H1h_, H2h_, dYh_, dA2h_, trh_})
     if (p) (void)hipFree(p);
-  Zh_ = H1h_ = H2h_ = dYh_ = dA2h_ = dA1h_ = nullptr;
+  Zh_ = H1h_ = H2h_ = dYh_ = dA2h_ = trh_ = nullptr;
+  if (part_) (void)hipFree(part_);
+  part_ = nullptr;
   if (act_ == 1) {
-    for (__bf16 **p : {&H1h_, &H2h_, &dA2h_, &dA1h_})
-      if (hipMalloc(p, sizeof(__bf16) * B * w) != hipSuccess) return VES3D_MEMORY_ERROR;
+    // the hidden activations hold both signs' rows (odd_forward)
+    for (__bf16 **p : {&H1h_, &H2h_})
+      if (hipMalloc(p, sizeof(__bf16) * 2 * B * w) != hipSuccess) return VES3D_MEMORY_ERROR;
+    if (hipMalloc(&dA2h_, sizeof(__bf16) * B * w) != hipSuccess) return VES3D_MEMORY_ERROR;
     for (__bf16 **p : {&Zh_, &dYh_})
       if (hipMalloc(p, sizeof(__bf16) * B * n) != hipSuccess) return VES3D_MEMORY_ERROR;
+    // transposed operands of the weight gradients: Z, dY, H1, H2, dA1, dA2
+    const long bt = (B + 7) / 8 * 8;
+    if (hipMalloc(&trh_, sizeof(__bf16) * bt * (2 * n + 4 * w)) != hipSuccess)
+      return VES3D_MEMORY_ERROR;
+    if (hipMalloc(&part_, sizeof(double) * cdiv(B, 32) * cdiv(n, 32)) != hipSuccess)
+      return VES3D_MEMORY_ERROR;
   }
   bcap_ = B;
   return VES3D_SUCCESS;
@@ -565,20 +655,22 @@ int LearnedPC::forward(const float *Z, long B, float *Y, hipStream_t st) {
   const int w = width_, n = nin_;
   if (act_ == 1) {
     // BF16 operands (weights rounded from the FP32 master copy), FP32
-    // accumulation, FP32 pre-activations and output
+    // accumulation, pre-activations and output
     V3D_CHECK(refresh_bf16(st));
-    const __bf16 *W1h = Wh_, *W2h = Wh_ + (long)w * n, *W3h = W2h + (long)w * w;
-    k_to_bf16<<<gb(B * n), 256, 0, st>>>(Z, B * n, Zh_);
+    const ToBf16 a{Z, Zh_, nullptr, (int)B, n, 0};
+    k_to_bf16<<<cdiv(B, 32) * cdiv(n, 32), 256, 0, st>>>(a, a, a);
     V3D_CHECK(launch_status());
-    V3D_CHECK((gemm_bf16<true, true>((int)B, w, n, Zh_, n, W1h, n, A1_, w, st)));
-    k_bias_gelu_bf<<<gb(B * w), 256, 0, st>>>(A1_, P_ + ob1_, B, w, H1h_);
-    V3D_CHECK(launch_status());
-    V3D_CHECK((gemm_bf16<true, true>((int)B, w, w, H1h_, w, W2h, w, A2_, w, st)));
-    k_bias_gelu_bf<<<gb(B * w), 256, 0, st>>>(A2_, P_ + ob2_, B, w, H2h_);
-    V3D_CHECK(launch_status());
-    V3D_CHECK((gemm_bf16<true, true>((int)B, n, w, H2h_, w, W3h, w, Y, n, st)));
-    k_add_bias<<<gb(B * n), 256, 0, st>>>(Y, P_ + ob3_, B, n);
-    return launch_status();
+    GemmEpi e;
+    e.bias = P_ + ob1_;
+    e.H = H1h_;
+    V3D_CHECK(gemm_bf16<kOutGelu>(B, w, n, Zh_, n, W1h(), n, e, st));
+    e.bias = P_ + ob2_;
+    e.H = H2h_;
+    V3D_CHECK(gemm_bf16<kOutGelu>(B, w, w, H1h_, w, W2h(), w, e, st));
+    GemmEpi y;
+    y.bias = P_ + ob3_;
+    y.C = Y;
+    return gemm_bf16<kOutBias>(B, n, w, H2h_, w, W3h(), w, y, st);
   }
   V3D_CHECK(gemm((int)B, w, n, Z, n, 1, P_ + oW1_, 1, n, A1_, st));   // Z W1^T
   k_bias_gelu<<<gb(B * w), 256, 0, st>>>(A1_, P_ + ob1_, B, w, H1_);
@@ -597,39 +689,67 @@ int LearnedPC::bias_grads(long B, hipStream_t st) {
   return launch_status();
 }
 
+// BF16 operands of every product, FP32 pre-activations, gradients and bias sums
+int LearnedPC::loss_grad_bf16(const float *Z, const float *T, long B, double *loss_host,
+                              hipStream_t st) {
+  V3D_CHECK(ensure_batch(B));
+  V3D_CHECK(refresh_bf16(st));
+  const int w = width_, n = nin_;
+  const long tot = B * n, bt = (B + 7) / 8 * 8;
+  __bf16 *Zt = trh_, *dYt = Zt + bt * n, *H1t = dYt + bt * n, *H2t = H1t + bt * w,
+         *dA1t = H2t + bt * w, *dA2t = dA1t + bt * w;
+  const ToBf16 a{Z, Zh_, Zt, (int)B, n, (int)bt};
+  k_to_bf16<<<cdiv(B, 32) * cdiv(n, 32), 256, 0, st>>>(a, a, a);
+  V3D_CHECK(launch_status());
+  auto epi = [&](float *C, const float *bias, __bf16 *H, __bf16 *HT) {
+    GemmEpi e;
+    e.C = C;
+    e.bias = bias;
+    e.H = H;
+    e.HT = HT;
+    e.ldt = (int)bt;
+    return e;
+  };
+  V3D_CHECK(gemm_bf16<kOutGelu>(B, w, n, Zh_, n, W1h(), n, epi(A1_, P_ + ob1_, H1h_, H1t), st));
+  V3D_CHECK(gemm_bf16<kOutGelu>(B, w, w, H1h_, w, W2h(), w, epi(A2_, P_ + ob2_, H2h_, H2t), st));
+  GemmEpi l = epi(dY_, P_ + ob3_, dYh_, dYt);
+  l.T = T;
+  l.invn = 1.0f / (float)tot;
+  l.part = part_;
+  V3D_CHECK(gemm_bf16<kOutLoss>(B, n, w, H2h_, w, W3h(), w, l, st));
+  k_sum_parts<<<1, 256, 0, st>>>(part_, (int)(cdiv(B, 32) * cdiv(n, 32)), 0.5 / (double)tot,
+                                 lossbuf_ + 4100);
+  V3D_CHECK(launch_status());
+  // input gradients, dY W3 and dA2 W2, through the activations
+  GemmEpi g = epi(dA2_, nullptr, dA2h_, dA2t);
+  g.P = A2_;
+  V3D_CHECK(gemm_bf16<kOutBack>(B, w, n, dYh_, n, W3t(), n, g, st));
+  g = epi(dA1_, nullptr, nullptr, dA1t);
+  g.P = A1_;
+  V3D_CHECK(gemm_bf16<kOutBack>(B, w, w, dA2h_, w, W2t(), w, g, st));
+  // weight gradients dY^T H2, dA2^T H1, dA1^T Z: K is the batch, padded to bt
+  V3D_CHECK(gemm_bf16<kOutStore>(n, w, bt, dYt, bt, H2t, bt, epi(G_ + oW3_, nullptr, nullptr, nullptr), st));
+  V3D_CHECK(gemm_bf16<kOutStore>(w, w, bt, dA2t, bt, H1t, bt, epi(G_ + oW2_, nullptr, nullptr, nullptr), st));
+  V3D_CHECK(gemm_bf16<kOutStore>(w, n, bt, dA1t, bt, Zt, bt, epi(G_ + oW1_, nullptr, nullptr, nullptr), st));
+  V3D_CHECK(bias_grads(B, st));
+  if (loss_host) {
+    V3D_HIP(hipMemcpyAsync(loss_host, lossbuf_ + 4100, sizeof(double), hipMemcpyDeviceToHost, st));
+    V3D_HIP(hipStreamSynchronize(st));
+  }
+  return VES3D_SUCCESS;
+}
+
 int LearnedPC::loss_grad(const float *Z, const float *T, long B, double *loss_host,
                          hipStream_t st) {
-  V3D_CHECK(forward(Z, B, Y_, st));
   const int w = width_, n = nin_;
   const long tot = B * n;
+  if (act_ == 1) return loss_grad_bf16(Z, T, B, loss_host, st);
+  V3D_CHECK(forward(Z, B, Y_, st));
   const int nb = (int)std::min<long>(4096, std::max<long>(1, (tot + 255) / 256));
   k_diff_loss<<<nb, 256, 0, st>>>(Y_, T, tot, 1.0f / (float)tot, dY_, lossbuf_);
   V3D_CHECK(launch_status());
   k_sum_parts<<<1, 256, 0, st>>>(lossbuf_, nb, 0.5 / (double)tot, lossbuf_ + 4100);
   V3D_CHECK(launch_status());
-  if (act_ == 1) {
-    // BF16 operands of every product, FP32 gradients and bias sums
-    const __bf16 *W2h = Wh_ + (long)w * n, *W3h = W2h + (long)w * w;
-    const int Bi = (int)B;
-    k_to_bf16<<<gb(tot), 256, 0, st>>>(dY_, tot, dYh_);
-    V3D_CHECK(launch_status());
-    V3D_CHECK((gemm_bf16<false, false>(n, w, Bi, dYh_, n, H2h_, w, G_ + oW3_, w, st)));
-    V3D_CHECK((gemm_bf16<true, false>(Bi, w, n, dYh_, n, W3h, w, dA2_, w, st)));
-    k_gelu_back_bf<<<gb(B * w), 256, 0, st>>>(dA2_, A2_, B * w, dA2h_);
-    V3D_CHECK(launch_status());
-    V3D_CHECK((gemm_bf16<false, false>(w, w, Bi, dA2h_, w, H1h_, w, G_ + oW2_, w, st)));
-    V3D_CHECK((gemm_bf16<true, false>(Bi, w, w, dA2h_, w, W2h, w, dA1_, w, st)));
-    k_gelu_back_bf<<<gb(B * w), 256, 0, st>>>(dA1_, A1_, B * w, dA1h_);
-    V3D_CHECK(launch_status());
-    V3D_CHECK((gemm_bf16<false, false>(w, n, Bi, dA1h_, w, Zh_, n, G_ + oW1_, n, st)));
-    V3D_CHECK(bias_grads(B, st));
-    if (loss_host) {
-      V3D_HIP(hipMemcpyAsync(loss_host, lossbuf_ + 4100, sizeof(double), hipMemcpyDeviceToHost,
-                             st));
-      V3D_HIP(hipStreamSynchronize(st));
-    }
-    return VES3D_SUCCESS;
-  }
   // layer 3
   V3D_CHECK(gemm(n, w, (int)B, dY_, 1, n, H2_, w, 1, G_ + oW3_, st));  // dY^T H2
   V3D_CHECK(gemm((int)B, w, n, dY_, n, 1, P_ + oW3_, w, 1, dA2_, st));  // dY W3
@@ -761,16 +881,47 @@ int LearnedPC::apply_inplace(double *y, long nv, int p, int tcut, const int2 *ci
   V3D_CHECK(ensure_batch(nv));
   k_row_norms<<<(unsigned)nv, 256, 0, st>>>(y, nv, nc, cinfo, scale_);
   V3D_CHECK(launch_status());
-  k_gather_rows<<<gb(nv * nin_), 256, 0, st>>>(y, nv, nc, cinfo, scale_, frames, Zb_);
-  V3D_CHECK(launch_status());
-  V3D_CHECK(odd_forward(Zb_, nv, Y_, st));
+  if (act_ == 1) {
+    k_gather_rows<<<gb(nv * nin_), 256, 0, st>>>(y, nv, nc, cinfo, scale_, frames, Zh_);
+    V3D_CHECK(launch_status());
+    V3D_CHECK(odd_forward_bf16(nv, Y_, st));
+  } else {
+    k_gather_rows<<<gb(nv * nin_), 256, 0, st>>>(y, nv, nc, cinfo, scale_, frames, Zb_);
+    V3D_CHECK(launch_status());
+    V3D_CHECK(odd_forward(Zb_, nv, Y_, st));
+  }
   k_scatter_add<<<gb(nv * nin_), 256, 0, st>>>(Y_, nv, nc, p, tcut, cinfo, scale_, frames,
                                                 y);
   return launch_status();
 }
 
+// The odd part on the rows of Zh_.  The first layer's product changes sign
+// with its input, so it serves both signs; the hidden layers run on 2 B rows
+// (z's, then -z's), and the last product forms half the difference.
+int LearnedPC::odd_forward_bf16(long B, float *Y, hipStream_t st) {
+  V3D_CHECK(refresh_bf16(st));
+  const int w = width_, n = nin_;
+  GemmEpi e;
+  e.bias = P_ + ob1_;
+  e.H = H1h_;
+  V3D_CHECK(gemm_bf16<kOutGeluOdd>(B, w, n, Zh_, n, W1h(), n, e, st));
+  e.bias = P_ + ob2_;
+  e.H = H2h_;
+  V3D_CHECK(gemm_bf16<kOutGelu>(2 * B, w, w, H1h_, w, W2h(), w, e, st));
+  GemmEpi y;
+  y.bias = P_ + ob3_;
+  y.C = Y;
+  return gemm_bf16<kOutOdd>(B, n, w, H2h_, w, W3h(), w, y, st);
+}
+
 int LearnedPC::odd_forward(const float *Z, long B, float *Y, hipStream_t st) {
   V3D_CHECK(ensure_batch(B));
+  if (act_ == 1) {
+    const ToBf16 a{Z, Zh_, nullptr, (int)B, nin_, 0};
+    k_to_bf16<<<cdiv(B, 32) * cdiv(nin_, 32), 256, 0, st>>>(a, a, a);
+    V3D_CHECK(launch_status());
+    return odd_forward_bf16(B, Y, st);
+  }
   const long n = B * nin_;
   V3D_CHECK(forward(Z, B, Y, st));
   k_negate<<<gb(n), 256, 0, st>>>(Z, n, Zneg_);

@@ -83,6 +83,14 @@ class LearnedPC {
   int ensure_batch(long B);
   int refresh_bf16(hipStream_t st);
   int bias_grads(long B, hipStream_t st);
+  int loss_grad_bf16(const float *Z, const float *T, long B, double *loss_host, hipStream_t st);
+  int odd_forward_bf16(long B, float *Y, hipStream_t st);
+  // the BF16 weights in Wh_: [W1 | W2 | W3 | W2^T | W3^T]
+  const __bf16 *W1h() const { return Wh_; }
+  const __bf16 *W2h() const { return Wh_ + (long)width_ * nin_; }
+  const __bf16 *W3h() const { return W2h() + (long)width_ * width_; }
+  const __bf16 *W2t() const { return W3h() + (long)width_ * nin_; }
+  const __bf16 *W3t() const { return W2t() + (long)width_ * width_; }
   int gemm(int M, int N, int K, const float *A, long ars, long acs, const float *Bm, long brs,
            long bcs, float *C, hipStream_t st);
 
@@ -106,9 +114,11 @@ class LearnedPC {
   std::map<std::tuple<int, int, int, long, long, long, long>, GemmDesc *> descs_;
   int act_ = 0;
   bool wdirty_ = true;
-  // BF16 weights [W1 | W2 | W3] and activation / gradient operands
+  // BF16 weights, activation / gradient operands, and the transposed ones of
+  // the weight gradients; partial sums of the loss
   __bf16 *Wh_ = nullptr, *Zh_ = nullptr, *H1h_ = nullptr, *H2h_ = nullptr, *dYh_ = nullptr,
-         *dA2h_ = nullptr, *dA1h_ = nullptr;
+         *dA2h_ = nullptr, *trh_ = nullptr;
+  double *part_ = nullptr;
 };
 
 }  // namespace v3d
