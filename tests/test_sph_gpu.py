@@ -59,6 +59,39 @@ def test_grid2shc_and_transpose(hip, p0, p1, N, dt, tol):
     assert rel(gs.double().cpu().numpy(), T) < tol
 
 
+@pytest.mark.parametrize("p0,p1,N", [(1, 1, 1), (2, 5, 3), (8, 8, 4), (9, 17, 1027), (16, 32, 683),
+                                     (17, 3, 130), (24, 25, 1), (25, 24, 513), (32, 33, 2),
+                                     (32, 32, 1365), (33, 12, 3)])
+@pytest.mark.parametrize("dt,tol", [(torch.float64, 1e-12), (torch.float32, 1e-5)])
+def test_one_kernel_transforms(hip, p0, p1, N, dt, tol):
+    """The one-kernel transforms against the grouped GEMMs (which a forced tile
+    selects) at the edges of their rules: padded and whole tiles of columns and
+    rows, every functions-per-workgroup, partial last groups, and the orders
+    and sizes on both sides of the line to the GEMMs."""
+    from ves3d_amd import call
+    S = torch.from_numpy(RNG.standard_normal((N, p0 * (p0 + 2)))).to("cuda", dt)
+    X = torch.from_numpy(RNG.standard_normal((N, 2 * p0 * (p0 + 1)))).to("cuda", dt)
+    grid = lambda: torch.zeros((N, 2 * p1 * (p1 + 1)), dtype=dt, device="cuda")
+    out = {}
+    try:
+        for tile in (-1, 0):
+            call("ves3d_hip_set_gemm_tile", tile)
+            synth, a, t = [grid() for _ in range(4)], *(
+                torch.zeros((N, p1 * (p1 + 2)), dtype=dt, device="cuda") for _ in range(2))
+            G.shc2grid(S, N, p0, p1, *synth[:3])
+            G.shc2grid(S, N, p0, p1, synth[3])
+            G.grid2shc(X, N, p0, p1, a)
+            G.shc2grid_transpose(X, N, p0, p1, t)
+            torch.cuda.synchronize()
+            out[tile] = [x.double() for x in synth + [a, t]]
+    finally:
+        call("ves3d_hip_set_gemm_tile", -1)
+    scale = max(float(x.abs().max()) for x in out[0][:4])
+    for k, (x, y) in enumerate(zip(out[-1], out[0])):
+        err = float((x - y).abs().max()) / (scale if k < 4 else float(y.abs().max()))
+        assert err < tol, (k, err)
+
+
 @pytest.mark.parametrize("p,N", [(6, 4), (16, 9)])
 def test_shc2pole(hip, p, N):
     S = RNG.standard_normal((N, p * (p + 2)))

@@ -13,6 +13,7 @@
 #include <vector>
 
 #include "gemm.hpp"
+#include "mfma.hpp"
 
 namespace v3d {
 
@@ -101,31 +102,6 @@ __global__ __launch_bounds__(GB_T) void k_gemm_grouped(
     }
   }
 }
-
-// MFMA operand layout.  For both v_mfma_f64_16x16x4f64 and
-// v_mfma_f32_16x16x4f32 lane l supplies A(l%16, l/16) and B(l/16, l%16) of a
-// 16x4 / 4x16 step and holds 4 results of column l%16; their rows differ:
-// l/16 + 4r (f64) and 4(l/16) + r (f32) for result register r (the
-// accumulator layouts composable_kernel's xdlops_gemm.hpp records as
-// group_size 1 / 4).
-template <typename T>
-struct Mfma;
-template <>
-struct Mfma<double> {
-  typedef double v4 __attribute__((ext_vector_type(4)));
-  static __device__ __forceinline__ v4 step(double a, double b, v4 c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ int row(int lk, int r) { return lk + 4 * r; }
-};
-template <>
-struct Mfma<float> {
-  typedef float v4 __attribute__((ext_vector_type(4)));
-  static __device__ __forceinline__ v4 step(float a, float b, v4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ int row(int lk, int r) { return 4 * lk + r; }
-};
 
 // MFMA output tile of BM = 64 NTM rows by BN = 16 NTN columns: wave w owns
 // rows [16 NTM w, 16 NTM (w + 1)) and all BN columns, as NTM x NTN MFMA
@@ -399,6 +375,10 @@ bool use_mfma() { return g_gemm_kind.load(std::memory_order_relaxed) == 1; }
 
 // Forced MFMA tile (-1: the caller's choice), set by ves3d_hip_set_gemm_tile.
 std::atomic<int> g_gemm_tile{-1};
+
+bool gemm_is_default() {
+  return use_mfma() && g_gemm_tile.load(std::memory_order_relaxed) < 0;
+}
 
 template <typename T, int NTM, int NTN>
 int launch_mfma(bool av, const GemmDesc *d_descs, int ndesc, int batch, int max_m, int max_n,

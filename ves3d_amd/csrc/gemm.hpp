@@ -38,6 +38,9 @@ int gemm_grouped(const GemmDesc *d_descs, int ndesc, int batch, int max_m,
 // 64x64 tile pads most of its work.
 int gemm_pick_tile(const GemmDesc *h, int n);
 
+// True unless the VALU kernel or a tile was selected (ves3d_hip_set_gemm_*).
+bool gemm_is_default();
+
 // Uploads a host descriptor list to a new device array.
 GemmDesc *upload_descs(const GemmDesc *h, int n);
 

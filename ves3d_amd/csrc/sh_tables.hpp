@@ -36,6 +36,7 @@ struct ShMatsHost {
   long Mf, Mdf, Mfinv;          // MatFourier(p0,p1), MatFourierGrad(p0,p1), MatFourierInv(p0,p1): [2p0][2p1]
   long MfT;                     // MatFourier(p1,p0): [2p1][2p0] (read transposed by SHC2GridTranspose)
   long Md2f;                    // second longitude derivative of MatFourier: [2p0][2p1]
+  // per order m the four blocks Ml, Mdl, Mdln, Md2l follow each other, and so do the orders'
   std::vector<long> Ml, Mdl;    // MatLegendre(p0,p1)[m], MatLegendreGrad: [(p0+1-m)][(p1+1)], m=0..p0
   std::vector<long> Mdln;       // -MatLegendreGrad (SHTrans's first latitude derivative), same shape
   std::vector<long> Md2l;       // second latitude derivative (ladder of d2legTrans), same shape

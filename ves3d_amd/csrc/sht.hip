@@ -8,6 +8,8 @@
 // in the opposite order with the inverse / transposed matrices.  The block
 // gather of the coefficient layout and the transposes between the stages are
 // operand strides of the GEMM descriptors; nothing is re-laid out in memory.
+// Where a function's intermediate fits in LDS the two stages run as one kernel
+// (sht_fused.hip).
 #include <map>
 #include <mutex>
 #include <tuple>
@@ -123,6 +125,10 @@ int run(int kind, int p0, int p1, long N, const ShMatsDev *m, const T *A, T *C,
 
 bool valid_order(int p) { return p >= 1 && p <= 255; }
 
+// The place of a latitude derivative among an order's Legendre blocks (neg:
+// SHTrans's sign of the first derivative).
+int leg_kind(int dleg, int neg) { return dleg == 0 ? 0 : (dleg == 1 ? (neg ? 2 : 1) : 3); }
+
 // plans of sht_synth_multi: the Legendre and the Fourier stage of every
 // variant, keyed by (device, p0, p1, N, variants, x_stride)
 struct MultiPlan {
@@ -201,6 +207,15 @@ int sht_synth_multi(const T *S, long N, int p0, int p1, int nvar, const int *dle
   if (N == 0) return VES3D_SUCCESS;
   const ShMatsDev *m = sh_mats(p0, p1);
   if (!m) return VES3D_MEMORY_ERROR;
+  int kind[kMaxSynth], status;
+  T *out[kMaxSynth];
+  for (int v = 0; v < nvar; ++v) {
+    kind[v] = leg_kind(dleg[v], neg[v]);
+    out[v] = X + v * x_stride;
+  }
+  if (synth_fused<T>(S, N, p0, p1, nvar, *m->h, mats_ptr<T>(m), kind, dfour, out, T(1), st,
+                     &status))
+    return status;
   const MultiPlan *mp = get_multi_plan(p0, p1, N, nvar, dleg, dfour, neg, x_stride, *m->h);
   if (!mp) return VES3D_MEMORY_ERROR;
   V3D_CHECK(gemm_grouped<T>(mp->leg.d, mp->leg.n, 1, mp->leg.max_m, mp->leg.max_n, S,
@@ -216,6 +231,18 @@ int sht_shc2grid(const T *S, long N, int p0, int p1, T *X, T *Xt, T *Xp, T *work
   if (N == 0) return VES3D_SUCCESS;
   const ShMatsDev *m = sh_mats(p0, p1);
   if (!m) return VES3D_MEMORY_ERROR;
+  int dleg[kMaxSynth] = {0}, dfour[kMaxSynth] = {0}, n = 1, status;
+  T *out[kMaxSynth] = {X};
+  if (Xt) {
+    dfour[n] = 1;
+    out[n++] = Xt;
+  }
+  if (Xp) {
+    dleg[n] = 1;
+    out[n++] = Xp;
+  }
+  if (synth_fused<T>(S, N, p0, p1, n, *m->h, mats_ptr<T>(m), dleg, dfour, out, T(1), st, &status))
+    return status;
   V3D_CHECK(run<T>(kS2GLeg, p0, p1, N, m, S, work, st));
   V3D_CHECK(run<T>(kS2GFour, p0, p1, N, m, work, X, st));
   if (Xt) V3D_CHECK(run<T>(kS2GFour + 16, p0, p1, N, m, work, Xt, st));
@@ -235,6 +262,11 @@ int sht_synth(const T *S, long N, int p0, int p1, int dleg, int dfour, T *X, T *
   if (N == 0) return VES3D_SUCCESS;
   const ShMatsDev *m = sh_mats(p0, p1);
   if (!m) return VES3D_MEMORY_ERROR;
+  const int kind = leg_kind(dleg, 0);
+  int status;
+  if (synth_fused<T>(S, N, p0, p1, 1, *m->h, mats_ptr<T>(m), &kind, &dfour, &X, alpha, st,
+                     &status))
+    return status;
   V3D_CHECK(run<T>(kS2GLeg + 16 * dleg, p0, p1, N, m, S, work, st, alpha));
   return run<T>(kS2GFour + 16 * dfour, p0, p1, N, m, work, X, st);
 }
@@ -245,6 +277,9 @@ int sht_grid2shc(const T *X, long N, int p0, int p1, T *S, T *work, hipStream_t 
   if (N == 0) return VES3D_SUCCESS;
   const ShMatsDev *m = sh_mats(p0, p1);
   if (!m) return VES3D_MEMORY_ERROR;
+  int status;
+  if (analysis_fused<T>(X, N, p0, p1, false, *m->h, mats_ptr<T>(m), S, st, &status))
+    return status;
   V3D_CHECK(run<T>(kG2SFour, p0, p1, N, m, X, work, st));
   return run<T>(kG2SLeg, p0, p1, N, m, work, S, st);
 }
@@ -256,6 +291,9 @@ int sht_shc2grid_transpose(const T *X, long N, int p0, int p1, T *S, T *work,
   if (N == 0) return VES3D_SUCCESS;
   const ShMatsDev *m = sh_mats(p0, p1);
   if (!m) return VES3D_MEMORY_ERROR;
+  int status;
+  if (analysis_fused<T>(X, N, p0, p1, true, *m->h, mats_ptr<T>(m), S, st, &status))
+    return status;
   V3D_CHECK(run<T>(kTFour, p0, p1, N, m, X, work, st));
   return run<T>(kTLeg, p0, p1, N, m, work, S, st);
 }

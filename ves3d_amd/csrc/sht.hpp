@@ -49,6 +49,22 @@ int sht_synth_multi(const T *S, long N, int p0, int p1, int nvar, const int *dle
                     const int *dfour, const int *neg, T *X, long x_stride, T *work,
                     hipStream_t st);
 
+// One-kernel forms of the transforms (sht_fused.hip).  They return false
+// where they do not apply (the caller then runs the grouped GEMMs), else
+// true with the launch's status in *status.
+constexpr int kMaxSynth = 4;
+// nvar syntheses of the same coefficients: variant v with the latitude
+// derivative dleg[v] (0, 1, 2: the negated first, 3: the second) and the
+// longitude derivative dfour[v] into X[v]; mats the device copy of h's data.
+template <typename T>
+bool synth_fused(const T *S, long N, int p0, int p1, int nvar, const ShMatsHost &h, const T *mats,
+                 const int *dleg, const int *dfour, T *const *X, T alpha, hipStream_t st,
+                 int *status);
+// Grid2SHC or (transpose) SHC2GridTranspose: X [N][(p0+1) 2p0] -> S [N][p1(p1+2)].
+template <typename T>
+bool analysis_fused(const T *X, long N, int p0, int p1, bool transpose, const ShMatsHost &h,
+                    const T *mats, T *S, hipStream_t st, int *status);
+
 // The matrices of SHC2GridTranspose (p1 -> p0) on the device, for a caller
 // that runs its stages itself: sht_mft gives MatFourier(p1, p0) ([2p1][2p0]:
 // frequency row jj, longitude column), sht_mlt MatLegendre(p1, p0)[m] for
