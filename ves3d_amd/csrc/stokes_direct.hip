@@ -514,7 +514,8 @@ static Split choose_split(long n_trg, long n_groups, long spg, long max_slices =
   const long finest = (spg + FF_PART - 1) / FF_PART;
   const long nsub = n_groups >= 8 * want ? 1 : std::min((8 * want + n_groups - 1) / n_groups, finest);
   const long units = n_groups * nsub;
-  const long per = std::max(1L, (units + want - 1) / want);
+  long per = std::max(1L, units / want);
+  if ((units + per - 1) / per > max_slices * share) per = (units + want - 1) / want;
   const long slices = (units + per - 1) / per;
   Split s;
   s.nsplit = (int)((slices + share - 1) / share);
