@@ -312,10 +312,10 @@ int ves3d_hip_rotate_transpose_f64(const double *S_in, size_t N, int p, int dof,
 
 /* Kernel choice of the singular-operator build (no counterpart in the
  * reference, global per process): 1 (the default) evaluates the FP64 build's
- * pole kernel and its transposed synthesis (Fourier stage on FP64 MFMA,
- * Legendre stage) in one kernel, where p1 = 2 p0 and p0 <= 16; 0 runs them
- * as the pole kernel and two grouped GEMMs with the kernel values in HBM
- * between them (the FP32 build always does). */
+ * pole kernel, its transposed synthesis (Fourier stage on FP64 MFMA, Legendre
+ * stage) and RotateTranspose in one kernel, where p1 is even, 12 <= p1 <= 32
+ * and p1 >= 2 p0; 0 runs them as separate kernels with the kernel values in
+ * HBM between them (the FP32 build always does). */
 int ves3d_hip_set_pole_kernel(int fused);
 /* The fused stage's launch on the current device for orders (p0, p1) of the
  * FP64 build (no counterpart in the reference): latitude rows per pass,

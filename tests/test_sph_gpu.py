@@ -230,6 +230,30 @@ def test_self_apply(hip, dt, tol):
     assert rel(V.cpu().numpy(), ref1) < tol
 
 
+@pytest.mark.parametrize("p0,p1,nv", [(6, 12, 1), (7, 14, 2), (9, 18, 5), (10, 20, 2), (12, 24, 9),
+                                      (13, 26, 2), (15, 30, 4), (5, 12, 2), (3, 32, 2), (16, 32, 3)])
+def test_pole_kernel_orders(hip, p0, p1, nv):
+    """The fused pole kernel's instances against the separate kernels: orders
+    whose longitudes and columns fill the matrix tiles in part, odd orders,
+    upsampled orders above 2 p0, and fewer and more rotations (nv p0 (p0 + 1))
+    than persistent workgroups.  Both sum the same products in FP64: 1e-12 as
+    test_singular_build_fused_pole_stage."""
+    from ves3d_amd import call
+    X = cu(_singular_case(nv, p0, seed=p0 + p1))
+    n = 3 * p0 * (p0 + 2)
+    out = {}
+    try:
+        for fused in (1, 0):
+            call("ves3d_hip_set_pole_kernel", fused)
+            sl, dl = (torch.zeros((nv, n, n), dtype=torch.float64, device="cuda") for _ in range(2))
+            G.singular_build(X, nv, p0, p1, sl, dl)
+            torch.cuda.synchronize()
+            out[fused] = sl.cpu().numpy(), dl.cpu().numpy()
+    finally:
+        call("ves3d_hip_set_pole_kernel", 1)
+    assert rel(out[1][0], out[0][0]) < 1e-12 and rel(out[1][1], out[0][1]) < 1e-12
+
+
 @pytest.mark.parametrize("p0", [16, 8])
 def test_singular_build_fused_pole_stage(hip, p0):
     """The FP64 build's fused pole kernel + transposed synthesis (the default

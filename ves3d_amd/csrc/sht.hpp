@@ -65,13 +65,9 @@ template <typename T>
 bool analysis_fused(const T *X, long N, int p0, int p1, bool transpose, const ShMatsHost &h,
                     const T *mats, T *S, hipStream_t st, int *status);
 
-// The matrices of SHC2GridTranspose (p1 -> p0) on the device, for a caller
-// that runs its stages itself: sht_mft gives MatFourier(p1, p0) ([2p1][2p0]:
-// frequency row jj, longitude column), sht_mlt MatLegendre(p1, p0)[m] for
-// m = 0..p1, consecutive blocks [(p1+1-m)][p0+1].
+// MatFourier(p1, p0) of SHC2GridTranspose (p1 -> p0) on the device ([2p1][2p0]:
+// frequency row jj, longitude column), for a caller that runs its stages itself.
 template <typename T>
 const T *sht_mft(int p0, int p1);
-template <typename T>
-const T *sht_mlt(int p0, int p1);
 
 }  // namespace v3d

@@ -13,8 +13,8 @@
 //   Grid2SHC -> RotateAll -> SHC2Grid(p0 -> p1, +derivatives) & SHC2Pole
 //   -> pole kernel (FP64) -> SHC2GridTranspose(p1 -> p0) -> RotateTranspose
 //   -> rearrange -> Grid2SHC = [Nves][3 Ncoef][3 Ncoef]
-// The FP64 build of p1 = 2 p0 <= 32 fuses the pole kernel with
-// SHC2GridTranspose and RotateTranspose's gather (k_pole_transpose), and the
+// The FP64 build of 12 <= p1 <= 32 fuses the pole kernel with
+// SHC2GridTranspose and RotateTranspose (k_pole_transpose), and the
 // rearrangement with the last Grid2SHC (k_rearrange_g2s).  The FP32 form runs
 // every GEMM stage in FP32 and keeps the pole kernel (singular weights, 1/r
 // near the rotated pole) in FP64.  Both write the operator's (a, b) and
@@ -44,9 +44,9 @@ struct BuildOrder {
   bool recorded = false;
 };
 std::map<int, BuildOrder> g_build_order;
-// 1: the singular build's pole kernel runs fused with the transposed
-// synthesis (k_pole_transpose) where its shapes allow; 0: as separate
-// kernel and grouped GEMMs (ves3d_hip_set_pole_kernel)
+// 1: the singular build's pole kernel runs fused with the transposed synthesis
+// and rotation (k_pole_transpose) where its shapes allow; 0: as separate
+// kernels (ves3d_hip_set_pole_kernel)
 std::atomic<int> g_pole_fused{1};
 struct RotPlan {
   GemmDesc *d;
@@ -249,11 +249,9 @@ int rotate_all(const T *S, long Nv, int p, int dof, T *out, T *work, hipStream_t
   return launch_status();
 }
 
-// RotateTranspose: in/out [Nv][p+1][p][dof][Ncoef]; work: 2 * that size
-// (that size when gathered: the input rows are already in degree-major order).
+// RotateTranspose: in/out [Nv][p+1][p][dof][Ncoef]; work: 2 * that size.
 template <typename T>
-int rotate_transpose(const T *in, long Nv, int p, int dof, T *out, T *work, hipStream_t st,
-                     bool gathered) {
+int rotate_transpose(const T *in, long Nv, int p, int dof, T *out, T *work, hipStream_t st) {
   const RotMatsDev *r = rot_mats(p);
   if (!r) return VES3D_MEMORY_ERROR;
   const auto *pl = rot_plan(p, dof, true, *r->h);
@@ -261,15 +259,10 @@ int rotate_transpose(const T *in, long Nv, int p, int dof, T *out, T *work, hipS
   const int nc = sh_ncoef(p);
   const long rows = Nv * (p + 1) * (long)p * dof;
   if (rows / 4 >= 0x7fffffffL) return VES3D_INVALID_PARAMETER;
-  const T *Ap = in;
-  T *Bp = work;
-  if (!gathered) {
-    k_gather_coef<T><<<row_blocks(rows), 256, 0, st>>>(in, rows, nc, r->perm, work);
-    V3D_CHECK(launch_status());
-    Ap = work;
-    Bp = work + rows * nc;
-  }
-  V3D_CHECK(gemm_grouped<T>(pl->d, pl->n, (int)Nv, p * dof, 2 * p, Ap,
+  T *Bp = work + rows * nc;
+  k_gather_coef<T><<<row_blocks(rows), 256, 0, st>>>(in, rows, nc, r->perm, work);
+  V3D_CHECK(launch_status());
+  V3D_CHECK(gemm_grouped<T>(pl->d, pl->n, (int)Nv, p * dof, 2 * p, work,
                             rot_ptr<T>(r), Bp, T(1), T(0), st, pl->tile));
   const size_t stage = 4 * nc * sizeof(T);
   if (stage <= kScatterStageBytes)
@@ -334,210 +327,380 @@ __global__ void k_pole_kernel(const T *__restrict__ X, const T *__restrict__ Xt,
   }
 }
 
+// 1/sqrt(x), x > 0: the hardware estimate and one third-order step (as
+// rsqrt_pair of the direct sums).
+__device__ __forceinline__ double rsqrt_refined(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(y * -x, y, 1.0);
+  return fma(y * e, fma(e, 0.375, 0.5), y);
+}
+
 // The pole kernel fused with SHC2GridTranspose(p1 -> p0) of its values:
-// K1[r][t*6+c][dpos[k]] = sum over the grid (lat, lon) of the kernel value of
+// K1[r][t*6+c][k] = sum over the grid (lat, lon) of the kernel value of
 // rotation r, pole t, tensor component c at (lat, lon), times MatFourier(p0,
 // p1)[jj][lon] (the Fourier stage) and MatLegendre(p0, p1)[m][n][lat] (the
 // Legendre stage), k = blockoff(p0, jj) + n, m = (jj + 1) / 2 -- the products
 // the two grouped GEMMs of sht_shc2grid_transpose form, without the kernel
 // values (12 functions on the upsampled grid per rotation) or the Fourier
-// stage's output passing through HBM.  dpos (RotateTranspose's degree-major
-// position of each coefficient) lays the rows out as RotateTranspose's
-// per-degree products read them, so its gather pass is not needed.
+// stage's output passing through HBM -- and K2 = RotateTranspose of the rows
+// (src/SphericalHarmonics.cc:451-541), which is what leaves.
+// Both tables have a mirror symmetry: MatFourier of order m at lon + pi is
+// (-1)^m of that at lon, and MatLegendre of degree n and order m at the
+// latitude P1 - lat is (-1)^(n-m) of that at lat.  So the sums and differences
+// of the values at the four mirror points (lat or P1 - lat, lon or lon + pi)
+// serve one parity of m and of n - m each, with a quarter of the products.
 // Persistent workgroups walk the rotations r = blockIdx.x + i gridDim.x and,
-// within a rotation, the latitude rows in passes of R rows:
-//   1. thread (row, lon, t) evaluates pole t's 6 kernel values at (lat, lon)
-//      into Kv[row][lon][t * 6 + q] (kPtKs doubles per point, an odd stride);
-//   2. wave (row, tile) forms the 16 x 16 tile T[row][c][16 tile + j] =
-//      sum_lon Kv[row][lon][c] Mf[lon][16 tile + j] on v_mfma_f64_16x16x4f64
-//      (lane l: A(l % 16, l / 16), B(l / 16, l % 16), results at rows
-//      l / 16 + 4 i, column l % 16; rows c >= 12 read as zero), its B operand
-//      (the wave's 16 columns of MatFourier) in registers for the whole kernel;
-//   3. thread (c, jj) adds T[row][c][jj] times the rows' Legendre values into
-//      its p0 + 1 - m accumulators (FP64 registers).
-// Two barriers per pass; each kernel-value thread loads the geometry of its
-// point of the next pass while the current pass runs.  At a rotation's end
-// the accumulators go through LDS (over Kv and T) in the output layout and
-// leave as whole rows, as many rows per round as that space holds.  The Legendre blocks and the weights sit in LDS for the workgroup's
-// lifetime.
+// within a rotation, the latitude pairs (lat, P1 - lat):
+//   1. four lanes evaluate pole t's 6 kernel values at the four mirror points
+//      of (lat, lon < P1), form the four combinations by lane swaps and store
+//      them in Kv[n - m parity][m parity][lon][t * 6 + q] (kPtKs doubles per
+//      point, an odd stride, the four parts kPtPad further apart);
+//   2. wave (n - m parity, m parity) forms T[n - m parity][c][jj] = sum_lon
+//      Kv[..][lon][c] Mf[lon][jj] over its P0 columns jj on
+//      v_mfma_f64_16x16x4f64 (lane l: A(l % 16, l / 16), B(l / 16, l % 16),
+//      results at rows l / 16 + 4 i, column l % 16; rows c >= 12 are not used),
+//      its columns of MatFourier in registers for the whole kernel;
+//   3. thread (6 components, 3 degrees of one parity of a frequency jj) adds
+//      T[parity][c][jj] times the pair's Legendre values into its 6 x 3
+//      accumulators (FP64 registers).
+// One barrier per pass: Kv and T have two buffers, and stage 3 runs a pass
+// late, beside stage 2's matrix products.  Each thread loads the geometry and
+// the Legendre values (which lie by latitude, degree and triple: consecutive
+// words for the lanes of a wave) of its next pass while the current one runs.
+// At a rotation's end the accumulators go to LDS (over Kv and T) as 12
+// degree-major rows (dpos: the place of each coefficient), the waves form the
+// per-degree products with the rotation's blocks on v_mfma_f64_16x16x4f64 (12
+// of 16 rows used, the others are whatever follows; the blocks lie in `frag` in operand order, 512 contiguous
+// bytes per load), and a thread per coefficient applies the longitude phase to
+// the 12 rows and stores them.
+// Bound: the geometry's reads (72 bytes per point, 2.7 TB/s at p0 = 16) beside
+// FP64 issue, matrix and vector, where three workgroups of one wave per SIMD
+// each run at a time: 1.9 ms per 104 vesicles and layer at p0 = 16, 1.3 ms
+// without the reads; leaving out any of the other stages changes little.
+// Workgroups of 384 threads on three latitudes, without the mirror sums, took
+// 3.7 ms: at 168 VGPRs two of them per CU would have needed 3 waves on every
+// SIMD, the dispatcher places 2, 2, 1, 1 of each, so one ran at a time.
+// With rotation products and phases as passes of their own 1.55 GB per 104
+// vesicles were written and read again, 0.8 ms.
 constexpr int kPtKs = 13;
-
-// LDS doubles of k_pole_transpose: Kv, T, the weights, the Legendre blocks
-// and LMAX - 1 zero rows after them (the branch-free degree loop's reads
-// past a block's end).
-inline long pole_lds_doubles(int R, int p0, int p1, int lmax) {
-  const long L = 2 * p1, Nlat = p1 + 1, FP = 16 * ((2L * p0 + 15) / 16);
-  return R * L * kPtKs + R * 12 * FP + Nlat + (long)(p0 + 1) * (p0 + 2) / 2 * Nlat +
-         (lmax - 1) * Nlat;
+constexpr int kPtPad = 4;
+constexpr int kPtThreads = 256;
+// Doubles of one mirror combination's values.
+__host__ __device__ constexpr int pole_kv_part(int p1) { return p1 * kPtKs + kPtPad; }
+// Degree l's rotation block in operand order: 4 loads of 64 doubles (one tile
+// of 16 columns, 16 entries) for the nsmall degrees of at most 16 entries, 16
+// loads (two tiles of 16 columns, 32 entries) for the others.
+__host__ __device__ inline int rot_frag_off(int l, int nsmall) {
+  return l < nsmall ? 256 * l : 256 * nsmall + 1024 * (l - nsmall);
 }
 
-template <int LMAX, int P1>
-__global__ __launch_bounds__(384) void k_pole_transpose(
+// Degrees of a block of len degrees with parity par of n - m, and its triples.
+__host__ __device__ inline int pole_degrees(int len, int par) { return (len + 1 - par) / 2; }
+__host__ __device__ inline int pole_block_triples(int len) {
+  return (pole_degrees(len, 0) + 2) / 3 + (pole_degrees(len, 1) + 2) / 3;
+}
+// Degree triples of the orders before m (blocks of p0 + 1 - m degrees).
+__host__ __device__ inline int pole_triples(int p0, int m) {
+  int n = 0;
+  for (int i = 0; i < m; ++i) n += pole_block_triples(p0 + 1 - i);
+  return n;
+}
+// Threads of the Legendre role: two component halves of every frequency's
+// triples (two frequencies for the orders 1 .. p0 - 1).
+inline int pole_legendre_threads(int p0) {
+  return 2 * (2 * pole_triples(p0, p0 + 1) - pole_triples(p0, 1) - 1);
+}
+
+// LDS doubles of k_pole_transpose: Kv and T, which the rotation's rows share.
+__host__ __device__ inline long pole_lds_doubles(int p0, int p1) {
+  const int kt = 2 * (4 * pole_kv_part(p1) + 2 * 12 * p1), st = 12 * (p0 * (p0 + 2) + 1);
+  return kt > st ? kt : st;
+}
+
+// a and b become a + b and a - b after the odd rows of 16 lanes (kRows == 16)
+// or the upper half wave (32) of a have changed places with the even rows or
+// the lower half of b: the even lanes hold the sum and the difference of a's
+// mirror values, the odd ones of b's.
+template <int kRows>
+__device__ __forceinline__ void mirror_sums(double &a, double &b) {
+  const long long x = __double_as_longlong(a), y = __double_as_longlong(b);
+  const auto swap = [](unsigned u, unsigned v) {
+    if constexpr (kRows == 16)
+      return __builtin_amdgcn_permlane16_swap(u, v, false, false);
+    else
+      return __builtin_amdgcn_permlane32_swap(u, v, false, false);
+  };
+  const auto lo = swap((unsigned)x, (unsigned)y);
+  const auto hi = swap((unsigned)(x >> 32), (unsigned)(y >> 32));
+  const double u = __longlong_as_double(((long long)hi[0] << 32) | lo[0]);
+  const double v = __longlong_as_double(((long long)hi[1] << 32) | lo[1]);
+  a = u + v;
+  b = u - v;
+}
+
+template <int P1>
+__global__ __launch_bounds__(kPtThreads, 3) void k_pole_transpose(
     const double *__restrict__ X, const double *__restrict__ Xt, const double *__restrict__ Xp,
-    const double *__restrict__ trg, const double *__restrict__ qw, long nrot, int p0, int R,
+    const double *__restrict__ trg, const double *__restrict__ qw, long nrot, int p0,
     const double *__restrict__ mft, const double *__restrict__ mlt, int layer,
-    const int *__restrict__ dpos, double *__restrict__ K1) {
+    const int *__restrict__ dpos, const double *__restrict__ frag, long frag_t,
+    int nsmall, const int4 *__restrict__ sources,
+    const double *__restrict__ phase, double *__restrict__ K2) {
   typedef double v4d __attribute__((ext_vector_type(4)));
-  // FOLD (p1 = 32): longitudes lon and lon + L/2 differ by pi, where the
-  // Fourier functions of order m change sign by (-1)^m, so a wave forms the
-  // 16 columns of one parity of m from Kv[lon] +- Kv[lon + L/2], lon < L/2:
-  // half the MFMA steps.  Wave tiles: the two parities (FOLD), else 16
-  // consecutive columns.
-  constexpr bool FOLD = P1 == 32;
-  constexpr int L = 2 * P1, Nlat = P1 + 1, M1 = L * Nlat, KS = FOLD ? L / 8 : L / 4;
+  static_assert(P1 % 2 == 0 && 8 * P1 <= kPtThreads);
+  constexpr int L = 2 * P1, Nlat = P1 + 1, NP = P1 / 2 + 1, M1 = L * Nlat, KS = (P1 + 3) / 4;
+  constexpr int kPart = pole_kv_part(P1);
   extern __shared__ double lds[];
-  const int F = 2 * p0, FP = 16 * ((F + 15) / 16), NT = FOLD ? 2 : FP / 16,
-            Nc = p0 * (p0 + 2);
-  const int nmlt = (p0 + 1) * (p0 + 2) / 2 * Nlat;
-  double *Kv = lds;                 // [R][L][kPtKs]
-  double *Ts = Kv + R * L * kPtKs;  // [R][12][FP]
-  double *Qw = Ts + R * 12 * FP;    // [Nlat]
-  double *Ml = Qw + Nlat;           // blocks m = 0..p0: [(p0+1-m)][Nlat], then zeros
-  double *St = lds;                 // [cs][Nc], over Kv and Ts at a rotation's end
-  const int cs = min(12, (R * L * kPtKs + R * 12 * FP) / Nc);
+  const int F = 2 * p0, Nc = p0 * (p0 + 2);
+  const int ntri = pole_triples(p0, p0 + 1);
+  double *Kv = lds;                                // [buffer][2][2][P1][kPtKs]
+  double *Ts = Kv + 8 * kPart;                     // [buffer][2][12][P1]
+  double *St = lds;                                // [12][Nc + 1], over Kv and Ts
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  for (int i = tid; i < nmlt + (LMAX - 1) * Nlat; i += blockDim.x)
-    Ml[i] = i < nmlt ? mlt[i] : 0.0;
-  for (int i = tid; i < Nlat; i += blockDim.x) Qw[i] = qw[i];
-  // kernel-value role: point (krow, lon) of the pass, pole t
-  const bool kvt = tid < R * 2 * L;
-  const int krow = kvt ? tid / (2 * L) : 0, lon = kvt ? (tid >> 1) % L : 0, t = tid & 1;
-  // Fourier role (wave-uniform): row frow, output columns 16 tile .. 16 tile + 15
-  const bool fw = wv < R * NT;
-  const int frow = fw ? wv / NT : 0, tile = fw ? wv % NT : 0;
+  // kernel-value role: pole t (the wave's) at longitude j + half P1 of the
+  // pair's row; 16 lanes read 16 consecutive longitudes.  (With the four mirror
+  // points in a lane quad every four lanes of a load touch four lines: 2.7 ms
+  // instead of 1.9.)
+  constexpr int kBlocks = (P1 + 15) / 16;  // longitude blocks of half a circle
+  const int uwv = __builtin_amdgcn_readfirstlane(wv);
+  const int row = (tid >> 4) & 1, half = (tid >> 5) & 1;
+  const int t = (uwv / kBlocks) & 1, j = 16 * (uwv % kBlocks) + (tid & 15);
+  const bool kvt = uwv < 2 * kBlocks && j < P1;
+  // Fourier role: the columns of order parity tile from the row combination frow
+  const int frow = wv >> 1, tile = wv & 1;
   const int li = lane & 15, lk = lane >> 4;
   // the wave's output column for lane li (-1: a padding column)
-  int fcol = 16 * tile + li;
-  if constexpr (FOLD) {
-    fcol = -1;
-    for (int cc = 0, seen = 0; cc < F; ++cc)
-      if ((((cc + 1) / 2) & 1) == tile) {
-        if (seen == li) fcol = cc;
-        ++seen;
-      }
-  }
-  const bool fcv = fw && fcol >= 0 && fcol < F;
+  int fcol = -1;
+  for (int cc = 0, seen = 0; cc < F; ++cc)
+    if ((((cc + 1) / 2) & 1) == tile) {
+      if (seen == li) fcol = cc;
+      ++seen;
+    }
   double mf[KS];
 #pragma unroll
-  for (int s = 0; s < KS; ++s) mf[s] = fcv ? mft[(long)fcol * L + 4 * s + lk] : 0.0;
-  // Legendre role: component c, frequency row jj of the order-p0 layout,
-  // whose block starts at off (after block 0 of length p0 + 1, the blocks
-  // of order m' = 1 .. p0 come in pairs of length p0 + 1 - m')
-  const bool lt = tid < 12 * F;
-  const int c = lt ? tid / F : 0, jj = lt ? tid % F : 0;
-  const int m = (jj + 1) / 2, len = p0 + 1 - m;
-  const int mloff = Nlat * (m * (p0 + 1) - m * (m - 1) / 2);
+  for (int s = 0; s < KS; ++s)
+    mf[s] = fcol >= 0 && 4 * s + lk < P1 ? mft[(long)fcol * L + 4 * s + lk] : 0.0;
+  // Legendre role: components c .. c + 5 and the degrees m + par + 2 (3 q + n)
+  // of frequency row jj of the order-p0 layout, whose block starts at off
+  // (after block 0 of length p0 + 1, the blocks of order m' = 1 .. p0 come in
+  // pairs of length p0 + 1 - m').  Lanes take the triples of all cosine rows,
+  // then those of the sine rows (m = 1 .. p0 - 1).
+  const int ntri1 = pole_triples(p0, 1);
+  const int nrow = 2 * ntri - ntri1 - 1;
+  const bool lt = tid < 2 * nrow;
+  const int c = lt ? tid / nrow * 6 : 0;
+  const int tr = lt ? tid % nrow : 0;
+  const bool sine = tr >= ntri;
+  const int tm = sine ? tr - ntri + ntri1 : tr;  // triple within the table
+  int m = 0, q = tm;
+  while (q >= pole_block_triples(p0 + 1 - m)) q -= pole_block_triples(p0 + 1 - m++);
+  const int len = p0 + 1 - m, even = (pole_degrees(len, 0) + 2) / 3;
+  const int par = q >= even ? 1 : 0;
+  const int d0 = par + 6 * (q - par * even);  // first degree less m
+  const int jj = m == 0 ? 0 : 2 * m - (sine ? 0 : 1);
   const int off = jj == 0 ? 0 : (p0 + 1) + 2 * ((m - 1) * (p0 + 1) - (m - 1) * m / 2) +
-                                    ((jj % 2 == 0) ? (p0 + 1 - m) : 0);
-  const int ng = (Nlat + R - 1) / R;
+                                    (sine ? p0 + 1 - m : 0);
+  int dp[3];  // the places of the thread's coefficients
+#pragma unroll
+  for (int n = 0; n < 3; ++n) dp[n] = lt && d0 + 2 * n < len ? dpos[off + d0 + 2 * n] : -1;
   const double eps = 2.220446049250313e-16;
-  const double csl = 1.0 / (8.0 * kPi), cdl = 3.0 / (4.0 * kPi);
-  // geometry and poles of the next (rotation, pass), loaded by every thread
-  // at indices clamped into range: unconditional loads leave no value to
-  // merge after a branch, so nothing waits for them before their use in the
-  // next pass
-  double g[9], tg[3];
+  // geometry, pole and Legendre values of the next (rotation, pass), loaded by
+  // every thread at indices in range: unconditional loads leave no value to
+  // merge after a branch, so nothing waits for them before their use.  The
+  // rotation's base is uniform, the place in it 32 bits.
+  double g[9], tg[3], w, ml[3];
+  const unsigned place = 8 * ((row ? P1 * L : 0) + half * P1 + min(j, P1 - 1)),
+                 wplace = 8 * (2 * row + t);
+  const int step = row ? -8 * L : 8 * L;
+  auto at = [](const double *base, unsigned bytes) {
+    typedef const char __attribute__((address_space(1))) gchar;
+    typedef const double __attribute__((address_space(1))) gdouble;
+    gchar *b = (gchar *)base;
+    asm("" : "+s"(b));  // a scalar base and a 32-bit place, not 64-bit vector sums
+    return *(gdouble *)(b + bytes);
+  };
   auto load = [&](long r_, int g_) {
     const long rc = r_ < nrot ? r_ : nrot - 1;
-    const int lat_ = min(g_ * R + krow, Nlat - 1);
-    const long b = rc * 3 * (long)M1 + (long)lat_ * L + lon;
-    g[0] = X[b]; g[1] = X[b + M1]; g[2] = X[b + 2 * M1];
-    g[3] = Xt[b]; g[4] = Xt[b + M1]; g[5] = Xt[b + 2 * M1];
-    g[6] = Xp[b]; g[7] = Xp[b + M1]; g[8] = Xp[b + 2 * M1];
-    for (int d = 0; d < 3; ++d) tg[d] = trg[(rc * 3 + d) * 2 + t];
+    const unsigned o = place + g_ * step;
+    const double *x = X + rc * 3 * M1, *xt = Xt + rc * 3 * M1, *xp = Xp + rc * 3 * M1;
+    g[0] = at(x, o); g[1] = at(x + M1, o); g[2] = at(x + 2 * M1, o);
+    g[3] = at(xt, o); g[4] = at(xt + M1, o); g[5] = at(xt + 2 * M1, o);
+    g[6] = at(xp, o); g[7] = at(xp + M1, o); g[8] = at(xp + 2 * M1, o);
+    w = at(qw + 4 * g_, wplace);
+  };
+  auto load_pole = [&](long r_) {
+    const long rc = r_ < nrot ? r_ : nrot - 1;
+    for (int d = 0; d < 3; ++d) tg[d] = at(trg + (rc * 3 + d) * 2 + t, 0);
+  };
+  const unsigned mplace = 8 * tm;
+  auto load_ml = [&](int g_) {
+    for (int n = 0; n < 3; ++n) ml[n] = at(mlt + (g_ * 3 + n) * ntri, mplace);
   };
   load(blockIdx.x, 0);
-  __syncthreads();  // Ml, Qw in
+  load_pole(blockIdx.x);
   for (long r = blockIdx.x; r < nrot; r += gridDim.x) {
-    const double tx = tg[0], ty = tg[1], tz = tg[2];
-    double acc[LMAX];
+    double acc[6][3] = {};
+    double f[6];
+    auto load_t = [&](int g_) {
+      const double *tc = Ts + ((g_ & 1) * 24 + par * 12 + c) * P1 + jj;
 #pragma unroll
-    for (int n = 0; n < LMAX; ++n) acc[n] = 0.0;
-    for (int gi = 0; gi < ng; ++gi) {
-      const double x0 = g[0], y0 = g[1], z0 = g[2];
-      const double xt = g[3], yt = g[4], zt = g[5];
-      const double xp = g[6], yp = g[7], zp = g[8];
-      if (gi + 1 < ng)
-        load(r, gi + 1);
-      else
-        load(r + gridDim.x, 0);
-      const int lat = gi * R + krow;
-      if (kvt && lat < Nlat) {
+      for (int i = 0; i < 6; ++i) f[i] = tc[i * P1];
+    };
+    auto legendre = [&] {
+#pragma unroll
+      for (int i = 0; i < 6; ++i)
+#pragma unroll
+        for (int n = 0; n < 3; ++n) acc[i][n] = fma(f[i], ml[n], acc[i][n]);
+    };
+#pragma unroll 1
+    for (int gi = 0; gi < NP; ++gi) {
+      {
+        const double yt = g[4], zt = g[5], xt = g[3], xp = g[6], yp = g[7], zp = g[8];
         const double nx = yt * zp - zt * yp, ny = zt * xp - xt * zp, nz = xt * yp - yt * xp;
-        const double w = Qw[t ? lat : P1 - lat];
-        const double dx = tx - x0, dy = ty - y0, dz = tz - z0;
+        const double dx = tg[0] - g[0], dy = tg[1] - g[1], dz = tg[2] - g[2];
+        const double wt = w;
+        const bool more = gi + 1 < NP;
+        load(more ? r : r + gridDim.x, more ? gi + 1 : 0);
         const double r2 = dx * dx + dy * dy + dz * dz;
-        double rinv = 1.0 / sqrt(r2);
-        if (r2 <= eps) rinv = 0;
+        const double rinv = r2 <= eps ? 0.0 : rsqrt_refined(r2);
         const double rinv2 = rinv * rinv;
         const double dd[6] = {dx * dx, dx * dy, dx * dz, dy * dy, dy * dz, dz * dz};
-        double *kv = Kv + (krow * L + lon) * kPtKs + t * 6;
+        double val, diag = 0.0;
         if (layer == 1) {
-          const double rn5 = cdl * w * (nx * dx + ny * dy + nz * dz) * rinv2 * rinv2 * rinv;
-#pragma unroll
-          for (int q = 0; q < 6; ++q) kv[q] = dd[q] * rn5;
+          val = wt * (nx * dx + ny * dy + nz * dz) * rinv2 * rinv2 * rinv;
         } else {
-          const double area = sqrt(nx * nx + ny * ny + nz * nz);
-          const double ar = csl * w * area * rinv;
-          const double ar2 = ar * rinv2;
+          const double n2 = nx * nx + ny * ny + nz * nz;
+          const double area = n2 > 0.0 ? n2 * rsqrt_refined(n2) : 0.0;
+          diag = wt * area * rinv;
+          val = diag * rinv2;
+        }
+        double v[6];
 #pragma unroll
-          for (int q = 0; q < 6; ++q)
-            kv[q] = dd[q] * ar2 + ((q == 0 || q == 3 || q == 5) ? ar : 0.0);
+        for (int i = 0; i < 6; ++i)
+          v[i] = (i == 0 || i == 3 || i == 5) ? fma(dd[i], val, diag) : dd[i] * val;
+        // v[2 q], v[2 q + 1]: first the rows' sum and difference of component
+        // 2 q + row, then the sums and differences over the half circles of
+        // the rows' combination half
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+          mirror_sums<16>(v[2 * q], v[2 * q + 1]);
+          mirror_sums<32>(v[2 * q], v[2 * q + 1]);
+        }
+        if (kvt) {
+          double *kv = Kv + ((gi & 1) * 4 + 2 * half) * kPart + j * kPtKs + t * 6 + row;
+#pragma unroll
+          for (int q = 0; q < 3; ++q) {
+            kv[2 * q] = v[2 * q];
+            kv[kPart + 2 * q] = v[2 * q + 1];
+          }
         }
       }
-      __syncthreads();  // Kv of the pass is in; the previous pass's T is consumed
-      if (fw && gi * R + frow < Nlat) {
-        const double *kv = Kv + frow * L * kPtKs + lk * kPtKs + li;
+      __syncthreads();  // Kv and the previous pass's T are in
+      {
+        // (the rows c >= 12 of A are other values; what they give is not read)
+        const double *kv = Kv + ((gi & 1) * 4 + wv) * kPart + li;
         v4d d = {0.0, 0.0, 0.0, 0.0}, e = {0.0, 0.0, 0.0, 0.0};
         double a[KS];
 #pragma unroll
-        for (int s = 0; s < KS; ++s) {
-          double v = kv[4 * s * kPtKs];
-          if constexpr (FOLD) {
-            const double w = kv[(4 * s + L / 2) * kPtKs];
-            v = tile ? v - w : v + w;
-          }
-          a[s] = li < 12 ? v : 0.0;
-        }
+        for (int s = 0; s < KS; ++s) a[s] = kv[min(4 * s + lk, P1 - 1) * kPtKs];
+        if (gi > 0) load_t(gi - 1);
 #pragma unroll
-        for (int s = 0; s < KS; s += 2) {  // two accumulation chains
-          d = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s], mf[s], d, 0, 0, 0);
-          e = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s + 1], mf[s + 1], e, 0, 0, 0);
+        for (int s = 0; s < KS; ++s) {  // two accumulation chains
+          if (s & 1)
+            e = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s], mf[s], e, 0, 0, 0);
+          else
+            d = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s], mf[s], d, 0, 0, 0);
         }
+        if (gi > 0) legendre();
+        load_ml(gi);
         d += e;
         if (fcol >= 0) {
+          double *o = Ts + ((gi & 1) * 24 + frow * 12 + lk) * P1 + fcol;
 #pragma unroll
-          for (int i = 0; i < 3; ++i) Ts[(frow * 12 + lk + 4 * i) * FP + fcol] = d[i];
-        }
-      }
-      __syncthreads();  // T of the pass is in
-      if (lt) {
-#pragma unroll 1
-        for (int row = 0; row < R; ++row) {
-          const int lat = gi * R + row;
-          if (lat >= Nlat) break;
-          // branch-free: degrees n >= len read finite values past the block
-          // (the next blocks, then zeros) into accumulators that are never
-          // written out
-          const double f = Ts[(row * 12 + c) * FP + jj];
-          const double *ml = Ml + mloff + lat;
-#pragma unroll
-          for (int n = 0; n < LMAX; ++n) acc[n] += f * ml[n * Nlat];
+          for (int i = 0; i < 3; ++i) o[4 * i * P1] = d[i];
         }
       }
     }
-    // the rotation's 12 output rows, cs rows per round through St
-    double *out = K1 + r * 12 * (long)Nc;
-    for (int c0 = 0; c0 < 12; c0 += cs) {
-      __syncthreads();  // T, or the previous round of St, is read
-      if (lt && c >= c0 && c < c0 + cs) {
+    __syncthreads();  // the last T is in
+    load_t(NP - 1);
+    legendre();
+    // the rotation's 12 rows, degree-major.  (The thread's index is opaque from
+    // here on: what is derived from it is not kept in registers over the passes.)
+    int id = tid, cc = c;
+    asm("" : "+v"(id), "+v"(cc));
+    const int lane = id & 63, li = lane & 15, lk = lane >> 4;
+    const unsigned v_rot = (unsigned)r / p0;  // rotations of a launch fit 32 bits
+    const double *fr = frag + v_rot % (p0 + 1) * frag_t + lane;
+    double op[16];
+    auto operand = [&](int l) {
+      const double *f = fr + rot_frag_off(l, nsmall);
+      if (l < nsmall) {
 #pragma unroll
-        for (int n = 0; n < LMAX; ++n)
-          if (n < len) St[(c - c0) * Nc + dpos[off + n]] = acc[n];
+        for (int k = 0; k < 4; ++k) op[k] = f[64 * k];
+      } else {
+#pragma unroll
+        for (int k = 0; k < 16; ++k) op[k] = f[64 * k];
       }
-      __syncthreads();
-      const int nrow = min(cs, 12 - c0);
-      for (int i = tid; i < nrow * Nc; i += blockDim.x) out[c0 * Nc + i] = St[i];
+    };
+    load_pole(r + gridDim.x);
+    __syncthreads();  // T is read
+#pragma unroll
+    for (int n = 0; n < 3; ++n) {
+      if (dp[n] < 0) continue;
+      double *o = St + cc * (Nc + 1) + dp[n];
+#pragma unroll
+      for (int i = 0; i < 6; ++i) o[i * (Nc + 1)] = acc[i][n];
+    }
+    int l = p0 - wv;
+    if (l >= 0) operand(l);
+    __syncthreads();
+    // per-degree products, in place: a degree's columns depend on its own
+    // entries only, and one wave forms them all.  The waves take the degrees
+    // from the longest down, back and forth; the next degree's operand is
+    // loaded while the current one's results are stored.
+#pragma unroll 1
+    for (int i = 0; l >= 0; ++i) {
+      const int n = min(2 * l + 1, 2 * p0);
+      double *ro = St + l * l;  // the degree's first entry
+      const double *av = ro + li * (Nc + 1);
+      v4d e0 = {0.0, 0.0, 0.0, 0.0}, e1 = {0.0, 0.0, 0.0, 0.0};
+      double a[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) a[k] = av[min(4 * k + lk, n - 1)];  // the operand's zeros past n
+      if (l < nsmall) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          e0 = __builtin_amdgcn_mfma_f64_16x16x4f64(a[k], op[k], e0, 0, 0, 0);
+      } else {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          e0 = __builtin_amdgcn_mfma_f64_16x16x4f64(a[k], op[k], e0, 0, 0, 0);
+          e1 = __builtin_amdgcn_mfma_f64_16x16x4f64(a[k], op[8 + k], e1, 0, 0, 0);
+        }
+      }
+      constexpr int nw = kPtThreads / 64;
+      l = p0 - (i + 1) * nw - (i & 1 ? wv : nw - 1 - wv);
+      if (l >= 0) operand(l);
+#pragma unroll
+      for (int u = 0; u < 3; ++u) {
+        double *o = ro + (lk + 4 * u) * (Nc + 1) + li;
+        if (li < n) o[0] = e0[u];
+        if (16 + li < n) o[16] = e1[u];
+      }
+    }
+    __syncthreads();
+    // longitude phases, in coefficient order
+    for (int k = id; k < Nc; k += kPtThreads) {
+      const int4 src = sources[k];
+      const double *ph = phase + 2 * (((unsigned)r % p0) * (p0 + 1) + src.z);
+      // a copy, cosine: x0 r0 - x1 r1, sine: x0 r1 + x1 r0
+      const double r0 = ph[0], r1 = ph[1];
+      const double w0 = src.w == 0 ? 1.0 : (src.w == 2 ? r1 : r0);
+      const double w1 = src.w == 0 ? 0.0 : (src.w == 2 ? r0 : -r1);
+      double *o = K2 + r * 12 * (long)Nc + k;
+#pragma unroll 4
+      for (int i = 0; i < 12; ++i)
+        o[i * Nc] = St[i * (Nc + 1) + src.x] * w0 + St[i * (Nc + 1) + src.y] * w1;
     }
     __syncthreads();  // St read before the next rotation's kernel values
   }
@@ -774,37 +937,124 @@ static long singular_elems_per_ves(int p0, int p1, bool fused) {
   e += 3 * nr * 3 * M1;                 // X, Xt, Xp
   e += nr * 3 * 2;                      // poles
   if (!fused) e += nr * 12 * M1;        // K0
-  e += nr * 12 * Nc;                    // K1
   e += nr * 12 * Nc;                    // K2
-  e += 3 * Nc * 3 * Ng;                 // M1 rearranged
   long w1 = shc2grid_work(nr * 3, p0, p1);
-  if (!fused) w1 = std::max(w1, grid2shc_work(nr * 12, p1, p0));
-  w1 = std::max(w1, grid2shc_work(9 * Nc, p0, p0));
-  w1 = std::max(w1, 3 * nr * 12 * Nc);  // rotation scratch
+  if (fused) {
+    w1 = std::max(w1, 3 * (p0 + nr) * Nc);  // rotation scratch
+  } else {
+    e += nr * 12 * Nc;                  // K1
+    e += 3 * Nc * 3 * Ng;               // M1 rearranged
+    w1 = std::max(w1, grid2shc_work(nr * 12, p1, p0));
+    w1 = std::max(w1, grid2shc_work(9 * Nc, p0, p0));
+    w1 = std::max(w1, 3 * nr * 12 * Nc);  // rotation scratch
+  }
   e += w1;
   return e;
 }
 
-// Launch shape of k_pole_transpose for (p0, p1) on the current device:
-// R latitude rows per pass (3 where the LDS allows, else fewer), threads
-// covering the three roles, and the persistent grid's workgroups per CU;
-// threads == 0 where the fused stage does not apply.
+// k_pole_transpose's tables: RotateTranspose's per-degree blocks Mr[t][l] in
+// operand order (rot_frag_off: tile ct, step s, lane: column 16 ct + lane % 16,
+// entry 4 s + lane / 16, zero past the degree's entries), MatLegendre(p0, p1)
+// by latitude, degree of a triple and triple (zero past a block), and for the
+// single and the double layer SingularWeights(p1) times the kernel's factor by
+// latitude pair, row of the pair and pole (zero where the equator is its own
+// mirror row).
+struct PoleTables {
+  double *frag = nullptr, *ml = nullptr, *qw = nullptr;
+  int nsmall = 0;
+  long per_t = 0;  // doubles per latitude
+};
+std::map<std::tuple<int, int, int>, PoleTables> g_pole_tables;  // (device, p0, p1)
+
+const PoleTables *pole_tables(int p0, int p1) {
+  const RotMatsDev *rm = rot_mats(p0);
+  const ShMatsDev *sm = sh_mats(p1, p0);
+  int dev = 0;
+  if (!rm || !sm || hipGetDevice(&dev) != hipSuccess) return nullptr;
+  std::lock_guard<std::mutex> lk(g_mu);
+  const auto key = std::make_tuple(dev, p0, p1);
+  auto it = g_pole_tables.find(key);
+  if (it != g_pole_tables.end()) return &it->second;
+  const RotMatsHost &h = *rm->h;
+  PoleTables r;
+  while (r.nsmall <= p0 && h.len[r.nsmall] <= 16) ++r.nsmall;
+  r.per_t = rot_frag_off(p0 + 1, r.nsmall);
+  const size_t nfrag = (size_t)(p0 + 1) * r.per_t;
+  const int ntri = pole_triples(p0, p0 + 1), NP = p1 / 2 + 1;
+  const size_t nml = (size_t)NP * 3 * ntri;
+  std::vector<double> f(nfrag + nml + 2 * 4 * NP, 0.0), qw;
+  singular_weights(p1, qw);
+  for (int t = 0; t <= p0; ++t)
+    for (int l = 0; l <= p0; ++l) {
+      const int len = h.len[l], steps = l < r.nsmall ? 4 : 8;
+      const double *M = &h.data[h.off[t * (p0 + 1) + l]];
+      double *o = &f[(size_t)t * r.per_t + rot_frag_off(l, r.nsmall)];
+      for (int col = 0; col < len; ++col)
+        for (int k = 0; k < len; ++k)
+          o[((col / 16) * steps + k / 4) * 64 + (k % 4) * 16 + col % 16] = M[(size_t)col * len + k];
+    }
+  for (int m = 0, t0 = 0; m <= p0; ++m)
+    for (int par = 0; par < 2; ++par) {
+      const int cnt = pole_degrees(p0 + 1 - m, par);
+      const double *src = &sm->h->data[sm->h->MlT[m]];
+      for (int n = 0; n < cnt; ++n)
+        for (int lat = 0; lat < NP; ++lat)
+          f[nfrag + (size_t)(lat * 3 + n % 3) * ntri + t0 + n / 3] =
+              src[(par + 2 * n) * (p1 + 1) + lat];
+      t0 += (cnt + 2) / 3;
+    }
+  for (int layer = 0; layer < 2; ++layer)
+    for (int i = 0; i < 4 * NP; ++i) {
+      const int row = i / 2 % 2, lat = row ? p1 - i / 4 : i / 4;
+      if (row && lat == i / 4) continue;
+      f[nfrag + nml + layer * 4 * NP + i] =
+          qw[i % 2 ? lat : p1 - lat] * (layer ? 3.0 / (4.0 * kPi) : 1.0 / (8.0 * kPi));
+    }
+  if (hipMalloc(&r.frag, sizeof(double) * f.size()) != hipSuccess) return nullptr;
+  r.ml = r.frag + nfrag;
+  r.qw = r.ml + nml;
+  if (hipMemcpy(r.frag, f.data(), sizeof(double) * f.size(), hipMemcpyHostToDevice) !=
+      hipSuccess) {
+    (void)hipFree(r.frag);
+    return nullptr;
+  }
+  return &(g_pole_tables[key] = r);
+}
+
+// k_pole_transpose's instance of the upsampled order p1; null where there is
+// none.
+const void *pole_instance(int p1) {
+  switch (p1) {
+    case 12: return (const void *)k_pole_transpose<12>;
+    case 14: return (const void *)k_pole_transpose<14>;
+    case 16: return (const void *)k_pole_transpose<16>;
+    case 18: return (const void *)k_pole_transpose<18>;
+    case 20: return (const void *)k_pole_transpose<20>;
+    case 22: return (const void *)k_pole_transpose<22>;
+    case 24: return (const void *)k_pole_transpose<24>;
+    case 26: return (const void *)k_pole_transpose<26>;
+    case 28: return (const void *)k_pole_transpose<28>;
+    case 30: return (const void *)k_pole_transpose<30>;
+    case 32: return (const void *)k_pole_transpose<32>;
+    default: return nullptr;
+  }
+}
+
+// Launch shape of k_pole_transpose for (p0, p1) on the current device: the
+// persistent grid's workgroups; kern == nullptr where the fused stage does not
+// apply.
 struct PoleShape {
-  int R = 0, threads = 0, blocks = 0;
+  const void *kern = nullptr;
+  int blocks = 0;
   size_t lds = 0;
-  bool small = false;  // the <9, 16> instance (p0 <= 8, p1 = 16)
 };
 
 PoleShape pole_fused_shape(int p0, int p1) {
   PoleShape sh;
-  // the instances' shapes: p0 <= 8 with p1 = 16, p0 <= 16 with p1 = 32
-  // (the build's upsampled order 2 p0)
-  const bool small = p0 <= 8 && p1 == 16;
-  if (!small && !(p0 <= 16 && p1 == 32)) return sh;
-  // MFMA wave tiles per row: the two parities of m at p1 = 32 (the kernel's
-  // FOLD), else 16 consecutive columns
-  const int L = 2 * p1, F = 2 * p0, FP = 16 * ((F + 15) / 16), NT = small ? FP / 16 : 2;
-  const long Nc = sh_ncoef(p0);
+  // The build's upsampled orders 2 p0 for p0 = 6 .. 16: 16 columns per parity
+  // and 256 threads hold the roles up to p0 = 16, p1 = 32.
+  const void *kern = 2 * p0 <= p1 ? pole_instance(p1) : nullptr;
+  if (!kern || pole_legendre_threads(p0) > kPtThreads) return sh;
   int dev = 0, maxlds = 0, cus = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&maxlds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) !=
@@ -813,32 +1063,17 @@ PoleShape pole_fused_shape(int p0, int p1) {
     (void)hipGetLastError();
     return sh;
   }
-  const void *kern = small ? (const void *)k_pole_transpose<9, 16>
-                           : (const void *)k_pole_transpose<17, 32>;
-  for (int R = 3; R >= 1; --R) {
-    const int threads =
-        64 * std::max({(int)cdiv(2L * R * L, 64), R * NT, (int)cdiv(12L * F, 64)});
-    const long stage = (long)R * L * kPtKs + (long)R * 12 * FP;
-    const size_t lds = sizeof(double) * (size_t)pole_lds_doubles(R, p0, p1, small ? 9 : 17);
-    if (threads > 384 || stage < Nc || lds > (size_t)maxlds) continue;
-    if (lds > 64 * 1024 && hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                               (int)lds) != hipSuccess) {
-      (void)hipGetLastError();
-      continue;
-    }
-    int nb = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kern, threads, lds) != hipSuccess) {
-      (void)hipGetLastError();
-      continue;
-    }
-    if (nb < 1) continue;
-    sh.R = R;
-    sh.threads = threads;
-    sh.blocks = nb * cus;
-    sh.lds = lds;
-    sh.small = small;
+  const size_t lds = sizeof(double) * (size_t)pole_lds_doubles(p0, p1);
+  if (lds > (size_t)maxlds) return sh;
+  int nb = 0;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kern, kPtThreads, lds) != hipSuccess) {
+    (void)hipGetLastError();
     return sh;
   }
+  if (nb < 1) return sh;
+  sh.kern = kern;
+  sh.blocks = nb * cus;
+  sh.lds = lds;
   return sh;
 }
 
@@ -856,7 +1091,7 @@ int singular_build(const double *X0, long Nv, int p0, int p1, T *SL, T *DL, hipS
   const PoleShape ps = std::is_same<T, double>::value && g_pole_fused.load(std::memory_order_relaxed)
                            ? pole_fused_shape(p0, p1)
                            : PoleShape();
-  const bool fused = ps.threads > 0;
+  const bool fused = ps.kern != nullptr;
   const long per = singular_elems_per_ves(p0, p1, fused);
   const long budget = (6L << 30) / (long)sizeof(T);
   long chunk = std::max(1L, std::min(Nv, budget / per));
@@ -885,9 +1120,9 @@ int singular_build(const double *X0, long Nv, int p0, int p1, T *SL, T *DL, hipS
     T *Xp = p; p += rot * 3 * M1;
     T *P = p; p += rot * 3 * 2;
     T *K0 = p; if (!fused) p += rot * 12 * M1;
-    T *K1 = p; p += rot * 12 * Nc;
+    T *K1 = p; if (!fused) p += rot * 12 * Nc;
     T *K2 = p; p += rot * 12 * Nc;
-    T *M1a = p; p += cv * 3 * Nc * 3 * Ng;
+    T *M1a = p; if (!fused) p += cv * 3 * Nc * 3 * Ng;
     T *w = p;
     const long nx0 = cv * 3 * Ng;
     k_copy_cast_grid<T><<<grid_for(nx0), 256, 0, st>>>(X0 + v0 * 3 * Ng, nx0, x0);
@@ -902,16 +1137,19 @@ int singular_build(const double *X0, long Nv, int p0, int p1, T *SL, T *DL, hipS
       if constexpr (std::is_same<T, double>::value) {
         if (fused) {
           const double *mft = sht_mft<double>(p1, p0);
-          const double *mlt = sht_mlt<double>(p1, p0);
           const RotMatsDev *rm = rot_mats(p0);
-          if (!mft || !mlt || !rm) return VES3D_MEMORY_ERROR;
+          const PoleTables *pt = pole_tables(p0, p1);
+          if (!mft || !rm || !pt) return VES3D_MEMORY_ERROR;
           const unsigned nb = (unsigned)std::min<long>(rot, ps.blocks);
-          if (ps.small)
-            k_pole_transpose<9, 16><<<nb, ps.threads, ps.lds, st>>>(
-                X, Xt, Xp, P, qw, rot, p0, ps.R, mft, mlt, layer, rm->iperm, K1);
-          else
-            k_pole_transpose<17, 32><<<nb, ps.threads, ps.lds, st>>>(
-                X, Xt, Xp, P, qw, rot, p0, ps.R, mft, mlt, layer, rm->iperm, K1);
+          const int *dpos = rm->iperm;
+          const double *pqw = pt->qw + layer * 4 * (p1 / 2 + 1);
+          const int4 *sources = (const int4 *)rm->scatter;
+          long nrot = rot, frag_t = pt->per_t;
+          int order = p0, lay = layer, nsmall = pt->nsmall;
+          void *args[] = {&X,   &Xt,   &Xp,       &P,      &pqw,     &nrot,
+                          &order, &mft,  (void *)&pt->ml,     &lay,    &dpos,    (void *)&pt->frag,
+                          &frag_t, &nsmall, &sources, (void *)&rm->phase, &K2};
+          V3D_HIP(hipLaunchKernel(ps.kern, dim3(nb), dim3(kPtThreads), args, ps.lds, st));
           V3D_CHECK(launch_status());
         }
       }
@@ -920,8 +1158,8 @@ int singular_build(const double *X0, long Nv, int p0, int p1, T *SL, T *DL, hipS
             X, Xt, Xp, P, qw, rot, p1, layer == 0 ? K0 : nullptr, layer == 1 ? K0 : nullptr);
         V3D_CHECK(launch_status());
         V3D_CHECK(sht_shc2grid_transpose<T>(K0, rot * 12, p1, p0, K1, w, st));
+        V3D_CHECK(rotate_transpose<T>(K1, cv, p0, 12, K2, w, st));
       }
-      V3D_CHECK(rotate_transpose<T>(K1, cv, p0, 12, K2, w, st, fused));
       if constexpr (std::is_same<T, double>::value) {
         if (fused) {  // rearrangement and Grid2SHC in one pass
           const ShMatsDev *sm = sh_mats(p0, p0);
@@ -1057,7 +1295,7 @@ int self_apply(const TM *SL, const double *F, const TM *DL, const double *G, lon
 
 template int rotate_all<double>(const double *, long, int, int, double *, double *, hipStream_t);
 template int rotate_transpose<double>(const double *, long, int, int, double *, double *,
-                                       hipStream_t, bool);
+                                      hipStream_t);
 template int singular_build<double>(const double *, long, int, int, double *, double *, hipStream_t);
 template int singular_build<float>(const double *, long, int, int, float *, float *, hipStream_t);
 template int self_apply<double>(const double *, const double *, const double *, const double *,
@@ -1084,15 +1322,15 @@ int ves3d_hip_rotate_transpose_f64(const double *S_in, size_t N, int p, int dof,
   const long nc = sh_ncoef(p);
   double *w = (double *)workspace(kWsSing1, sizeof(double) * 2L * N * (p + 1) * p * dof * nc);
   if (!w) return VES3D_MEMORY_ERROR;
-  return rotate_transpose<double>(S_in, (long)N, p, dof, S_out, w, (hipStream_t)stream, false);
+  return rotate_transpose<double>(S_in, (long)N, p, dof, S_out, w, (hipStream_t)stream);
 }
 int ves3d_hip_pole_kernel_shape(int p0, int p1, int *rows_host, int *threads_host,
                                 int *workgroups_host) {
   if (p0 < 1 || p1 < 1 || p0 > 128 || p1 > 255) return VES3D_INVALID_PARAMETER;
   const PoleShape ps =
       g_pole_fused.load(std::memory_order_relaxed) ? pole_fused_shape(p0, p1) : PoleShape();
-  if (rows_host) *rows_host = ps.R;
-  if (threads_host) *threads_host = ps.threads;
+  if (rows_host) *rows_host = ps.kern ? 2 : 0;  // a latitude and its mirror
+  if (threads_host) *threads_host = ps.kern ? kPtThreads : 0;
   if (workgroups_host) *workgroups_host = ps.blocks;
   return VES3D_SUCCESS;
 }
