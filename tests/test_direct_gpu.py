@@ -87,6 +87,44 @@ def test_direct_stokes_dl(hip, orc, dtype, tol, use_qw):
     assert _relerr(pot.double().cpu().numpy(), ref) < tol
 
 
+@pytest.mark.parametrize("dl", [False, True])
+@pytest.mark.parametrize("dtype,tol", [(torch.float64, 1e-12), (torch.float32, 2e-5)])
+@pytest.mark.parametrize("nv,ss,ts", [(3, 1, 1), (3, 31, 65), (3, 33, 64), (3, 514, 129),
+                                      (4100, 37, 3)])
+def test_direct_stokes_edges(hip, orc, nv, ss, ts, dtype, tol, dl):
+    """Sources split over 4 and 16 waves with parts of every length down to
+    none, runs around 32, and vesicles with coincident points (0), a distance
+    whose square is below the normal numbers (1) and one whose square
+    overflows (2, both single layer only); tolerances as in the tests above."""
+    src, den, nrm, trg, qw = (a.astype(np.float32).astype(np.float64)
+                              for a in _vesicle_case(nv, ss, ts))
+    n = min(ss, ts)
+    trg[0, :, :n] = src[0, :, :n]
+    tiny, huge = (1e-160, 1e200) if dtype == torch.float64 else (1e-20, 1e30)
+    if not dl:
+        src[1, :, ss - 1] = np.float64(np.float32(tiny)) if dtype == torch.float32 else tiny
+        trg[1, :, 0] = 0
+        trg[2, :, ts - 1] = np.float64(np.float32(huge)) if dtype == torch.float32 else huge
+    ref = np.zeros((nv, 3, ts))
+    geo = (OL.ci(ss), OL.ci(ts), OL.ci(nv), OL.ci(0), OL.ci(ts), OL.p(qw), OL.p(trg), OL.p(src))
+    pot = torch.zeros((nv, 3, ts), dtype=dtype, device="cuda")
+    c = lambda a: _cuda(a, dtype)
+    if dl:
+        orc.orc_direct_stokes_dl(*geo, OL.p(nrm), OL.p(den), OL.p(ref))
+        K.direct_stokes_dl(c(src), c(nrm), c(den), c(qw), ss, ts, nv, c(trg), 0, ts, pot)
+    else:
+        orc.orc_direct_stokes(*geo, OL.p(den), OL.p(ref))
+        K.direct_stokes(c(src), c(den), c(qw), ss, ts, nv, c(trg), 0, ts, pot)
+    out = pot.double().cpu().numpy()
+    assert np.all(np.isfinite(ref))
+    # a pair whose r^2 overflows is at least sqrt(largest number) apart and gives
+    # at most 2 w |f| / (8 pi r) < 1 / r per component, which the kernel drops
+    lost = 0 if dl else ss / float(torch.finfo(dtype).max) ** 0.5
+    for v in range(3):
+        assert np.max(np.abs(out[v] - ref[v])) <= tol * np.max(np.abs(ref[v])) + lost, v
+    assert _relerr(out[3:], ref[3:]) < tol if nv > 3 else True
+
+
 def test_direct_stokes_bad_range(hip):
     src = torch.zeros(3 * 8, dtype=torch.float64, device="cuda")
     pot = torch.zeros(3 * 8, dtype=torch.float64, device="cuda")
