@@ -9,9 +9,9 @@
 //     longitudes);
 //   analysis: the Fourier sums of the grid rows on MFMA, then the Legendre
 //     sums.
-// Orders 16 and 32 in FP64, here / as GEMMs in us: N = 6 functions synthesis 7.9
-// / 11.9, of three variants 8.7 / 30, analysis 8.4 / 11.6; N = 1536: 17 / 25, 35
-// / 61, 16 / 23; N = 6144: 38 / 56, 106 / 150, 54 / 55.
+// Orders 16 and 32 in FP64, here / as GEMMs in us (back to back): N = 6 functions
+// synthesis 7.9 / 11.9, of three variants 8.7 / 30, analysis 8.4 / 11.6; N =
+// 1536: 15 / 25, 30 / 61, 16 / 23; N = 6144: 35 / 56, 93 / 150, 54 / 55.
 // Longitudes lon and lon + p lie pi apart, where the Fourier functions of
 // order m differ by (-1)^m: the frequencies are kept as an even-order half E
 // and an odd-order half O (p of each), a synthesis writes E + O and E - O, an
@@ -33,6 +33,7 @@ namespace {
 constexpr int kThreads = 512, kWaves = kThreads / 64;
 constexpr size_t kLdsMost = 64 * 1024;  // two workgroups per CU
 constexpr int kMaxSteps = 8;            // orders of the contracted side up to 32
+constexpr int kBatch = 8;               // table values a thread has in flight
 
 __host__ __device__ __forceinline__ int up16(int v) { return (v + 15) & ~15; }
 
@@ -119,7 +120,14 @@ size_t analysis_lds(int p0, int p1, int fg, size_t es) {
 }
 
 // Latency-bound with few functions (one workgroup per function and variant),
-// else by the Legendre sums' LDS reads.
+// else by the writes (2112 per function and variant at order 32: 93 us for 6144
+// functions and three variants are 3.4 TB/s).  A thread takes a latitude and its
+// mirror together, whose sums share the products of the even and the odd
+// degrees, and has kBatch table values in flight, past an order's last degree
+// as zeros: one latitude per thread, with the last few values one by one, took
+// 7.3 instead of 6.0 us for 6 functions at order 24, 106 instead of 93 us there.
+// (The analysis gains nothing from either: its sums are bound by the LDS reads,
+// which stay, 50 -> 60 us.)
 template <typename T, int FG, int KS>
 __global__ __launch_bounds__(kThreads) void k_synth(const SynthArgs<T> a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
@@ -147,21 +155,39 @@ __global__ __launch_bounds__(kThreads) void k_synth(const SynthArgs<T> a) {
     }
   }
   __syncthreads();
-  for (int i = tid; i < 2 * p0 * L; i += kThreads) {
-    const int j = i / L, l = i % L, m = (j + 1) / 2;
+  // a table value and its mirror latitude's differ by (-1)^(n - m) (the first
+  // derivatives' by the opposite sign)
+  const int Lh = (L + 1) / 2;
+  const T mirror = kind == 1 || kind == 2 ? T(-1) : T(1);
+  for (int i = tid; i < 2 * p0 * Lh; i += kThreads) {
+    const int j = i / Lh, l = i % Lh, m = (j + 1) / 2, len = p0 + 1 - m;
     // an order's blocks of the four derivative kinds follow each other
-    const T *__restrict__ t = leg + 4 * legendre_off(p0, m, L) + kind * (p0 + 1 - m) * L + l;
+    const T *__restrict__ t = leg + 4 * legendre_off(p0, m, L) + kind * len * L + l;
     const T *c = C + block_off(p0, j) * FG;
-    T s[FG] = {};
-#pragma unroll 8
-    for (int n = 0; n <= p0 - m; ++n) {
-      const T x = t[n * L];
+    T se[FG] = {}, so[FG] = {};
+    for (int n0 = 0; n0 < len; n0 += kBatch) {
+      T x[kBatch];
 #pragma unroll
-      for (int f = 0; f < FG; ++f) s[f] = fma(x, c[n * FG + f], s[f]);
+      for (int u = 0; u < kBatch; ++u) x[u] = t[min(n0 + u, len - 1) * L];
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u) {
+        const T v = n0 + u < len ? x[u] : T(0);
+        const T *cu = c + min(n0 + u, len - 1) * FG;
+#pragma unroll
+        for (int f = 0; f < FG; ++f) {
+          if (u & 1)
+            so[f] = fma(v, cu[f], so[f]);
+          else
+            se[f] = fma(v, cu[f], se[f]);
+        }
+      }
     }
-    T *b = B + l * ldr + (m & 1 ? K : 0) + half_place(j);
+    const int place = (m & 1 ? K : 0) + half_place(j), lm = L - 1 - l;
 #pragma unroll
-    for (int f = 0; f < FG; ++f) b[f * L * ldr] = a.alpha * s[f];
+    for (int f = 0; f < FG; ++f) {
+      B[(f * L + l) * ldr + place] = a.alpha * (se[f] + so[f]);
+      if (lm != l) B[(f * L + lm) * ldr + place] = a.alpha * (mirror * (se[f] - so[f]));
+    }
   }
   __syncthreads();
   const long rows = (a.N - f0) * L;  // rows left from this workgroup on
@@ -325,16 +351,10 @@ const T *frag_table(int p0, int p1, int kind, const ShMatsHost &h) {
 }
 
 // Functions per workgroup: as many as share the tables without leaving CUs
-// idle (0: the GEMMs run).  With both orders above 24 in FP64 a workgroup's
-// LDS holds one function, so every function reads the Legendre tables again;
-// from `many` functions on the GEMMs, which share them over 64, are faster:
-// orders 32 -> 32, synthesis of N = 1536 / 6144 functions 31.4 / 104 us here
-// and 32.4 / 93 us there, of three variants 82 / 304 and 82 / 248 us, analysis
-// 42 / 155 and 38 / 100 us.
-int functions_per_group(long N, int nvar, long many, size_t (*lds)(int, int, int, size_t), int p0,
-                        int p1, size_t es) {
+// idle (0: the GEMMs run).
+int functions_per_group(long N, int nvar, size_t (*lds)(int, int, int, size_t), int p0, int p1,
+                        size_t es) {
   if (!gemm_is_default() || p0 > 4 * kMaxSteps || N >= (1L << 31)) return 0;
-  if (es == 8 && p0 > 24 && p1 > 24 && N * nvar >= many) return 0;
   for (int fg : {4, 2, 1}) {
     if (lds(p0, p1, fg, es) > kLdsMost) continue;
     if (fg == 1 || (N + fg - 1) / fg * nvar >= 512) return fg;
@@ -376,7 +396,7 @@ template <typename T>
 bool synth_fused(const T *S, long N, int p0, int p1, int nvar, const ShMatsHost &h, const T *mats,
                  const int *dleg, const int *dfour, T *const *X, T alpha, hipStream_t st,
                  int *status) {
-  const int fg = functions_per_group(N, nvar, 4096, synth_lds, p0, p1, sizeof(T));
+  const int fg = functions_per_group(N, nvar, synth_lds, p0, p1, sizeof(T));
   if (fg == 0) return false;
   SynthArgs<T> a{};
   a.S = S;
@@ -401,7 +421,15 @@ bool synth_fused(const T *S, long N, int p0, int p1, int nvar, const ShMatsHost 
 template <typename T>
 bool analysis_fused(const T *X, long N, int p0, int p1, bool transpose, const ShMatsHost &h,
                     const T *mats, T *S, hipStream_t st, int *status) {
-  const int fg = functions_per_group(N, 1, 1024, analysis_lds, p0, p1, sizeof(T));
+  // With both orders above 24 in FP64 a workgroup's LDS holds one or two
+  // functions, which read the Legendre tables again; for many functions the
+  // GEMMs, which share them over 64, are faster.  Orders 32 -> 32 (one fits), N =
+  // 1024 / 1536 / 6144: 29 / 43 / 157 us here and 32 / 38 / 100 us there; orders 28
+  // -> 28 (two), N = 3072 / 6144: 41 / 80 and 43 / 75 us.
+  if (sizeof(T) == 8 && p0 > 24 && p1 > 24 &&
+      N >= (analysis_lds(p0, p1, 2, sizeof(T)) > kLdsMost ? 1280 : 5120))
+    return false;
+  const int fg = functions_per_group(N, 1, analysis_lds, p0, p1, sizeof(T));
   if (fg == 0) return false;
   const T *frag = frag_table<T>(p0, p1, transpose ? 4 : 3, h);
   if (!frag) {
