@@ -254,6 +254,29 @@ def test_pole_kernel_orders(hip, p0, p1, nv):
     assert rel(out[1][0], out[0][0]) < 1e-12 and rel(out[1][1], out[0][1]) < 1e-12
 
 
+@pytest.mark.parametrize("p,nv", [(1, 1), (2, 3), (4, 70), (12, 2), (12, 330), (16, 5)])
+@pytest.mark.parametrize("dt", [torch.float64, torch.float32])
+def test_self_apply_rows_split(hip, p, nv, dt):
+    """Rows split over 16 waves with parts down to none, partial and whole blocks
+    of columns, one layer and both, and the sizes of the unsplit kernel (order
+    12, 330 vesicles).  The matrices' entries are taken as they are and summed
+    in FP64: n = 6 Ncoef products, n eps of the sum of their sizes."""
+    n = 3 * p * (p + 2)
+    g = torch.Generator(device="cuda").manual_seed(p + nv)
+    M, D = (torch.randn((nv, n, n), dtype=dt, device="cuda", generator=g) for _ in range(2))
+    F, H = (torch.randn((nv, n), dtype=torch.float64, device="cuda", generator=g) for _ in range(2))
+    for both in (False, True):
+        V = torch.full((nv, n), 7.0, dtype=torch.float64, device="cuda")
+        G.self_apply(M, F, D if both else None, H if both else None, nv, p, V)
+        size = torch.zeros_like(V)
+        ref = torch.zeros_like(V)
+        for A, x in ((M, F),) + (((D, H),) if both else ()):
+            for v in range(nv):
+                ref[v] += x[v] @ A[v].double()
+                size[v] += x[v].abs() @ A[v].double().abs()
+        assert bool(((V - ref).abs() <= 2 * n * 2.3e-16 * size).all())
+
+
 @pytest.mark.parametrize("p0", [16, 8])
 def test_singular_build_fused_pole_stage(hip, p0):
     """The FP64 build's fused pole kernel + transposed synthesis (the default

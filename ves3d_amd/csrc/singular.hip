@@ -19,7 +19,7 @@
 // every GEMM stage in FP32 and keeps the pole kernel (singular weights, 1/r
 // near the rotated pole) in FP64.  Both write the operator's (a, b) and
 // (b, a) blocks equal (the rows of one symmetric tensor component), which
-// the step's self apply relies on (k_self_apply_sym).
+// the step's self apply relies on (k_self_apply_split).
 #include <algorithm>
 #include <atomic>
 #include <cmath>
@@ -1229,49 +1229,65 @@ __global__ __launch_bounds__(256) void k_self_apply(const TM *__restrict__ SL,
   V[v * n + c] = (acc0 + acc1) + (acc2 + acc3);
 }
 
-// As k_self_apply for the singular build's operators, whose 3 x 3 blocks of
-// Ncoef x Ncoef satisfy B_ab = B_ba (block (a, b) holds the rows of the
-// symmetric tensor component c(a, b), formed once and written to both):
-// thread cc reads the six blocks a <= b at column cc once and forms
-// V[b Nc + cc] = sum_a sum_k F[a Nc + k] B_ab[k][cc] for b = 0, 1, 2 --
-// two thirds of the general kernel's matrix reads.
-template <typename TM>
-__global__ __launch_bounds__(512) void k_self_apply_sym(const TM *__restrict__ SL,
-                                                         const double *__restrict__ F,
-                                                         const TM *__restrict__ DL,
-                                                         const double *__restrict__ G, int nc,
-                                                         double *__restrict__ V) {
-  extern __shared__ double sh[];
-  const int n = 3 * nc;
+// The same with a workgroup's 16 waves on parts of the rows of 64 columns, the
+// parts added in order through LDS.  SYM: the singular build's operators, whose
+// 3 x 3 blocks of Ncoef x Ncoef satisfy B_ab = B_ba (block (a, b) holds the rows
+// of the symmetric tensor component c(a, b), formed once and written to both):
+// lane cc reads the six blocks a <= b at column cc once and forms V[b Nc + cc] =
+// sum_a sum_k F[a Nc + k] B_ab[k][cc] for b = 0, 1, 2 -- two thirds of the
+// general form's matrix reads.
+// Bound: the matrix reads (5.9 TB/s for 512 vesicles at order 16) or, with few
+// vesicles, their latency.  A thread per column down all rows, before -> after
+// in us (FP64, order 12, symmetric): 2 vesicles 23 -> 9, 48: 39 -> 13, 512: 122
+// -> 125; order 16: 66 -> 14, 72 -> 29, 353 -> 344; general: 37 -> 9, 116 -> 45,
+// 508 -> 504.
+template <typename TM, bool SYM>
+__global__ __launch_bounds__(1024) void k_self_apply_split(const TM *__restrict__ SL,
+                                                           const double *__restrict__ F,
+                                                           const TM *__restrict__ DL,
+                                                           const double *__restrict__ G, int nc,
+                                                           double *__restrict__ V) {
+  constexpr int kSums = SYM ? 3 : 1;
+  __shared__ double part[15][kSums][64];
+  const int n = 3 * nc, lines = SYM ? nc : n;  // rows and columns of a block
   const long v = blockIdx.y;
-  const int cc = blockIdx.x * blockDim.x + threadIdx.x;
-  double *f = sh, *g = sh + n;
-  for (int i = threadIdx.x; i < n; i += blockDim.x) {
-    f[i] = SL ? F[v * n + i] : 0.0;
-    g[i] = DL ? G[v * n + i] : 0.0;
-  }
-  __syncthreads();
-  if (cc >= nc) return;
-  double v0 = 0, v1 = 0, v2 = 0;
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int col = blockIdx.x * 64 + lane, per = (lines + 15) / 16;
+  const int k0 = min(wv * per, lines), k1 = min(k0 + per, lines);
+  double s[kSums] = {};
   auto run = [&](const TM *M, const double *x) {
-    const TM *m = M + v * (long)n * n + cc;  // element (row, b nc + cc) at row n + b nc
-#pragma unroll 2
-    for (int k = 0; k < nc; ++k) {
-      const TM *r0 = m + (long)k * n, *r1 = m + (long)(nc + k) * n,
-               *r2 = m + (long)(2 * nc + k) * n;
-      const double b00 = (double)r0[0], b01 = (double)r0[nc], b02 = (double)r0[2 * nc];
-      const double b11 = (double)r1[nc], b12 = (double)r1[2 * nc], b22 = (double)r2[2 * nc];
-      const double x0 = x[k], x1 = x[nc + k], x2 = x[2 * nc + k];
-      v0 += x0 * b00 + x1 * b01 + x2 * b02;
-      v1 += x0 * b01 + x1 * b11 + x2 * b12;
-      v2 += x0 * b02 + x1 * b12 + x2 * b22;
+    const TM *m = M + v * (long)n * n + min(col, lines - 1);
+    x += v * n;
+#pragma unroll 4
+    for (int k = k0; k < k1; ++k) {
+      const TM *r0 = m + (long)k * n;
+      if constexpr (SYM) {
+        const TM *r1 = r0 + (long)nc * n, *r2 = r1 + (long)nc * n;
+        const double b00 = (double)r0[0], b01 = (double)r0[nc], b02 = (double)r0[2 * nc];
+        const double b11 = (double)r1[nc], b12 = (double)r1[2 * nc], b22 = (double)r2[2 * nc];
+        const double x0 = x[k], x1 = x[nc + k], x2 = x[2 * nc + k];
+        s[0] += x0 * b00 + x1 * b01 + x2 * b02;
+        s[1] += x0 * b01 + x1 * b11 + x2 * b12;
+        s[2] += x0 * b02 + x1 * b12 + x2 * b22;
+      } else {
+        s[0] += x[k] * (double)r0[0];
+      }
     }
   };
-  if (SL) run(SL, f);
-  if (DL) run(DL, g);
-  V[v * n + cc] = v0;
-  V[v * n + nc + cc] = v1;
-  V[v * n + 2 * nc + cc] = v2;
+  if (SL) run(SL, F);
+  if (DL) run(DL, G);
+  if (wv > 0) {
+#pragma unroll
+    for (int b = 0; b < kSums; ++b) part[wv - 1][b][lane] = s[b];
+  }
+  __syncthreads();
+  if (wv > 0 || col >= lines) return;
+#pragma unroll
+  for (int b = 0; b < kSums; ++b) {
+    for (int w = 0; w < 15; ++w) s[b] += part[w][b][lane];
+    V[v * n + b * nc + col] = s[b];
+  }
 }
 
 template <typename TM>
@@ -1282,14 +1298,19 @@ int self_apply(const TM *SL, const double *F, const TM *DL, const double *G, lon
   if (!V || (SL && !F) || (DL && !G)) return VES3D_INVALID_PARAMETER;
   const int n = 3 * sh_ncoef(p);
   if (!SL && !DL) return hip_status(hipMemsetAsync(V, 0, sizeof(double) * n * Nv, st));
-  if (sym) {
-    const int nc = sh_ncoef(p), bs = 64 * (int)cdiv(std::min(nc, 512), 64);
-    dim3 g2(cdiv(nc, bs), (unsigned)Nv);
-    k_self_apply_sym<TM><<<g2, bs, 2 * n * sizeof(double), st>>>(SL, F, DL, G, nc, V);
-    return launch_status();
-  }
-  dim3 grid(cdiv(n, 256), (unsigned)Nv);
-  k_self_apply<TM><<<grid, 256, 2 * n * sizeof(double), st>>>(SL, F, DL, G, n, V);
+  const int nc = sh_ncoef(p);
+  const dim3 gs(cdiv(sym ? nc : n, 64), (unsigned)Nv);
+  // Many vesicles whose columns nearly fill blocks of 256 read longer runs with a
+  // thread per column: order 12 (504 columns), 320 / 512 vesicles in FP64 108 /
+  // 168 us against 114 / 180; 192: 86 against 66.
+  const bool wide = !sym && (long)cdiv(n, 64) * Nv >= 2560 && (long)cdiv(n, 256) * 256 - n <= n / 32;
+  if (sym)
+    k_self_apply_split<TM, true><<<gs, 1024, 0, st>>>(SL, F, DL, G, nc, V);
+  else if (!wide)
+    k_self_apply_split<TM, false><<<gs, 1024, 0, st>>>(SL, F, DL, G, nc, V);
+  else
+    k_self_apply<TM><<<dim3(cdiv(n, 256), (unsigned)Nv), 256, 2 * n * sizeof(double), st>>>(
+        SL, F, DL, G, n, V);
   return launch_status();
 }
 
