@@ -211,15 +211,13 @@ __global__ __launch_bounds__(kThreads) void k_synth(const SynthArgs<T> a) {
   }
 }
 
-// Element (lat, n) of order m's Legendre block at lat l_lat (or, if 0, the
-// block's degree count) + n l_n.
+// leg: per order m the block [latitude][degree].
 template <typename T>
 struct AnalysisArgs {
   const T *X;
   long N;
   int p0, p1;
   const T *frag, *leg;
-  int l_lat, l_n;
   T *S;
 };
 
@@ -274,8 +272,8 @@ __global__ __launch_bounds__(kThreads) void k_analysis(const AnalysisArgs<T> a) 
   __syncthreads();
   for (int c = tid; c < nc; c += kThreads) {
     const int j = J[c], m = (j + 1) / 2, n = c - block_off(p1, j);
-    const int ls = a.l_lat ? a.l_lat : p1 + 1 - m;
-    const T *__restrict__ t = a.leg + legendre_off(p1, m, L) + n * a.l_n;
+    const int ls = p1 + 1 - m;
+    const T *__restrict__ t = a.leg + legendre_off(p1, m, L) + n;
     const T *g = G + (m & 1 ? p1 : 0) + half_place(j);
     T s[FG] = {};
 #pragma unroll 8
@@ -292,7 +290,8 @@ __global__ __launch_bounds__(kThreads) void k_analysis(const AnalysisArgs<T> a) 
 
 // Operand tables, built once per (device, orders, kind): kinds 0, 1, 2 the
 // longitude derivatives of MatFourier (synthesis), 3 MatFourierInv, 4 the
-// transpose of MatFourier(p1, p0).
+// transpose of MatFourier(p1, p0); kind 5 the transposed MatLegendre(p1, p0) by
+// latitude, so that consecutive lanes (degrees) read consecutive words.
 struct FragTable {
   double *d64 = nullptr;
   float *d32 = nullptr;
@@ -307,34 +306,9 @@ const double *frag_ptr<double>(const FragTable &t) { return t.d64; }
 template <>
 const float *frag_ptr<float>(const FragTable &t) { return t.d32; }
 
+// Under g_frag_mu.
 template <typename T>
-const T *frag_table(int p0, int p1, int kind, const ShMatsHost &h) {
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return nullptr;
-  std::lock_guard<std::mutex> lk(g_frag_mu);
-  const auto key = std::make_tuple(dev, p0, p1, kind);
-  auto it = g_frags.find(key);
-  if (it != g_frags.end()) return frag_ptr<T>(it->second);
-  // element (k, col) of a half: synthesis: order place k at longitude col,
-  // analysis: longitude k of order place col
-  const int KS = up16(2 * p0) / 8, ct = up16(p1) / 16;
-  const double *M = &h.data[kind == 0   ? h.Mf
-                            : kind == 1 ? h.Mdf
-                            : kind == 2 ? h.Md2f
-                            : kind == 3 ? h.Mfinv
-                                        : h.MfT];
-  std::vector<double> f((size_t)ct * 2 * KS * 64, 0.0);
-  for (int c = 0; c < ct; ++c)
-    for (int odd = 0; odd < 2; ++odd)
-      for (int s = 0; s < KS; ++s)
-        for (int lane = 0; lane < 64; ++lane) {
-          const int k = 4 * s + lane / 16, col = 16 * c + lane % 16;
-          if (k >= p0 || col >= p1) continue;
-          f[((size_t)(c * 2 + odd) * KS + s) * 64 + lane] =
-              kind < 3    ? M[(long)half_block(odd, k) * 2 * p1 + col]
-              : kind == 3 ? M[(long)k * 2 * p1 + half_block(odd, col)]
-                          : M[(long)half_block(odd, col) * 2 * p0 + k];
-        }
+const T *frag_upload(const std::tuple<int, int, int, int> &key, const std::vector<double> &f) {
   std::vector<float> f32(f.begin(), f.end());
   FragTable t;
   if (hipMalloc(&t.d64, sizeof(double) * f.size()) != hipSuccess) return nullptr;
@@ -348,6 +322,44 @@ const T *frag_table(int p0, int p1, int kind, const ShMatsHost &h) {
     return nullptr;
   }
   return frag_ptr<T>(g_frags[key] = t);
+}
+
+template <typename T>
+const T *frag_table(int p0, int p1, int kind, const ShMatsHost &h) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return nullptr;
+  std::lock_guard<std::mutex> lk(g_frag_mu);
+  const auto key = std::make_tuple(dev, p0, p1, kind);
+  auto it = g_frags.find(key);
+  if (it != g_frags.end()) return frag_ptr<T>(it->second);
+  std::vector<double> f;
+  if (kind == 5) {
+    for (int m = 0; m <= p1; ++m)
+      for (int lat = 0; lat <= p0; ++lat)
+        for (int n = 0; n <= p1 - m; ++n) f.push_back(h.data[h.MlT[m] + (long)n * (p0 + 1) + lat]);
+    return frag_upload<T>(key, f);
+  }
+  // element (k, col) of a half: synthesis: order place k at longitude col,
+  // analysis: longitude k of order place col
+  const int KS = up16(2 * p0) / 8, ct = up16(p1) / 16;
+  const double *M = &h.data[kind == 0   ? h.Mf
+                            : kind == 1 ? h.Mdf
+                            : kind == 2 ? h.Md2f
+                            : kind == 3 ? h.Mfinv
+                                        : h.MfT];
+  f.assign((size_t)ct * 2 * KS * 64, 0.0);
+  for (int c = 0; c < ct; ++c)
+    for (int odd = 0; odd < 2; ++odd)
+      for (int s = 0; s < KS; ++s)
+        for (int lane = 0; lane < 64; ++lane) {
+          const int k = 4 * s + lane / 16, col = 16 * c + lane % 16;
+          if (k >= p0 || col >= p1) continue;
+          f[((size_t)(c * 2 + odd) * KS + s) * 64 + lane] =
+              kind < 3    ? M[(long)half_block(odd, k) * 2 * p1 + col]
+              : kind == 3 ? M[(long)k * 2 * p1 + half_block(odd, col)]
+                          : M[(long)half_block(odd, col) * 2 * p0 + k];
+        }
+  return frag_upload<T>(key, f);
 }
 
 // Functions per workgroup: as many as share the tables without leaving CUs
@@ -429,15 +441,20 @@ bool analysis_fused(const T *X, long N, int p0, int p1, bool transpose, const Sh
   if (sizeof(T) == 8 && p0 > 24 && p1 > 24 &&
       N >= (analysis_lds(p0, p1, 2, sizeof(T)) > kLdsMost ? 1280 : 5120))
     return false;
+  // Where the order falls to half, a group's few results per function leave the
+  // GEMMs ahead once they fill the chip.  N = 12288 / 60000, FP64: orders 12 -> 6
+  // 23 / 95 and 23 / 70 us, 32 -> 16 103 / 568 and 104 / 504; FP32: 12 -> 6 14 / 60
+  // and 16 / 46 us, but 24 -> 12 31 / 149 and 38 / 166.
+  if (2 * p1 <= p0 && N >= 16384 && (sizeof(T) == 8 || p0 <= 16)) return false;
   const int fg = functions_per_group(N, 1, analysis_lds, p0, p1, sizeof(T));
   if (fg == 0) return false;
   const T *frag = frag_table<T>(p0, p1, transpose ? 4 : 3, h);
-  if (!frag) {
+  const T *leg = transpose ? frag_table<T>(p0, p1, 5, h) : mats + h.Mlinv[0];
+  if (!frag || !leg) {
     *status = VES3D_MEMORY_ERROR;
     return true;
   }
-  const AnalysisArgs<T> a{X, N, p0, p1, frag, mats + (transpose ? h.MlT[0] : h.Mlinv[0]),
-                          transpose ? 1 : 0, transpose ? p0 + 1 : 1, S};
+  const AnalysisArgs<T> a{X, N, p0, p1, frag, leg, S};
   *status = launch_groups<T>(a, fg, 1, st);
   return true;
 }
