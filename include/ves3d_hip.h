@@ -135,8 +135,10 @@ int ves3d_hip_set_gemm_kernel(int kind);
 /* Output tile of the MFMA grouped GEMM: -1 (the default) picks per
  * descriptor list the shape that minimises padded work plus operand
  * traffic; 0..8 force one of the shapes (rows x columns) 64x64, 64x16,
- * 128x16, 256x16, 64x32, 128x32, 64x48, 128x48, 128x64.  For tests and
- * tuning; no counterpart in the reference. */
+ * 128x16, 256x16, 64x32, 128x32, 64x48, 128x48, 128x64.  A forced shape (or
+ * the VALU kernel above) also takes every spherical-harmonic transform
+ * through the grouped GEMMs, where most otherwise run as one kernel.  For
+ * tests and tuning; no counterpart in the reference. */
 int ves3d_hip_set_gemm_tile(int tile);
 
 /* The sustained VALU rate of this GPU: lane fused multiply-adds per second
