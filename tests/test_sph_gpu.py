@@ -62,7 +62,8 @@ def test_grid2shc_and_transpose(hip, p0, p1, N, dt, tol):
 @pytest.mark.parametrize("p0,p1,N", [(1, 1, 1), (2, 5, 3), (8, 8, 4), (9, 17, 1027), (16, 32, 683),
                                      (17, 3, 130), (24, 25, 1), (25, 24, 513), (32, 33, 2),
                                      (32, 32, 1365), (33, 12, 3), (12, 6, 16383),
-                                     (12, 6, 16384)])
+                                     (12, 6, 16384), (6, 11, 6143), (6, 11, 6144), (6, 12, 12287),
+                                     (6, 12, 12288)])
 @pytest.mark.parametrize("dt,tol", [(torch.float64, 1e-12), (torch.float32, 1e-5)])
 def test_one_kernel_transforms(hip, p0, p1, N, dt, tol):
     """The one-kernel transforms against the grouped GEMMs (which a forced tile

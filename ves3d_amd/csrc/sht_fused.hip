@@ -408,6 +408,12 @@ template <typename T>
 bool synth_fused(const T *S, long N, int p0, int p1, int nvar, const ShMatsHost &h, const T *mats,
                  const int *dleg, const int *dfour, T *const *X, T alpha, hipStream_t st,
                  int *status) {
+  // For many functions on small grids the GEMMs, which form the Legendre sums of
+  // variants without a latitude derivative once, are faster.  FP64, three variants
+  // here / there in us: orders 6 -> 6, N = 3072 / 8192: 18, 41 / 21, 29; 12 -> 12,
+  // N = 8192 / 16384: 59, 120 / 61, 90; 10 -> 20: 81, 154 / 92, 144; but 14 -> 28,
+  // N = 16384 / 70000: 194, 1200 / 290, 1184, and 16 -> 32: 295, 1401 / 365, 1483.
+  if (p1 < 28 && N >= (p1 < 12 ? 6144 : 12288)) return false;
   const int fg = functions_per_group(N, nvar, synth_lds, p0, p1, sizeof(T));
   if (fg == 0) return false;
   SynthArgs<T> a{};

@@ -350,7 +350,8 @@ __device__ __forceinline__ double rsqrt_refined(double x) {
 // of the values at the four mirror points (lat or P1 - lat, lon or lon + pi)
 // serve one parity of m and of n - m each, with a quarter of the products.
 // Persistent workgroups walk the rotations r = blockIdx.x + i gridDim.x and,
-// within a rotation, the latitude pairs (lat, P1 - lat):
+// within a rotation, the latitude pairs (lat, P1 - lat), two per pass up to P1 =
+// 16 (331 vesicles of order 7, single layer, the whole build: 982 -> 901 us):
 //   1. four lanes evaluate pole t's 6 kernel values at the four mirror points
 //      of (lat, lon < P1), form the four combinations by lane swaps and store
 //      them in Kv[n - m parity][m parity][lon][t * 6 + q] (kPtKs doubles per
@@ -385,6 +386,9 @@ __device__ __forceinline__ double rsqrt_refined(double x) {
 constexpr int kPtKs = 13;
 constexpr int kPtPad = 4;
 constexpr int kPtThreads = 256;
+// Latitude pairs per pass: half a circle of at most 16 longitudes leaves half the
+// lanes of one pair's waves without a point.
+__host__ __device__ constexpr int pole_pairs(int p1) { return p1 <= 16 ? 2 : 1; }
 // Doubles of one mirror combination's values.
 __host__ __device__ constexpr int pole_kv_part(int p1) { return p1 * kPtKs + kPtPad; }
 // Degree l's rotation block in operand order: 4 loads of 64 doubles (one tile
@@ -413,7 +417,7 @@ inline int pole_legendre_threads(int p0) {
 
 // LDS doubles of k_pole_transpose: Kv and T, which the rotation's rows share.
 __host__ __device__ inline long pole_lds_doubles(int p0, int p1) {
-  const int kt = 2 * (4 * pole_kv_part(p1) + 2 * 12 * p1), st = 12 * (p0 * (p0 + 2) + 1);
+  const int kt = 2 * pole_pairs(p1) * (4 * pole_kv_part(p1) + 2 * 12 * p1), st = 12 * (p0 * (p0 + 2) + 1);
   return kt > st ? kt : st;
 }
 
@@ -449,12 +453,12 @@ __global__ __launch_bounds__(kPtThreads, 3) void k_pole_transpose(
   typedef double v4d __attribute__((ext_vector_type(4)));
   static_assert(P1 % 2 == 0 && 8 * P1 <= kPtThreads);
   constexpr int L = 2 * P1, Nlat = P1 + 1, NP = P1 / 2 + 1, M1 = L * Nlat, KS = (P1 + 3) / 4;
-  constexpr int kPart = pole_kv_part(P1);
+  constexpr int kPart = pole_kv_part(P1), PP = pole_pairs(P1), NS = (NP + PP - 1) / PP;
   extern __shared__ double lds[];
   const int F = 2 * p0, Nc = p0 * (p0 + 2);
   const int ntri = pole_triples(p0, p0 + 1);
-  double *Kv = lds;                                // [buffer][2][2][P1][kPtKs]
-  double *Ts = Kv + 8 * kPart;                     // [buffer][2][12][P1]
+  double *Kv = lds;                                // [buffer][pair][2][2][P1][kPtKs]
+  double *Ts = Kv + 8 * PP * kPart;                // [buffer][pair][2][12][P1]
   double *St = lds;                                // [12][Nc + 1], over Kv and Ts
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   // kernel-value role: pole t (the wave's) at longitude j + half P1 of the
@@ -465,7 +469,8 @@ __global__ __launch_bounds__(kPtThreads, 3) void k_pole_transpose(
   const int uwv = __builtin_amdgcn_readfirstlane(wv);
   const int row = (tid >> 4) & 1, half = (tid >> 5) & 1;
   const int t = (uwv / kBlocks) & 1, j = 16 * (uwv % kBlocks) + (tid & 15);
-  const bool kvt = uwv < 2 * kBlocks && j < P1;
+  const int pr = PP == 2 ? uwv >> 1 : 0;  // the pass's pair
+  const bool kvt = j < P1;
   // Fourier role: the columns of order parity tile from the row combination frow
   const int frow = wv >> 1, tile = wv & 1;
   const int li = lane & 15, lk = lane >> 4;
@@ -508,7 +513,7 @@ __global__ __launch_bounds__(kPtThreads, 3) void k_pole_transpose(
   // every thread at indices in range: unconditional loads leave no value to
   // merge after a branch, so nothing waits for them before their use.  The
   // rotation's base is uniform, the place in it 32 bits.
-  double g[9], tg[3], w, ml[3];
+  double g[9], tg[3], w, ml[PP][3];
   const unsigned place = 8 * ((row ? P1 * L : 0) + half * P1 + min(j, P1 - 1)),
                  wplace = 8 * (2 * row + t);
   const int step = row ? -8 * L : 8 * L;
@@ -521,12 +526,14 @@ __global__ __launch_bounds__(kPtThreads, 3) void k_pole_transpose(
   };
   auto load = [&](long r_, int g_) {
     const long rc = r_ < nrot ? r_ : nrot - 1;
-    const unsigned o = place + g_ * step;
+    const int lp = min(g_ * PP + pr, NP - 1);
+    const unsigned o = place + lp * step;
     const double *x = X + rc * 3 * M1, *xt = Xt + rc * 3 * M1, *xp = Xp + rc * 3 * M1;
     g[0] = at(x, o); g[1] = at(x + M1, o); g[2] = at(x + 2 * M1, o);
     g[3] = at(xt, o); g[4] = at(xt + M1, o); g[5] = at(xt + 2 * M1, o);
     g[6] = at(xp, o); g[7] = at(xp + M1, o); g[8] = at(xp + 2 * M1, o);
-    w = at(qw + 4 * g_, wplace);
+    w = at(qw + 4 * lp, wplace);
+    if (PP > 1 && g_ * PP + pr >= NP) w = 0.0;  // past the last pair
   };
   auto load_pole = [&](long r_) {
     const long rc = r_ < nrot ? r_ : nrot - 1;
@@ -534,32 +541,40 @@ __global__ __launch_bounds__(kPtThreads, 3) void k_pole_transpose(
   };
   const unsigned mplace = 8 * tm;
   auto load_ml = [&](int g_) {
-    for (int n = 0; n < 3; ++n) ml[n] = at(mlt + (g_ * 3 + n) * ntri, mplace);
+#pragma unroll
+    for (int u = 0; u < PP; ++u)
+      for (int n = 0; n < 3; ++n)
+        ml[u][n] = at(mlt + (min(g_ * PP + u, NP - 1) * 3 + n) * ntri, mplace);
   };
   load(blockIdx.x, 0);
   load_pole(blockIdx.x);
   for (long r = blockIdx.x; r < nrot; r += gridDim.x) {
     double acc[6][3] = {};
-    double f[6];
+    double f[PP][6];
     auto load_t = [&](int g_) {
-      const double *tc = Ts + ((g_ & 1) * 24 + par * 12 + c) * P1 + jj;
 #pragma unroll
-      for (int i = 0; i < 6; ++i) f[i] = tc[i * P1];
+      for (int u = 0; u < PP; ++u) {
+        const double *tc = Ts + (((g_ & 1) * PP + u) * 24 + par * 12 + c) * P1 + jj;
+#pragma unroll
+        for (int i = 0; i < 6; ++i) f[u][i] = tc[i * P1];
+      }
     };
     auto legendre = [&] {
 #pragma unroll
-      for (int i = 0; i < 6; ++i)
+      for (int u = 0; u < PP; ++u)
 #pragma unroll
-        for (int n = 0; n < 3; ++n) acc[i][n] = fma(f[i], ml[n], acc[i][n]);
+        for (int i = 0; i < 6; ++i)
+#pragma unroll
+          for (int n = 0; n < 3; ++n) acc[i][n] = fma(f[u][i], ml[u][n], acc[i][n]);
     };
 #pragma unroll 1
-    for (int gi = 0; gi < NP; ++gi) {
+    for (int gi = 0; gi < NS; ++gi) {
       {
         const double yt = g[4], zt = g[5], xt = g[3], xp = g[6], yp = g[7], zp = g[8];
         const double nx = yt * zp - zt * yp, ny = zt * xp - xt * zp, nz = xt * yp - yt * xp;
         const double dx = tg[0] - g[0], dy = tg[1] - g[1], dz = tg[2] - g[2];
         const double wt = w;
-        const bool more = gi + 1 < NP;
+        const bool more = gi + 1 < NS;
         load(more ? r : r + gridDim.x, more ? gi + 1 : 0);
         const double r2 = dx * dx + dy * dy + dz * dz;
         const double rinv = r2 <= eps ? 0.0 : rsqrt_refined(r2);
@@ -587,7 +602,7 @@ __global__ __launch_bounds__(kPtThreads, 3) void k_pole_transpose(
           mirror_sums<32>(v[2 * q], v[2 * q + 1]);
         }
         if (kvt) {
-          double *kv = Kv + ((gi & 1) * 4 + 2 * half) * kPart + j * kPtKs + t * 6 + row;
+          double *kv = Kv + (((gi & 1) * PP + pr) * 4 + 2 * half) * kPart + j * kPtKs + t * 6 + row;
 #pragma unroll
           for (int q = 0; q < 3; ++q) {
             kv[2 * q] = v[2 * q];
@@ -598,31 +613,37 @@ __global__ __launch_bounds__(kPtThreads, 3) void k_pole_transpose(
       __syncthreads();  // Kv and the previous pass's T are in
       {
         // (the rows c >= 12 of A are other values; what they give is not read)
-        const double *kv = Kv + ((gi & 1) * 4 + wv) * kPart + li;
-        v4d d = {0.0, 0.0, 0.0, 0.0}, e = {0.0, 0.0, 0.0, 0.0};
-        double a[KS];
+        const double *kv = Kv + ((gi & 1) * PP * 4 + wv) * kPart + li;
+        v4d d[2] = {};  // two accumulation chains: the pairs', or the steps' halves
+        double a[PP][KS];
 #pragma unroll
-        for (int s = 0; s < KS; ++s) a[s] = kv[min(4 * s + lk, P1 - 1) * kPtKs];
+        for (int u = 0; u < PP; ++u)
+#pragma unroll
+          for (int s = 0; s < KS; ++s)
+            a[u][s] = kv[u * 4 * kPart + min(4 * s + lk, P1 - 1) * kPtKs];
         if (gi > 0) load_t(gi - 1);
 #pragma unroll
-        for (int s = 0; s < KS; ++s) {  // two accumulation chains
-          if (s & 1)
-            e = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s], mf[s], e, 0, 0, 0);
-          else
-            d = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s], mf[s], d, 0, 0, 0);
-        }
+        for (int s = 0; s < KS; ++s)
+#pragma unroll
+          for (int u = 0; u < PP; ++u) {
+            v4d &e = d[PP == 2 ? u : s & 1];
+            e = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u][s], mf[s], e, 0, 0, 0);
+          }
         if (gi > 0) legendre();
         load_ml(gi);
-        d += e;
+        if (PP == 1) d[0] += d[1];
         if (fcol >= 0) {
-          double *o = Ts + ((gi & 1) * 24 + frow * 12 + lk) * P1 + fcol;
 #pragma unroll
-          for (int i = 0; i < 3; ++i) o[4 * i * P1] = d[i];
+          for (int u = 0; u < PP; ++u) {
+            double *o = Ts + (((gi & 1) * PP + u) * 24 + frow * 12 + lk) * P1 + fcol;
+#pragma unroll
+            for (int i = 0; i < 3; ++i) o[4 * i * P1] = d[u][i];
+          }
         }
       }
     }
     __syncthreads();  // the last T is in
-    load_t(NP - 1);
+    load_t(NS - 1);
     legendre();
     // the rotation's 12 rows, degree-major.  (The thread's index is opaque from
     // here on: what is derived from it is not kept in registers over the passes.)
