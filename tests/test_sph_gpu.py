@@ -183,6 +183,26 @@ def test_singular_closed_forms_gpu(hip, p0):
         assert np.max(np.abs(Vn)) < 1e-9
 
 
+@pytest.mark.parametrize("p0,p1,nv", [(6, 12, 5), (8, 16, 3), (12, 24, 2), (16, 32, 2), (24, 48, 1)])
+def test_singular_build_f32_transforms(hip, p0, p1, nv):
+    """The FP32 build's transforms are the grouped GEMMs (which a forced tile
+    selects), whose sums do not depend on the tile: the same bits."""
+    from ves3d_amd import call
+    X = cu(_singular_case(nv, p0, seed=p0))
+    n = 3 * p0 * (p0 + 2)
+    out = {}
+    try:
+        for tile in (-1, 0):
+            call("ves3d_hip_set_gemm_tile", tile)
+            out[tile] = [torch.zeros((nv, n, n), device="cuda") for _ in range(2)]
+            G.singular_build(X, nv, p0, p1, *out[tile])
+            torch.cuda.synchronize()
+    finally:
+        call("ves3d_hip_set_gemm_tile", -1)
+    for a, b in zip(out[-1], out[0]):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("p0,sl_tol", [(16, 5e-8), (24, 1e-8)])
 def test_singular_identities_on_ellipsoids_gpu(hip, p0, sl_tol):
     """Shape-sensitive identities at the workloads' orders, on two rotated

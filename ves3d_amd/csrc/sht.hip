@@ -226,7 +226,7 @@ int sht_synth_multi(const T *S, long N, int p0, int p1, int nvar, const int *dle
 
 template <typename T>
 int sht_shc2grid(const T *S, long N, int p0, int p1, T *X, T *Xt, T *Xp, T *work,
-                 hipStream_t st) {
+                 hipStream_t st, ShtForm form) {
   if (!valid_order(p0) || !valid_order(p1) || N < 0) return VES3D_INVALID_PARAMETER;
   if (N == 0) return VES3D_SUCCESS;
   const ShMatsDev *m = sh_mats(p0, p1);
@@ -241,7 +241,8 @@ int sht_shc2grid(const T *S, long N, int p0, int p1, T *X, T *Xt, T *Xp, T *work
     dleg[n] = 1;
     out[n++] = Xp;
   }
-  if (synth_fused<T>(S, N, p0, p1, n, *m->h, mats_ptr<T>(m), dleg, dfour, out, T(1), st, &status))
+  if (form == ShtForm::kAuto &&
+      synth_fused<T>(S, N, p0, p1, n, *m->h, mats_ptr<T>(m), dleg, dfour, out, T(1), st, &status))
     return status;
   V3D_CHECK(run<T>(kS2GLeg, p0, p1, N, m, S, work, st));
   V3D_CHECK(run<T>(kS2GFour, p0, p1, N, m, work, X, st));
@@ -272,13 +273,15 @@ int sht_synth(const T *S, long N, int p0, int p1, int dleg, int dfour, T *X, T *
 }
 
 template <typename T>
-int sht_grid2shc(const T *X, long N, int p0, int p1, T *S, T *work, hipStream_t st) {
+int sht_grid2shc(const T *X, long N, int p0, int p1, T *S, T *work, hipStream_t st,
+                 ShtForm form) {
   if (!valid_order(p0) || !valid_order(p1) || N < 0) return VES3D_INVALID_PARAMETER;
   if (N == 0) return VES3D_SUCCESS;
   const ShMatsDev *m = sh_mats(p0, p1);
   if (!m) return VES3D_MEMORY_ERROR;
   int status;
-  if (analysis_fused<T>(X, N, p0, p1, false, *m->h, mats_ptr<T>(m), S, st, &status))
+  if (form == ShtForm::kAuto &&
+      analysis_fused<T>(X, N, p0, p1, false, *m->h, mats_ptr<T>(m), S, st, &status))
     return status;
   V3D_CHECK(run<T>(kG2SFour, p0, p1, N, m, X, work, st));
   return run<T>(kG2SLeg, p0, p1, N, m, work, S, st);
@@ -286,13 +289,14 @@ int sht_grid2shc(const T *X, long N, int p0, int p1, T *S, T *work, hipStream_t 
 
 template <typename T>
 int sht_shc2grid_transpose(const T *X, long N, int p0, int p1, T *S, T *work,
-                           hipStream_t st) {
+                           hipStream_t st, ShtForm form) {
   if (!valid_order(p0) || !valid_order(p1) || N < 0) return VES3D_INVALID_PARAMETER;
   if (N == 0) return VES3D_SUCCESS;
   const ShMatsDev *m = sh_mats(p0, p1);
   if (!m) return VES3D_MEMORY_ERROR;
   int status;
-  if (analysis_fused<T>(X, N, p0, p1, true, *m->h, mats_ptr<T>(m), S, st, &status))
+  if (form == ShtForm::kAuto &&
+      analysis_fused<T>(X, N, p0, p1, true, *m->h, mats_ptr<T>(m), S, st, &status))
     return status;
   V3D_CHECK(run<T>(kTFour, p0, p1, N, m, X, work, st));
   return run<T>(kTLeg, p0, p1, N, m, work, S, st);
@@ -356,10 +360,12 @@ int sht_shc2pole(const T *S, long N, int p0, T *P, hipStream_t st) {
 }
 
 #define V3D_INST(T)                                                                       \
-  template int sht_shc2grid<T>(const T *, long, int, int, T *, T *, T *, T *, hipStream_t); \
-  template int sht_grid2shc<T>(const T *, long, int, int, T *, T *, hipStream_t);          \
-  template int sht_shc2grid_transpose<T>(const T *, long, int, int, T *, T *, hipStream_t); \
-  template int sht_shc2pole<T>(const T *, long, int, T *, hipStream_t);                 \
+  template int sht_shc2grid<T>(const T *, long, int, int, T *, T *, T *, T *, hipStream_t, \
+                               ShtForm);                                                   \
+  template int sht_grid2shc<T>(const T *, long, int, int, T *, T *, hipStream_t, ShtForm); \
+  template int sht_shc2grid_transpose<T>(const T *, long, int, int, T *, T *, hipStream_t, \
+                                         ShtForm);                                         \
+  template int sht_shc2pole<T>(const T *, long, int, T *, hipStream_t);                    \
   template int sht_synth<T>(const T *, long, int, int, int, int, T *, T *, hipStream_t, T); \
   template int sht_synth_multi<T>(const T *, long, int, int, int, const int *, const int *,    \
                                   const int *, T *, long, T *, hipStream_t);                   \

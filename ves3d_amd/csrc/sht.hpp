@@ -17,17 +17,22 @@ inline long shc2grid_multi_work(long N, int p0, int p1, int nvar) {
   return nvar * shc2grid_work(N, p0, p1);
 }
 
+// How a transform runs: in one kernel where that is the faster form, or always
+// as grouped GEMMs (the sums in their order).
+enum class ShtForm { kAuto, kGrouped };
+
 // S [N][p0(p0+2)] -> X [N][(p1+1)2p1]; X_theta / X_phi optional (may be null).
 template <typename T>
 int sht_shc2grid(const T *S, long N, int p0, int p1, T *X, T *X_theta, T *X_phi,
-                 T *work, hipStream_t st);
+                 T *work, hipStream_t st, ShtForm form = ShtForm::kAuto);
 // X [N][(p0+1)2p0] -> S [N][p1(p1+2)].
 template <typename T>
-int sht_grid2shc(const T *X, long N, int p0, int p1, T *S, T *work, hipStream_t st);
+int sht_grid2shc(const T *X, long N, int p0, int p1, T *S, T *work, hipStream_t st,
+                 ShtForm form = ShtForm::kAuto);
 // Adjoint of SHC2Grid(p1 -> p0): X [N][(p0+1)2p0] -> S [N][p1(p1+2)].
 template <typename T>
 int sht_shc2grid_transpose(const T *X, long N, int p0, int p1, T *S, T *work,
-                           hipStream_t st);
+                           hipStream_t st, ShtForm form = ShtForm::kAuto);
 // Synthesis with the latitude (Legendre) stage differentiated dleg times and
 // the longitude (Fourier) stage dfour times, dleg, dfour in {0,1,2}; the
 // Legendre stage is scaled by alpha.  Same workspace as sht_shc2grid.

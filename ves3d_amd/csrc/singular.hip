@@ -1113,6 +1113,14 @@ int singular_build(const double *X0, long Nv, int p0, int p1, T *SL, T *DL, hipS
                            ? pole_fused_shape(p0, p1)
                            : PoleShape();
   const bool fused = ps.kern != nullptr;
+  // The FP32 form's transforms stay grouped GEMMs: the pole kernel subtracts
+  // FP32 positions and raises the difference to r^-5, so that another order of
+  // their sums moves the operators by far more than it rounds (2.7e-4 between
+  // the two at order 24, 40 vesicles), and the one-kernel forms' came out
+  // further from 64 bits (8.9e-6 -> 1.1e-5 there).  The price: one-kernel
+  // transforms took 0.7 of the time for a few vesicles (order 16, two: 196 ->
+  // 148 us), 0.94 for 30 at order 24, 1.1 for 300 at order 10.
+  const ShtForm form = std::is_same<T, float>::value ? ShtForm::kGrouped : ShtForm::kAuto;
   const long per = singular_elems_per_ves(p0, p1, fused);
   const long budget = (6L << 30) / (long)sizeof(T);
   long chunk = std::max(1L, std::min(Nv, budget / per));
@@ -1148,9 +1156,9 @@ int singular_build(const double *X0, long Nv, int p0, int p1, T *SL, T *DL, hipS
     const long nx0 = cv * 3 * Ng;
     k_copy_cast_grid<T><<<grid_for(nx0), 256, 0, st>>>(X0 + v0 * 3 * Ng, nx0, x0);
     V3D_CHECK(launch_status());
-    V3D_CHECK(sht_grid2shc<T>(x0, cv * 3, p0, p0, S0, w, st));
+    V3D_CHECK(sht_grid2shc<T>(x0, cv * 3, p0, p0, S0, w, st, form));
     V3D_CHECK(rotate_all<T>(S0, cv, p0, 3, S, w, st));
-    V3D_CHECK(sht_shc2grid<T>(S, rot * 3, p0, p1, X, Xt, Xp, w, st));
+    V3D_CHECK(sht_shc2grid<T>(S, rot * 3, p0, p1, X, Xt, Xp, w, st, form));
     V3D_CHECK(sht_shc2pole<T>(S, rot * 3, p0, P, st));
     for (int layer = 0; layer < 2; ++layer) {
       T *dst = layer == 0 ? SL : DL;
@@ -1178,7 +1186,7 @@ int singular_build(const double *X0, long Nv, int p0, int p1, T *SL, T *DL, hipS
         k_pole_kernel<T><<<grid_for(rot * M1), 256, 0, st>>>(
             X, Xt, Xp, P, qw, rot, p1, layer == 0 ? K0 : nullptr, layer == 1 ? K0 : nullptr);
         V3D_CHECK(launch_status());
-        V3D_CHECK(sht_shc2grid_transpose<T>(K0, rot * 12, p1, p0, K1, w, st));
+        V3D_CHECK(sht_shc2grid_transpose<T>(K0, rot * 12, p1, p0, K1, w, st, form));
         V3D_CHECK(rotate_transpose<T>(K1, cv, p0, 12, K2, w, st));
       }
       if constexpr (std::is_same<T, double>::value) {
@@ -1198,7 +1206,7 @@ int singular_build(const double *X0, long Nv, int p0, int p1, T *SL, T *DL, hipS
       if (ra_blocks > 0x7fffffffL) return VES3D_INVALID_PARAMETER;
       k_singular_rearrange<T><<<(unsigned)ra_blocks, 256, 0, st>>>(K2, cv, p0, M1a);
       V3D_CHECK(launch_status());
-      V3D_CHECK(sht_grid2shc<T>(M1a, cv * 9 * Nc, p0, p0, dst + v0 * 9 * Nc * Nc, w, st));
+      V3D_CHECK(sht_grid2shc<T>(M1a, cv * 9 * Nc, p0, p0, dst + v0 * 9 * Nc * Nc, w, st, form));
     }
   }
   return hip_status(hipEventRecord(done, st));
