@@ -362,6 +362,15 @@ const T *frag_table(int p0, int p1, int kind, const ShMatsHost &h) {
   return frag_upload<T>(key, f);
 }
 
+// Whether n values at a and k values at b share memory.  A workgroup writes its
+// functions over others that no workgroup has read yet; the GEMMs read all of
+// their input into the work buffer before they write.
+template <typename T>
+bool overlap(const T *a, long n, const T *b, long k) {
+  const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
+  return x < y + sizeof(T) * k && y < x + sizeof(T) * n;
+}
+
 // Functions per workgroup: as many as share the tables without leaving CUs
 // idle (0: the GEMMs run).
 int functions_per_group(long N, int nvar, size_t (*lds)(int, int, int, size_t), int p0, int p1,
@@ -416,6 +425,8 @@ bool synth_fused(const T *S, long N, int p0, int p1, int nvar, const ShMatsHost 
   if (p1 < 28 && N >= (p1 < 12 ? 6144 : 12288)) return false;
   const int fg = functions_per_group(N, nvar, synth_lds, p0, p1, sizeof(T));
   if (fg == 0) return false;
+  for (int v = 0; v < nvar; ++v)
+    if (overlap(S, N * sh_ncoef(p0), X[v], N * sh_ngrid(p1))) return false;
   SynthArgs<T> a{};
   a.S = S;
   a.N = N;
@@ -453,7 +464,7 @@ bool analysis_fused(const T *X, long N, int p0, int p1, bool transpose, const Sh
   // and 16 / 46 us, but 24 -> 12 31 / 149 and 38 / 166.
   if (2 * p1 <= p0 && N >= 16384 && (sizeof(T) == 8 || p0 <= 16)) return false;
   const int fg = functions_per_group(N, 1, analysis_lds, p0, p1, sizeof(T));
-  if (fg == 0) return false;
+  if (fg == 0 || overlap(X, N * sh_ngrid(p0), S, N * sh_ncoef(p1))) return false;
   const T *frag = frag_table<T>(p0, p1, transpose ? 4 : 3, h);
   const T *leg = transpose ? frag_table<T>(p0, p1, 5, h) : mats + h.Mlinv[0];
   if (!frag || !leg) {
