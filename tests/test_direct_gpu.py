@@ -229,6 +229,35 @@ def test_direct_eval_split_edges(hip, orc, sl, dl, ns, nt, spg):
         assert _relerr(got[pick], ref[pick]) < tol, (mixed, _relerr(got[pick], ref[pick]))
 
 
+@pytest.mark.parametrize("mixed", [False, True])
+@pytest.mark.parametrize("sl,dl", [(True, False), (False, True), (True, True)])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), 1e300])
+def test_direct_eval_own_group_not_read(hip, sl, dl, mixed, bad):
+    """A target's own group is no part of its sum, whatever its densities and
+    positions hold, in waves that one group fills and in waves that span
+    groups: group k's targets get the same bits with any values in group k."""
+    rng = np.random.default_rng(3)
+    groups, spg, tpg = 5, 84, 90
+    pos = _cuda(rng.uniform(-1, 1, (groups, spg, 3)) + 4.0 * np.arange(groups)[:, None, None])
+    trg = _cuda(rng.uniform(-1, 1, (groups, tpg, 3)) + 4.0 * np.arange(groups)[:, None, None])
+    f, q = _cuda(rng.uniform(-1, 1, (groups, spg, 3))), _cuda(rng.uniform(-1, 1, (groups, spg, 6)))
+
+    def run(x, a, b):
+        out = torch.full((groups, tpg, 3), 7.0, dtype=torch.float64, device="cuda")
+        K.direct_eval(x, a if sl else None, b if dl else None, trg, out, spg, tpg, mixed=mixed)
+        return out
+
+    ref = run(pos, f, q)
+    assert bool(torch.isfinite(ref).all())
+    for k in range(groups):
+        for what in range(3):
+            args = [pos.clone(), f.clone(), q.clone()]
+            args[what][k, spg // 2] = bad
+            if what == 0 and mixed:
+                args[0][k, spg // 2, 0] = float("nan")
+            assert torch.equal(run(*args)[k], ref[k]), (k, what)
+
+
 def test_full_size_far_field_properties(hip, orc):
     """512 vesicles at p=16 (278,528 points): f32c vs f64 on every target,
     and f64 vs the oracle on a sample of 96 targets."""

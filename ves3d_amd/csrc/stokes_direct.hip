@@ -55,7 +55,10 @@ __device__ __forceinline__ float rsqrt_pair(float x) { return __frsqrt_rn(x); }
 // The r^2 bias that removes a target's own group from a sum without making
 // control flow divergent.  FP32: 1/sqrt(inf) = 0 and every term is an exact
 // zero.  FP64: infinity would turn the refinement step into a NaN; with 1e200
-// an own-group source adds 1e-100 |f|, nothing at 53 bits.
+// an own-group source adds 1e-100 |f|, nothing at 53 bits.  Both hold for finite
+// densities; the public sums (k_pairs_*), whose groups may hold anything, also
+// take a lane's sums from before its own group, and the bias keeps its
+// coincident points from repeating runs.
 constexpr double kOwnGroupBias64 = 1e200;
 constexpr float kOwnGroupBias = __builtin_inff();
 
@@ -179,10 +182,11 @@ __device__ __forceinline__ unsigned order_key(float x) { return __float_as_uint(
 constexpr int FF_RUN = 32;
 
 // n consecutive FP64 sources (positions p, densities f, (g, n) at q) at one
-// target, U at a time.
+// target, U at a time.  A lane with a bias keeps its sums (spans: the wave may
+// have such lanes).
 template <int U, bool SL, bool DL, bool GUARD>
-__device__ __forceinline__ void add_sources64(double tx, double ty, double tz, double bias, int n,
-                                              const double *__restrict__ p,
+__device__ __forceinline__ void add_sources64(double tx, double ty, double tz, double bias,
+                                              bool spans, int n, const double *__restrict__ p,
                                               const double *__restrict__ f,
                                               const double *__restrict__ q, double k, double eps2,
                                               double (&S)[3]) {
@@ -223,6 +227,10 @@ __device__ __forceinline__ void add_sources64(double tx, double ty, double tz, d
       for (int c = 0; c < 3; ++c) S[c] = S0[c];
 #pragma unroll 1
       for (i = i0; i < i1; ++i) block(i, One(), true);
+    }
+    if (spans) {
+#pragma unroll
+      for (int c = 0; c < 3; ++c) S[c] = bias != 0.0 ? S0[c] : S[c];
     }
   }
 }
@@ -324,6 +332,7 @@ __global__ __launch_bounds__(FF_BLOCK) void k_pairs_f64(
   const double tx = tpos[3 * w.tc], ty = tpos[3 * w.tc + 1], tz = tpos[3 * w.tc + 2];
   double S[3] = {0, 0, 0};
   Slice k = slice_of(map, slice);
+  const bool spans = tpg > 0 && w.own < 0;
   constexpr int U = DL ? 2 : 4;
   while (k.u < k.u1) {
     // the slice's parts of group k.g, in one run
@@ -335,8 +344,8 @@ __global__ __launch_bounds__(FF_BLOCK) void k_pairs_f64(
       const double *__restrict__ f = SL ? sld + 3 * s0 : p;
       const double *__restrict__ q = DL ? dld + 6 * s0 : p;
       for (long i = 0; i < n; i += 1 << 24)
-        add_sources64<U, SL, DL, GUARD>(tx, ty, tz, bias, (int)min(n - i, 1L << 24), p + 3 * i,
-                                        f + 3 * i, q + 6 * i, ratio, eps2, S);
+        add_sources64<U, SL, DL, GUARD>(tx, ty, tz, bias, spans, (int)min(n - i, 1L << 24),
+                                        p + 3 * i, f + 3 * i, q + 6 * i, ratio, eps2, S);
     }
     k.u += take;
     k.j = 0;
@@ -412,7 +421,8 @@ __global__ __launch_bounds__(FF_BLOCK, DL ? 8 : (GUARD ? 6 : 7)) void k_pairs_f3
       const long c0 = g * spg + (long)tile * FF_TILE;
       const int cnt = (int)min((long)FF_TILE, spg - (long)tile * FF_TILE);
       const int r0 = (int)k.j * plen, r1 = min(cnt, r0 + (int)take * plen);
-      const float bias = w.group == g ? kOwnGroupBias : 0.0f;
+      const bool mine = w.group == g;
+      const float bias = mine ? kOwnGroupBias : 0.0f;
       const double *a = spos + 3 * c0;
       const float lx = (float)(tx - a[0]), ly = (float)(ty - a[1]), lz = (float)(tz - a[2]);
       for (int i0 = r0; i0 < r1; i0 += FF_SUB) {
@@ -442,6 +452,8 @@ __global__ __launch_bounds__(FF_BLOCK, DL ? 8 : (GUARD ? 6 : 7)) void k_pairs_f3
             }
           }
         }
+#pragma unroll
+        for (int c = 0; c < 3; ++c) S[c] = mine ? 0.0f : S[c];
         acc_merge(A, S);
       }
     }
