@@ -333,6 +333,27 @@ def test_self_apply_rows_split(hip, p, nv, dt):
         assert bool(((V - ref).abs() <= 2 * n * 2.3e-16 * size).all())
 
 
+@pytest.mark.parametrize("p,nv", [(3, 3), (4, 200), (5, 70), (7, 40), (8, 3), (8, 600)])
+@pytest.mark.parametrize("dt", [torch.float64, torch.float32])
+def test_self_apply_in_place(hip, p, nv, dt):
+    """Up to order 8 a vesicle's coefficients are read before any of its results
+    is written, so V may be F or G itself.  The sums of the call with a V of its
+    own in any order: 2 n eps of the sum of their sizes, as above."""
+    n = 3 * p * (p + 2)
+    g = torch.Generator(device="cuda").manual_seed(p + nv)
+    M, D = (torch.randn((nv, n, n), dtype=dt, device="cuda", generator=g) for _ in range(2))
+    F, H = (torch.randn((nv, n), dtype=torch.float64, device="cuda", generator=g) for _ in range(2))
+    for both, over in ((False, 0), (True, 0), (True, 1)):
+        V = torch.zeros_like(F)
+        G.self_apply(M, F, D if both else None, H if both else None, nv, p, V)
+        size = torch.bmm(F.abs()[:, None], M.double().abs())[:, 0]
+        if both:
+            size += torch.bmm(H.abs()[:, None], D.double().abs())[:, 0]
+        f, h = F.clone(), H.clone()
+        G.self_apply(M, f, D if both else None, h if both else None, nv, p, h if over else f)
+        assert bool((((h if over else f) - V).abs() <= 2 * n * 2.3e-16 * size).all())
+
+
 @pytest.mark.parametrize("p0", [16, 8])
 def test_singular_build_fused_pole_stage(hip, p0):
     """The FP64 build's fused pole kernel + transposed synthesis (the default

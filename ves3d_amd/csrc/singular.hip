@@ -1333,9 +1333,12 @@ int self_apply(const TM *SL, const double *F, const TM *DL, const double *G, lon
   // thread per column: order 12 (504 columns), 320 / 512 vesicles in FP64 108 /
   // 168 us against 114 / 180; 192: 86 against 66.
   const bool wide = !sym && (long)cdiv(n, 64) * Nv >= 2560 && (long)cdiv(n, 256) * 256 - n <= n / 32;
+  // V over F or G: one workgroup per vesicle, which has read both before it
+  // writes (up to order 8; the blocks of more columns read what others write)
+  const bool over = !sym && n <= 256 && ((SL && V == F) || (DL && V == G));
   if (sym)
     k_self_apply_split<TM, true><<<gs, 1024, 0, st>>>(SL, F, DL, G, nc, V);
-  else if (!wide)
+  else if (!wide && !over)
     k_self_apply_split<TM, false><<<gs, 1024, 0, st>>>(SL, F, DL, G, nc, V);
   else
     k_self_apply<TM><<<dim3(cdiv(n, 256), (unsigned)Nv), 256, 2 * n * sizeof(double), st>>>(
