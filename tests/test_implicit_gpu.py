@@ -329,3 +329,41 @@ def test_extrapolated_initial_guess(hip):
     assert i1[:2] == i0[:2]
     assert all(a <= b for a, b in zip(i1[2:], i0[2:])), (i0, i1)
     assert np.linalg.norm(U1 - U0) / np.linalg.norm(U0) < 1e-6
+
+
+@pytest.mark.parametrize("p,precision", [(5, 0), (8, 0), (8, 2)])
+def test_self_apply_symmetric_forms(hip, p, precision):
+    """The symmetric self apply of 1024 vesicles (a thread per column) against
+    eight times that of 128 (rows split over waves), through the vesicles' own
+    operator: the same products in FP64 in another order, 1e-12 of the largest."""
+    nv, part, nc = 1024, 128, p * (p + 2)
+    X = W.implicit_step_case(nv=nv, p=p, seed=2)
+    rng = np.random.default_rng(4)
+    U, S = rng.standard_normal((3 * nv, nc)), rng.standard_normal((nv, nc))
+
+    def order_major(rows):  # blocks of p + 1 - m coefficients, function-major in each
+        off = np.cumsum([0] + [p + 1 - (j + 1) // 2 for j in range(2 * p)])
+        return np.concatenate([rows[:, a:b].ravel() for a, b in zip(off, off[1:])])
+
+    def functions(y, n):
+        out, at = np.empty((n, nc)), 0
+        off = np.cumsum([0] + [p + 1 - (j + 1) // 2 for j in range(2 * p)])
+        for a, b in zip(off, off[1:]):
+            out[:, a:b] = y[at:at + n * (b - a)].reshape(n, b - a)
+            at += n * (b - a)
+        return out
+
+    def local(v0, n):
+        st = I.Stepper(n, p, precision=precision, near=False)
+        st.set_state(torch.from_numpy(np.ascontiguousarray(X[v0:v0 + n])).cuda())
+        st.prepare()
+        x = np.concatenate([order_major(U[3 * v0:3 * (v0 + n)]), order_major(S[v0:v0 + n])])
+        y = st.matvec_local(torch.from_numpy(x).cuda()).cpu().numpy()
+        st.close()
+        return functions(y[:3 * n * nc], 3 * n), functions(y[3 * n * nc:], n)
+
+    u, s = local(0, nv)
+    for v0 in range(0, nv, part):
+        a, b = local(v0, part)
+        assert np.max(np.abs(u[3 * v0:3 * (v0 + part)] - a)) < 1e-12 * np.max(np.abs(a))
+        assert np.max(np.abs(s[v0:v0 + part] - b)) < 1e-12 * np.max(np.abs(b))

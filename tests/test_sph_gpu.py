@@ -333,6 +333,28 @@ def test_self_apply_rows_split(hip, p, nv, dt):
         assert bool(((V - ref).abs() <= 2 * n * 2.3e-16 * size).all())
 
 
+@pytest.mark.parametrize("dt,p,nv", [
+    (torch.float64, 4, 767), (torch.float64, 4, 768), (torch.float64, 7, 511),
+    (torch.float64, 7, 512), (torch.float64, 8, 683), (torch.float32, 4, 1023),
+    (torch.float32, 4, 1024), (torch.float32, 9, 511), (torch.float32, 9, 512),
+    (torch.float32, 13, 512)])
+def test_self_apply_many_vesicles(hip, dt, p, nv):
+    """Both sides of the line between a thread per column and split rows: 2 n eps
+    of the sum of the products' sizes, as above."""
+    n = 3 * p * (p + 2)
+    g = torch.Generator(device="cuda").manual_seed(p + nv)
+    M, D = (torch.randn((nv, n, n), dtype=dt, device="cuda", generator=g) for _ in range(2))
+    F, H = (torch.randn((nv, n), dtype=torch.float64, device="cuda", generator=g) for _ in range(2))
+    V = torch.full((nv, n), 7.0, dtype=torch.float64, device="cuda")
+    G.self_apply(M, F, D, H, nv, p, V)
+    size, ref = torch.zeros_like(V), torch.zeros_like(V)
+    for A, x in ((M, F), (D, H)):
+        for v in range(nv):
+            ref[v] += x[v] @ A[v].double()
+            size[v] += x[v].abs() @ A[v].double().abs()
+    assert bool(((V - ref).abs() <= 2 * n * 2.3e-16 * size).all())
+
+
 @pytest.mark.parametrize("p,nv", [(3, 3), (4, 200), (5, 70), (7, 40), (8, 3), (8, 600)])
 @pytest.mark.parametrize("dt", [torch.float64, torch.float32])
 def test_self_apply_in_place(hip, p, nv, dt):

@@ -19,7 +19,7 @@
 // every GEMM stage in FP32 and keeps the pole kernel (singular weights, 1/r
 // near the rotated pole) in FP64.  Both write the operator's (a, b) and
 // (b, a) blocks equal (the rows of one symmetric tensor component), which
-// the step's self apply relies on (k_self_apply_split).
+// the step's self apply relies on (k_self_apply_sym, k_self_apply_split).
 #include <algorithm>
 #include <atomic>
 #include <cmath>
@@ -1258,18 +1258,57 @@ __global__ __launch_bounds__(256) void k_self_apply(const TM *__restrict__ SL,
   V[v * n + c] = (acc0 + acc1) + (acc2 + acc3);
 }
 
-// The same with a workgroup's 16 waves on parts of the rows of 64 columns, the
-// parts added in order through LDS.  SYM: the singular build's operators, whose
-// 3 x 3 blocks of Ncoef x Ncoef satisfy B_ab = B_ba (block (a, b) holds the rows
-// of the symmetric tensor component c(a, b), formed once and written to both):
-// lane cc reads the six blocks a <= b at column cc once and forms V[b Nc + cc] =
-// sum_a sum_k F[a Nc + k] B_ab[k][cc] for b = 0, 1, 2 -- two thirds of the
-// general form's matrix reads.
+// As k_self_apply for the singular build's operators, whose 3 x 3 blocks of
+// Ncoef x Ncoef satisfy B_ab = B_ba (block (a, b) holds the rows of the
+// symmetric tensor component c(a, b), formed once and written to both):
+// thread cc reads the six blocks a <= b at column cc once and forms
+// V[b Nc + cc] = sum_a sum_k F[a Nc + k] B_ab[k][cc] for b = 0, 1, 2 -- two
+// thirds of the general kernel's matrix reads.  One workgroup per vesicle.
+template <typename TM>
+__global__ __launch_bounds__(256) void k_self_apply_sym(const TM *__restrict__ SL,
+                                                         const double *__restrict__ F,
+                                                         const TM *__restrict__ DL,
+                                                         const double *__restrict__ G, int nc,
+                                                         double *__restrict__ V) {
+  extern __shared__ double sh[];
+  const int n = 3 * nc;
+  const long v = blockIdx.y;
+  const int cc = threadIdx.x;
+  double *f = sh, *g = sh + n;
+  for (int i = threadIdx.x; i < n; i += blockDim.x) {
+    f[i] = SL ? F[v * n + i] : 0.0;
+    g[i] = DL ? G[v * n + i] : 0.0;
+  }
+  __syncthreads();
+  if (cc >= nc) return;
+  double v0 = 0, v1 = 0, v2 = 0;
+  auto run = [&](const TM *M, const double *x) {
+    const TM *m = M + v * (long)n * n + cc;  // element (row, b nc + cc) at row n + b nc
+#pragma unroll 2
+    for (int k = 0; k < nc; ++k) {
+      const TM *r0 = m + (long)k * n, *r1 = m + (long)(nc + k) * n,
+               *r2 = m + (long)(2 * nc + k) * n;
+      const double b00 = (double)r0[0], b01 = (double)r0[nc], b02 = (double)r0[2 * nc];
+      const double b11 = (double)r1[nc], b12 = (double)r1[2 * nc], b22 = (double)r2[2 * nc];
+      const double x0 = x[k], x1 = x[nc + k], x2 = x[2 * nc + k];
+      v0 += x0 * b00 + x1 * b01 + x2 * b02;
+      v1 += x0 * b01 + x1 * b11 + x2 * b12;
+      v2 += x0 * b02 + x1 * b12 + x2 * b22;
+    }
+  };
+  if (SL) run(SL, f);
+  if (DL) run(DL, g);
+  V[v * n + cc] = v0;
+  V[v * n + nc + cc] = v1;
+  V[v * n + 2 * nc + cc] = v2;
+}
+
+// Both with a workgroup's 16 waves on parts of the rows of 64 columns (SYM: lane
+// cc as the thread above), the parts added in order through LDS.
 // Bound: the matrix reads (5.9 TB/s for 512 vesicles at order 16) or, with few
 // vesicles, their latency.  A thread per column down all rows, before -> after
-// in us (FP64, order 12, symmetric): 2 vesicles 23 -> 9, 48: 39 -> 13, 512: 122
-// -> 125; order 16: 66 -> 14, 72 -> 29, 353 -> 344; general: 37 -> 9, 116 -> 45,
-// 508 -> 504.
+// in us (FP64, order 12, symmetric): 2 vesicles 23 -> 9, 48: 39 -> 13; order 16:
+// 66 -> 14, 72 -> 29; general: 37 -> 9, 116 -> 45.
 template <typename TM, bool SYM>
 __global__ __launch_bounds__(1024) void k_self_apply_split(const TM *__restrict__ SL,
                                                            const double *__restrict__ F,
@@ -1328,21 +1367,44 @@ int self_apply(const TM *SL, const double *F, const TM *DL, const double *G, lon
   const int n = 3 * sh_ncoef(p);
   if (!SL && !DL) return hip_status(hipMemsetAsync(V, 0, sizeof(double) * n * Nv, st));
   const int nc = sh_ncoef(p);
-  const dim3 gs(cdiv(sym ? nc : n, 64), (unsigned)Nv);
-  // Many vesicles whose columns nearly fill blocks of 256 read longer runs with a
-  // thread per column: order 12 (504 columns), 320 / 512 vesicles in FP64 108 /
-  // 168 us against 114 / 180; 192: 86 against 66.
-  const bool wide = !sym && (long)cdiv(n, 64) * Nv >= 2560 && (long)cdiv(n, 256) * 256 - n <= n / 32;
+  const int lines = sym ? nc : n;  // columns with a sum of their own
+  const dim3 gs(cdiv(lines, 64), (unsigned)Nv);
+  const long waves = (long)gs.x * Nv;
+  const bool f64 = sizeof(TM) == 8;
+  // From about two workgroups per CU on a thread per column reads longer runs
+  // and needs no sums over waves, unless a vesicle's block of 256 threads is
+  // large enough to leave the last CUs waiting.  Us, thread per column / split,
+  // matrices of 512 vesicles (1024: *):
+  //   symmetric, FP64: orders 5* 12 / 15, 8 24 / 29, 12 119 / 124, 13 161 / 178,
+  //     16 (288 coefficients) 355 / 341; FP32: 8* 26 / 39, 11* 94 / 115, 13 93 / 112;
+  //     but order 6 14 / 12 and 320 vesicles of order 14 155 / 131
+  //   general, FP32: orders 5* 12 / 15, 8* 34 / 45, 11* 140 / 158, 13 124 / 144, but
+  //     16 259 / 248; FP64: 5* 14 / 19, 7 22 / 27, 7* 43 / 52, 12 168 / 174, but from
+  //     256 columns on 10 93 / 89, 10* 202 / 175, and where the matrices outgrow the
+  //     256 MB last-level cache, 2000 vesicles of order 6: 66 / 58
+  // FP64 of order 12 nearly fills its blocks of 256: 108 / 114 for 320 vesicles,
+  // 86 / 66 for 192.
+  bool wide;
+  if (sym)
+    wide = nc < 256 && Nv >= 512 && waves >= 1024;
+  else if (f64)
+    wide = (Nv >= 512 && waves >= 1536 && n < 256 &&
+            (n < 128 || Nv * n * n <= (300L << 20) / 8)) ||
+           (waves >= 2560 && (int)cdiv(n, 256) * 256 - n <= n / 32 && n <= 4096);
+  else
+    wide = Nv >= 512 && waves >= 2048 && n < 640;
   // V over F or G: one workgroup per vesicle, which has read both before it
   // writes (up to order 8; the blocks of more columns read what others write)
   const bool over = !sym && n <= 256 && ((SL && V == F) || (DL && V == G));
-  if (sym)
+  const size_t lds = 2 * n * sizeof(double);
+  if (sym && wide)
+    k_self_apply_sym<TM><<<dim3(1, (unsigned)Nv), 64 * gs.x, lds, st>>>(SL, F, DL, G, nc, V);
+  else if (sym)
     k_self_apply_split<TM, true><<<gs, 1024, 0, st>>>(SL, F, DL, G, nc, V);
-  else if (!wide && !over)
-    k_self_apply_split<TM, false><<<gs, 1024, 0, st>>>(SL, F, DL, G, nc, V);
+  else if (wide || over)
+    k_self_apply<TM><<<dim3(cdiv(n, 256), (unsigned)Nv), 256, lds, st>>>(SL, F, DL, G, n, V);
   else
-    k_self_apply<TM><<<dim3(cdiv(n, 256), (unsigned)Nv), 256, 2 * n * sizeof(double), st>>>(
-        SL, F, DL, G, n, V);
+    k_self_apply_split<TM, false><<<gs, 1024, 0, st>>>(SL, F, DL, G, nc, V);
   return launch_status();
 }
 
