@@ -128,6 +128,33 @@ def test_transforms_over_their_input(hip, p0, p1, N, dt, tol):
             assert err(o.reshape(N, -1), ref) < tol
 
 
+@pytest.mark.parametrize("p0,p1,N", [
+    (4, 4, 4095), (4, 4, 4096), (12, 12, 6143), (12, 12, 6144), (30, 20, 2047), (30, 20, 2048),
+    (32, 32, 1279), (32, 32, 1280), (32, 32, 3071), (32, 32, 3072), (24, 12, 6143),
+    (24, 12, 6144), (3, 3, 10239), (3, 3, 10240), (8, 8, 24575), (8, 8, 24576), (6, 3, 12287),
+    (6, 3, 12288), (32, 32, 20480)])
+@pytest.mark.parametrize("dt,tol", [(torch.float64, 1e-12), (torch.float32, 1e-5)])
+def test_transform_lines_to_gemms(hip, p0, p1, N, dt, tol):
+    """Both sides of the lines between the one-kernel transforms and the GEMMs,
+    as test_one_kernel_transforms, and the value with its longitude derivative,
+    which has a line of its own."""
+    from ves3d_amd import call
+    test_one_kernel_transforms(hip, p0, p1, N, dt, tol)
+    S = torch.from_numpy(RNG.standard_normal((N, p0 * (p0 + 2)))).to("cuda", dt)
+    out = {}
+    try:
+        for tile in (-1, 0):
+            call("ves3d_hip_set_gemm_tile", tile)
+            out[tile] = [torch.zeros((N, 2 * p1 * (p1 + 1)), dtype=dt, device="cuda")
+                         for _ in range(2)]
+            G.shc2grid(S, N, p0, p1, *out[tile])
+            torch.cuda.synchronize()
+    finally:
+        call("ves3d_hip_set_gemm_tile", -1)
+    for x, y in zip(out[-1], out[0]):
+        assert float((x - y).abs().max() / y.abs().max()) < tol
+
+
 @pytest.mark.parametrize("p,N", [(6, 4), (16, 9)])
 def test_shc2pole(hip, p, N):
     S = RNG.standard_normal((N, p * (p + 2)))

@@ -32,7 +32,10 @@ namespace {
 
 constexpr int kThreads = 512, kWaves = kThreads / 64;
 constexpr size_t kLdsMost = 64 * 1024;  // two workgroups per CU
-constexpr int kMaxSteps = 8;            // orders of the contracted side up to 32
+// Orders of the contracted side up to 32: at 33 to 48 a handful of functions is
+// faster in one kernel (2 at order 48: 10.6 us, 16.7 as GEMMs), many are slower
+// (6144: 196, 122 us), and more instances would have to be kept for the few.
+constexpr int kMaxSteps = 8;
 constexpr int kBatch = 8;               // table values a thread has in flight
 
 __host__ __device__ __forceinline__ int up16(int v) { return (v + 15) & ~15; }
@@ -413,16 +416,72 @@ int launch_groups(const A &a, int fg, int nvar, hipStream_t st) {
 
 }  // namespace
 
+namespace {
+
+constexpr long kAlways = 1L << 60;
+
+// The number of functions from which the GEMMs synthesise nvar variants of order
+// p0 on the grid of p1.  A workgroup of 512 threads takes at most four functions,
+// which is little work on a small grid, and forms the Legendre sums of every
+// variant; the GEMMs share the tables over 64 functions and, of a value and its
+// longitude derivative (nvar = 2), the sums.  Drawn from orders 1 to 32 with 512
+// to 131072 functions; here / as GEMMs in us:
+//  - FP64, three variants: orders 6 -> 6, N = 3072 / 4608: 17 / 21, 24 / 22; 6 ->
+//    12, 6144 / 12288: 34 / 39, 71 / 57; 12 -> 12, 8192 / 16384: 59 / 59, 120 / 89;
+//    16 -> 16, 12288: 110 / 110; one variant, 6 -> 6, 6144 / 8192: 11 / 11, 15 / 12
+//  - order above 24 (two functions or one fit the LDS): 30 -> 20, 1536 / 3072: 43 /
+//    56, 88 / 80; 32 -> 32, 3072 / 12288: 121 / 142, 569 / 473; one variant, 30 ->
+//    30, 12288 / 16384: 152 / 163, 226 / 204
+//  - the value and its longitude derivative: 12 -> 12, 6144 / 8192: 30 / 31, 40 / 34
+//  - FP32, three variants: 6 -> 6, 4608 / 8192: 17 / 22, 28 / 23; 24 -> 12, 6144 /
+//    8192: 50 / 55, 68 / 63; 32 -> 32, 16384 / 24000: 309 / 348, 575 / 514
+template <typename T>
+long synth_line(int p0, int p1, int nvar) {
+  if (sizeof(T) == 8) {
+    if (p0 > 24) return p1 < p0 ? 2048 : (nvar == 1 ? 12288 : 3072);
+    if (p0 >= 20 && p1 < p0) return nvar == 2 ? 4096 : 6144;
+    if (p1 >= 28) return p1 >= 36 && nvar > 1 ? 12288 : kAlways;
+    if (p1 <= 8) return nvar == 1 ? 6144 : 4096;
+    return p1 < 12 || (p1 == 12 && nvar == 2) ? 6144 : 12288;
+  }
+  if (p0 >= 20 && (p1 < p0 || (nvar == 2 && p1 == p0 && p0 <= 24))) return 6144;
+  if (p0 > 24) return 20480;
+  return p1 < 12 ? 6144 : (p1 < 28 ? 12288 : kAlways);
+}
+
+// The same for the analysis of grids of p0 to order p1.  Here / as GEMMs in us:
+//  - small grids, FP64: 3 -> 3, N = 8192 / 12288: 9 / 11, 13 / 11; 6 -> 6, 24000 /
+//    32768: 25 / 25, 34 / 26; 8 -> 8, 65536: 75 / 60; FP32: 3 -> 3, 12288 / 16384: 10
+//    / 12, 13 / 12; 12 -> 12, 65536: 85 / 73; but FP64 8 -> 16, 65536: 94 / 126
+//  - half the order, few results per function: FP64 8 -> 4, 12288: 14 / 14, 32 -> 16,
+//    16384: 159 / 128; FP32 16 -> 8, 16384 / 32768: 25 / 25, 46 / 42
+//  - both orders above 24, FP64, where one function (order 32) or two fit the LDS:
+//    32 -> 32, 1024 / 1536: 29 / 33, 42 / 38; 28 -> 28, 4608 / 6144: 61 / 64, 80 / 75;
+//    FP32, 32 -> 32, 16384 / 24000: 140 / 137, 230 / 202
+//  - FP64 from order 20 on: 24 -> 24, 24000 / 32768: 214 / 210, 290 / 261
+template <typename T>
+long analysis_line(int p0, int p1) {
+  const bool f64 = sizeof(T) == 8;
+  long line = kAlways;
+  if (p0 > 24 && p1 > 24)
+    line = f64 ? (analysis_lds(p0, p1, 2, sizeof(T)) > kLdsMost ? 1280 : 5120) : 20480;
+  else if (f64 && p0 >= 20)
+    line = 24576;
+  if (2 * p1 <= p0 && (f64 || p0 <= 20)) line = std::min(line, f64 ? 12288L : 16384L);
+  if (p0 <= 4)
+    line = std::min(line, f64 ? 10240L : 12288L);
+  else if (p0 <= 6 || (p0 <= 12 && p1 <= p0))
+    line = std::min(line, 24576L);
+  return line;
+}
+
+}  // namespace
+
 template <typename T>
 bool synth_fused(const T *S, long N, int p0, int p1, int nvar, const ShMatsHost &h, const T *mats,
                  const int *dleg, const int *dfour, T *const *X, T alpha, hipStream_t st,
                  int *status) {
-  // For many functions on small grids the GEMMs, which form the Legendre sums of
-  // variants without a latitude derivative once, are faster.  FP64, three variants
-  // here / there in us: orders 6 -> 6, N = 3072 / 8192: 18, 41 / 21, 29; 12 -> 12,
-  // N = 8192 / 16384: 59, 120 / 61, 90; 10 -> 20: 81, 154 / 92, 144; but 14 -> 28,
-  // N = 16384 / 70000: 194, 1200 / 290, 1184, and 16 -> 32: 295, 1401 / 365, 1483.
-  if (p1 < 28 && N >= (p1 < 12 ? 6144 : 12288)) return false;
+  if (N >= synth_line<T>(p0, p1, nvar)) return false;
   const int fg = functions_per_group(N, nvar, synth_lds, p0, p1, sizeof(T));
   if (fg == 0) return false;
   for (int v = 0; v < nvar; ++v)
@@ -450,19 +509,7 @@ bool synth_fused(const T *S, long N, int p0, int p1, int nvar, const ShMatsHost 
 template <typename T>
 bool analysis_fused(const T *X, long N, int p0, int p1, bool transpose, const ShMatsHost &h,
                     const T *mats, T *S, hipStream_t st, int *status) {
-  // With both orders above 24 in FP64 a workgroup's LDS holds one or two
-  // functions, which read the Legendre tables again; for many functions the
-  // GEMMs, which share them over 64, are faster.  Orders 32 -> 32 (one fits), N =
-  // 1024 / 1536 / 6144: 29 / 43 / 157 us here and 32 / 38 / 100 us there; orders 28
-  // -> 28 (two), N = 3072 / 6144: 41 / 80 and 43 / 75 us.
-  if (sizeof(T) == 8 && p0 > 24 && p1 > 24 &&
-      N >= (analysis_lds(p0, p1, 2, sizeof(T)) > kLdsMost ? 1280 : 5120))
-    return false;
-  // Where the order falls to half, a group's few results per function leave the
-  // GEMMs ahead once they fill the chip.  N = 12288 / 60000, FP64: orders 12 -> 6
-  // 23 / 95 and 23 / 70 us, 32 -> 16 103 / 568 and 104 / 504; FP32: 12 -> 6 14 / 60
-  // and 16 / 46 us, but 24 -> 12 31 / 149 and 38 / 166.
-  if (2 * p1 <= p0 && N >= 16384 && (sizeof(T) == 8 || p0 <= 16)) return false;
+  if (N >= analysis_line<T>(p0, p1)) return false;
   const int fg = functions_per_group(N, 1, analysis_lds, p0, p1, sizeof(T));
   if (fg == 0 || overlap(X, N * sh_ngrid(p0), S, N * sh_ncoef(p1))) return false;
   const T *frag = frag_table<T>(p0, p1, transpose ? 4 : 3, h);
