@@ -125,6 +125,51 @@ def test_direct_stokes_edges(hip, orc, nv, ss, ts, dtype, tol, dl):
     assert _relerr(out[3:], ref[3:]) < tol if nv > 3 else True
 
 
+@pytest.mark.parametrize("dl", [False, True])
+@pytest.mark.parametrize("dtype,tol", [(torch.float64, 1e-12), (torch.float32, 2e-5)])
+@pytest.mark.parametrize("nv,ss,ts", [(3, 16, 70), (3, 17, 70), (2, 40, 129), (2, 100, 64),
+                                      (2, 300, 10), (1100, 65, 3), (2999, 128, 20),
+                                      (3000, 128, 20), (3000, 127, 20)])
+def test_direct_stokes_forms(hip, orc, nv, ss, ts, dtype, tol, dl):
+    """Both sides of the lines between sources staged by one wave and split over
+    1, 2, 4, 8 and 16; half of the targets on sources, head and tail inside.
+    Tolerances as above; the vesicles at both ends are compared."""
+    head, tail = min(2, ts - 1), ts
+    src, den, nrm, trg, qw = _vesicle_case(nv, ss, ts)
+    n = min(ss, ts) // 2
+    trg[:, :, :n] = src[:, :, :n]
+    c = lambda a: _cuda(a, dtype)
+    pot = torch.full((nv, 3, ts), 7.0, dtype=dtype, device="cuda")
+    if dl:
+        K.direct_stokes_dl(c(src), c(nrm), c(den), c(qw), ss, ts, nv, c(trg), head, tail, pot)
+    else:
+        K.direct_stokes(c(src), c(den), c(qw), ss, ts, nv, c(trg), head, tail, pot)
+    out = pot.double().cpu().numpy()
+    assert np.all(out[:, :, :head] == 7.0) and np.all(np.isfinite(out))
+    for v0 in sorted({0, max(0, nv - 40)}):
+        m = min(40, nv - v0)
+        cut = lambda a: np.ascontiguousarray(a[v0:v0 + m])
+        s, d, t, ref = cut(src), cut(den), cut(trg), np.zeros((m, 3, ts))
+        geo = (OL.ci(ss), OL.ci(ts), OL.ci(m), OL.ci(head), OL.ci(tail), OL.p(qw), OL.p(t), OL.p(s))
+        if dl:
+            nn = cut(nrm)
+            orc.orc_direct_stokes_dl(*geo, OL.p(nn), OL.p(d), OL.p(ref))
+        else:
+            orc.orc_direct_stokes(*geo, OL.p(d), OL.p(ref))
+        if dtype == torch.float64:
+            assert _relerr(out[v0:v0 + m, :, head:], ref[:, :, head:]) < tol
+        else:
+            # random clouds: a pair at distance r carries the rounding of its two
+            # positions, 2 sqrt(3) eps / r, in r^-1 (double layer: r^-2) terms; the
+            # closest of the pairs dominates the error as it does the sum
+            x = s.transpose(0, 2, 1)[:, None] - t.transpose(0, 2, 1)[:, :, None]
+            r = np.linalg.norm(x, axis=3)
+            r[r == 0] = np.inf
+            terms = (3 / (4 * np.pi) / r ** 2 if dl else 1 / (8 * np.pi) / r)
+            bound = 40 * 6e-8 * (terms * (3 + 3.5 / r)).sum(2)[:, None, head:]
+            assert np.all(np.abs(out[v0:v0 + m, :, head:] - ref[:, :, head:]) <= bound)
+
+
 def test_direct_stokes_bad_range(hip):
     src = torch.zeros(3 * 8, dtype=torch.float64, device="cuda")
     pot = torch.zeros(3 * 8, dtype=torch.float64, device="cuda")

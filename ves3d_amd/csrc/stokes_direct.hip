@@ -26,7 +26,8 @@
 //     DirectStokesDoubleLayer sums (src/CPUKernels.cc:8-118, :1059-1136) on
 //     AxisMajor [ves][xyz][stride] data: 64 targets of one vesicle per
 //     workgroup, its sources split over the workgroup's waves and read through
-//     the scalar cache.
+//     the scalar cache, or staged through LDS by one wave where they are few or
+//     come from memory.
 #include <algorithm>
 #include <atomic>
 #include <type_traits>
@@ -972,6 +973,83 @@ __global__ __launch_bounds__(1024) void k_vesicle_stokes(
   }
 }
 
+// One wave per 64 targets of a vesicle, whose sources go through LDS.
+constexpr int VS_TILE = 256;
+template <typename Real, bool DLK>
+__global__ __launch_bounds__(64) void k_vesicle_staged(
+    const Real *__restrict__ src, const Real *__restrict__ nrm, const Real *__restrict__ den,
+    const Real *__restrict__ qw, long ss, long ts, long head, long tail,
+    const Real *__restrict__ trg, Real *__restrict__ pot, Real scal) {
+  __shared__ Real sh[VS_TILE][DLK ? 10 : 6];
+  const long vt = blockIdx.y;
+  const long t = head + (long)blockIdx.x * 64 + threadIdx.x;
+  const bool tvalid = t < tail;
+  const Real *S = src + 3 * ss * vt;
+  const Real *D = den + 3 * ss * vt;
+  const Real *N = DLK ? nrm + 3 * ss * vt : nullptr;
+  Real tx = 0, ty = 0, tz = 0;
+  if (tvalid) {
+    const Real *T = trg + 3 * ts * vt;
+    tx = T[t];
+    ty = T[ts + t];
+    tz = T[2 * ts + t];
+  }
+  Real px = 0, py = 0, pz = 0;
+  for (long c0 = 0; c0 < ss; c0 += VS_TILE) {
+    const int cnt = (int)min((long)VS_TILE, ss - c0);
+    __syncthreads();
+    for (int i = threadIdx.x; i < cnt; i += 64) {
+      const long s = c0 + i;
+      const Real w = qw ? qw[s] : Real(1);
+      sh[i][0] = S[s];
+      sh[i][1] = S[ss + s];
+      sh[i][2] = S[2 * ss + s];
+      if (DLK) {
+        sh[i][3] = D[s];
+        sh[i][4] = D[ss + s];
+        sh[i][5] = D[2 * ss + s];
+        sh[i][6] = N[s];
+        sh[i][7] = N[ss + s];
+        sh[i][8] = N[2 * ss + s];
+        sh[i][9] = w;
+      } else {
+        sh[i][3] = D[s] * w;
+        sh[i][4] = D[ss + s] * w;
+        sh[i][5] = D[2 * ss + s] * w;
+      }
+    }
+    __syncthreads();
+    if (tvalid) {
+#pragma unroll 4
+      for (int j = 0; j < cnt; ++j) {
+        const Real dx = sh[j][0] - tx, dy = sh[j][1] - ty, dz = sh[j][2] - tz;
+        const Real r2 = dx * dx + dy * dy + dz * dz;
+        const Real ri = (r2 != Real(0)) ? Real(1) / sqrt(r2) : Real(0);
+        if (DLK) {
+          const Real ri2 = ri * ri;
+          const Real rn = sh[j][6] * dx + sh[j][7] * dy + sh[j][8] * dz;
+          const Real rf = sh[j][3] * dx + sh[j][4] * dy + sh[j][5] * dz;
+          const Real c = rn * rf * (ri2 * ri2 * ri) * sh[j][9];
+          px += dx * c;
+          py += dy * c;
+          pz += dz * c;
+        } else {
+          const Real cc = (dx * sh[j][3] + dy * sh[j][4] + dz * sh[j][5]) * ri * ri;
+          px += (sh[j][3] + cc * dx) * ri;
+          py += (sh[j][4] + cc * dy) * ri;
+          pz += (sh[j][5] + cc * dz) * ri;
+        }
+      }
+    }
+  }
+  if (tvalid) {
+    Real *P = pot + 3 * ts * vt;
+    P[t] = px * scal;
+    P[ts + t] = py * scal;
+    P[2 * ts + t] = pz * scal;
+  }
+}
+
 template <typename Real, bool DLK>
 static int vesicle_stokes(const Real *src, const Real *nrm, const Real *den,
                           const Real *qw, size_t ss, size_t ts, size_t nv,
@@ -984,9 +1062,30 @@ static int vesicle_stokes(const Real *src, const Real *nrm, const Real *den,
   const Real scal = DLK ? Real(-3.0 / (4.0 * kPi)) : Real(1.0 / kPi / 8.0);
   const size_t nblocks = cdiv(tail - head, 64), groups = nblocks * nv;
   if (groups > 0x7fffffff) return VES3D_INVALID_PARAMETER;
-  // four waves per group fill the chip (16 waves per SIMD) from 4096 groups on;
-  // fewer groups get 16 waves each
-  const int nw = groups >= 4096 ? 4 : 16;
+  // Staged through LDS by one wave where a group has too few sources for the
+  // start and end of a wave that splits them (FP64 double layer, 16 sources, 1500
+  // vesicles of 544 targets 37 us, 40 to 96 split; single layer, 8, 4000 vesicles 44,
+  // 50 to 194), and in the double layer where at most two groups share a vesicle's
+  // sources and all vesicles' are too many for the caches, so that the scalar
+  // loads of ten streams wait for memory (2112 sources, 20 targets, 4000 vesicles:
+  // FP64 1142 us, 2757 split, FP32 623, 917; 512 sources, FP64 283, 337; but 1104
+  // sources of 1500 vesicles 324, 292, four groups per vesicle 1002, 717, 8 targets
+  // of 1500 vesicles with 2112 sources 928, 764, and in FP32 5000 sources 1055, 703).
+  const size_t src_bytes = nv * ss * 9 * sizeof(Real);
+  const bool many = groups >= 3000, large = src_bytes >= 200000000;
+  const bool waits = sizeof(Real) == 8 ? (many && ss >= 128) || (large && tail - head >= 16)
+                                       : many && large;
+  const bool staged = ss <= 16 || (DLK && nblocks <= 2 && waits);
+  if (staged) {
+    k_vesicle_staged<Real, DLK><<<dim3((unsigned)nblocks, (unsigned)nv), 64, 0, st>>>(
+        src, nrm, den, qw, (long)ss, (long)ts, (long)head, (long)tail, trg, pot, scal);
+    return launch_status();
+  }
+  // Four waves per group from 1024 groups on, 16 below, and no more than give each
+  // at least 8 (FP32: 16) sources: 4 / 16 waves for 1500 vesicles of 64 sources and
+  // 544 targets in FP32 43 / 164 us, two 36; 40 vesicles of 512 and 544 in FP64 22 / 21.
+  int nw = groups >= 1024 ? 4 : 16;
+  while (nw > 1 && (size_t)nw * (sizeof(Real) == 8 ? 8 : 16) > ss) nw /= 2;
   const long chunk = (long)((ss + nw - 1) / nw + 3) / 4 * 4;
   if (qw)
     k_vesicle_stokes<Real, DLK, true><<<(unsigned)groups, 64 * nw, 0, st>>>(
