@@ -274,6 +274,17 @@ def test_direct_eval_split_edges(hip, orc, sl, dl, ns, nt, spg):
         assert _relerr(got[pick], ref[pick]) < tol, (mixed, _relerr(got[pick], ref[pick]))
 
 
+@pytest.mark.parametrize("sl,dl", [(True, False), (False, True), (True, True)])
+@pytest.mark.parametrize("ns,nt,spg", [
+    (128, 300, 0), (129, 300, 0), (512, 300, 0), (513, 300, 0), (513, 65535, 0), (513, 65536, 0),
+    (700, 19999, 0), (700, 20000, 0), (20 * 64, 20 * 64, 64), (20 * 100, 20 * 77, 100),
+    (20 * 101, 20 * 77, 101), (40 * 64, 40 * 60, 64), (26000, 700, 0)])
+def test_direct_eval_forms(hip, orc, sl, dl, ns, nt, spg):
+    """Both sides of the lines between the mixed form's records and LDS tiles,
+    and slices in multiples of the XCDs, as test_direct_eval_split_edges."""
+    test_direct_eval_split_edges(hip, orc, sl, dl, ns, nt, spg)
+
+
 @pytest.mark.parametrize("mixed", [False, True])
 @pytest.mark.parametrize("sl,dl", [(True, False), (False, True), (True, True)])
 @pytest.mark.parametrize("bad", [float("nan"), float("inf"), 1e300])

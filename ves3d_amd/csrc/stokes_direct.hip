@@ -20,7 +20,8 @@
 //     shifts the lane's target by the same anchor in FP64 before rounding, so
 //     coordinate differences keep FP32 relative accuracy independent of the
 //     box size; pair terms are summed in FP32 over 64 sources and merged into
-//     an FP32 (hi, lo) TwoSum pair.
+//     an FP32 (hi, lo) TwoSum pair.  Few sources, and most single layers, take
+//     the same FP32 terms from LDS tiles (k_tiles_f32c).
 //
 //  2. k_vesicle_*: the per-vesicle Device<>::DirectStokes /
 //     DirectStokesDoubleLayer sums (src/CPUKernels.cc:8-118, :1059-1136) on
@@ -471,6 +472,84 @@ __global__ __launch_bounds__(FF_BLOCK, DL ? 8 : (GUARD ? 6 : 7)) void k_pairs_f3
   store_sums(w, map.share, n_trg, v, part + (long)slice * n_trg * 3);
 }
 
+// The FP32 form with its sources converted into LDS tile by tile, a workgroup's
+// 256 targets on one slice: whole groups, or (spg = 0) an even part of the
+// sources.  A lane leaves its own group out.
+template <bool SL, bool DL, bool GUARD>
+__global__ __launch_bounds__(FF_BLOCK) void k_tiles_f32c(
+    const double *__restrict__ spos, const double *__restrict__ sld,
+    const double *__restrict__ dld, long n_src, long spg, long n_groups,
+    const double *__restrict__ tpos, long n_trg, long tpg, int nsplit, float eps2, double scale,
+    float ratio, double *__restrict__ part) {
+  struct __align__(16) Rec {
+    float x[4], f[SL ? 4 : 1], q[DL ? 8 : 1];
+  };
+  __shared__ Rec sh[FF_TILE];
+  const long slice = blockIdx.x % nsplit, tb = blockIdx.x / nsplit;
+  const long t = tb * FF_BLOCK + threadIdx.x;
+  const bool tvalid = t < n_trg, grouped = spg > 0;
+  double tx = 0, ty = 0, tz = 0;
+  if (tvalid) {
+    tx = tpos[3 * t];
+    ty = tpos[3 * t + 1];
+    tz = tpos[3 * t + 2];
+  }
+  const long my_g = grouped && tvalid ? t / tpg : -1;
+  const long tfirst = tb * FF_BLOCK, tlast = min(tfirst + FF_BLOCK, n_trg) - 1;
+  // the group holding all the block's targets (or -1)
+  const long own_b = grouped && tfirst / tpg == tlast / tpg ? tfirst / tpg : -1;
+  Acc32 A = {{0, 0, 0}, {0, 0, 0}};
+  const long g0 = grouped ? slice * n_groups / nsplit : 0;
+  const long g1 = grouped ? (slice + 1) * n_groups / nsplit : 1;
+  for (long g = g0; g < g1; ++g) {
+    if (g == own_b) continue;  // block-uniform skip
+    const long sb = grouped ? g * spg : slice * n_src / nsplit;
+    const long se = grouped ? sb + spg : (slice + 1) * n_src / nsplit;
+    const bool lane_on = tvalid && my_g != g;
+    for (long c0 = sb; c0 < se; c0 += FF_TILE) {
+      const int cnt = (int)min((long)FF_TILE, se - c0);
+      __syncthreads();
+      const double *a = spos + 3 * c0;
+      if ((int)threadIdx.x < cnt) {
+        const long s = c0 + threadIdx.x;
+        Rec r;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) r.x[c] = (float)(spos[3 * s + c] - a[c]);
+        if constexpr (SL) {
+#pragma unroll
+          for (int c = 0; c < 3; ++c) r.f[c] = (float)sld[3 * s + c];
+        }
+        if constexpr (DL) {
+#pragma unroll
+          for (int c = 0; c < 6; ++c) r.q[c] = (float)dld[6 * s + c];
+        }
+        sh[threadIdx.x] = r;
+      }
+      __syncthreads();
+      if (!lane_on) continue;
+      const float lx = (float)(tx - a[0]), ly = (float)(ty - a[1]), lz = (float)(tz - a[2]);
+      for (int j0 = 0; j0 < cnt; j0 += FF_SUB) {
+        const int j1 = min(cnt, j0 + FF_SUB);
+        float S[3] = {0, 0, 0};
+#pragma unroll 4
+        for (int j = j0; j < j1; ++j) {
+          const float dx = lx - sh[j].x[0], dy = ly - sh[j].x[1], dz = lz - sh[j].x[2];
+          const float r2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
+          const float rq = rsqrt_pair(r2);
+          add_pair<SL, DL>(dx, dy, dz, GUARD ? (r2 > eps2 ? rq : 0.0f) : rq, sh[j].f, sh[j].q,
+                           ratio, S);
+        }
+        acc_merge(A, S);
+      }
+    }
+  }
+  if (tvalid) {
+    double *o = part + (slice * n_trg + t) * 3;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) o[c] = scale * ((double)A.h[c] + (double)A.l[c]);
+  }
+}
+
 // out[i] = the sum of the slices' partials: G threads per output add every
 // G-th slice, and their sums are added in order.
 template <int G>
@@ -493,9 +572,12 @@ __global__ __launch_bounds__(256) void k_sum_slices(const double *__restrict__ p
   }
 }
 static int sum_slices(const double *part, int nsplit, long n, double *out, hipStream_t st) {
-  // few slices: one coalesced 512-byte read per wave; many (few targets): 16
-  // threads share an output's chain of loads
-  if (nsplit >= 64)
+  // one or two slices (few sources): a thread per output; few: one coalesced
+  // 512-byte read per wave; many (few targets): 16 threads share an output's
+  // chain of loads
+  if (nsplit < 3)
+    k_sum_slices<1><<<cdiv(n, 256), 256, 0, st>>>(part, nsplit, n, out);
+  else if (nsplit >= 64)
     k_sum_slices<16><<<cdiv(n, 16), 256, 0, st>>>(part, nsplit, n, out);
   else
     k_sum_slices<4><<<cdiv(n, 64), 256, 0, st>>>(part, nsplit, n, out);
@@ -506,11 +588,16 @@ static int sum_slices(const double *part, int nsplit, long n, double *out, hipSt
 // or its last round leaves SIMDs idle: 32 waves per SIMD of the 256-CU part
 // (32 * 1024), as long as a slice keeps 128 sources (the partial sums are 48
 // bytes of traffic per slice and target); else 16 per SIMD in slices of at
-// least FF_PART sources.  Where the targets alone give less than 2048 waves,
-// the waves of a workgroup share their targets, which quarters the partial
-// sums; 1024 slices bound them where the targets are few.  Otherwise the
-// slices come in multiples of 8, one per XCD.  Parts of groups even out the
-// slices (about eight units each) unless there are many groups per slice.
+// least FF_PART sources.  Where the targets alone give less than 2048 waves
+// (1024 where the sources make fewer than four parts), the waves of a workgroup
+// share their targets, which quarters the partial sums; 1024 slices bound them
+// where the targets are few.  Otherwise the slices come in multiples of 8, one
+// per XCD, where there are sources for 8 (300 sources to 1,000,000 targets in
+// FP64: 251 us in two, 290 in eight); with shared targets they do on demand
+// (per_xcd), for sources past an L2 (both layers from 100,000 points, 9.6 MB, to
+// 10,000 in FP64: 1063 us, 1514 in 53 slices; not for fewer, 31,200 points in 100
+// groups, double layer, 846 -> 903 us).  Parts of groups even out the slices (about
+// eight units each) unless there are many groups per slice.
 // Measured: the far field of two vesicles (624 targets, 2404 sources) 10 us,
 // 348 us with whole groups per slice; 2400 points to themselves 14.5 us with
 // the sum, 22.7 us in slices of 256 sources.
@@ -518,23 +605,51 @@ struct Split {
   int nsplit;
   SliceMap map;
 };
-static Split choose_split(long n_trg, long n_groups, long spg, long max_slices = 1024) {
+static Split choose_split(long n_trg, long n_groups, long spg, long max_slices = 1024,
+                          bool per_xcd = false) {
   const long waves = (n_trg + 63) / 64, total = n_groups * spg;
-  const unsigned share = waves < 2048 ? 4 : 1;
+  const unsigned share = waves < (total < 128 ? 1024 : 2048) ? 4 : 1;
   const long w16 = (16 * 1024 + waves - 1) / waves, w32 = 2 * w16;
   long want = total / 128 >= w16 ? std::min(w32, total / 128) : std::min(w16, total / FF_PART);
-  if (share == 1) want = std::max(8L, (want + 7) / 8 * 8);
+  if (share == 1) want = total / 128 >= 8 ? std::max(8L, (want + 7) / 8 * 8) : total / 128;
+  else if (per_xcd && want >= 32) want = (want + 31) / 32 * 32;
   want = std::max(1L, std::min(want, max_slices * share));
   const long finest = (spg + FF_PART - 1) / FF_PART;
   const long nsub = n_groups >= 8 * want ? 1 : std::min((8 * want + n_groups - 1) / n_groups, finest);
   const long units = n_groups * nsub;
   long per = std::max(1L, units / want);
+  // (eight units a slice and more: rounded up leaves no slice short by much)
+  const bool xcds = per_xcd && share > 1 && want % 32 == 0 && units >= 8 * want;
+  if (xcds) per = (units + want - 1) / want;
   if ((units + per - 1) / per > max_slices * share) per = (units + want - 1) / want;
   const long slices = (units + per - 1) / per;
   Split s;
-  s.nsplit = (int)((slices + share - 1) / share);
+  s.nsplit = (int)(((xcds ? want : slices) + share - 1) / share);
   s.map = SliceMap{(unsigned)units, (unsigned)per, (unsigned)nsub, share};
   return s;
+}
+// Slices of k_tiles_f32c, at most one per group or tile (cells): a multiple of 8
+// (one per XCD), raised until the grid holds about 16 waves per SIMD.
+static Split tile_split(long n_trg, long cells, long max_slices) {
+  const long tblocks = (n_trg + FF_BLOCK - 1) / FF_BLOCK;
+  long ns = 8;
+  while (ns < 64 && tblocks * ns * (FF_BLOCK / 64) < 16 * 1024) ns *= 2;
+  ns = std::min({ns, cells, max_slices});
+  return Split{(int)ns, SliceMap{0, 0, 1, 1}};
+}
+// Where the FP32 form takes its sources through LDS tiles (k_tiles_f32c): no
+// packing launch for few sources, and in the single layer, whose guarded record
+// loop waits for scalar loads and the smallest distance, also where the targets
+// alone fill the chip or groups are short.  Us, tiles / records: single layer, 64
+// sources and 1000 targets 11.8 / 15.1; 300 and 10,000: 13.7 / 14.8, 1,000,000: 164 /
+// 247; 2400 and 130,000: 152 / 165; 20,000 and 100,000: 897 / 931; but 1000 and 1000
+// 18.7 / 14.6; groups of 12, 60,000 points 1839 / 2235, of 84, 21,000: 229 / 231, but of
+// 312, 31,200: 567 / 491; both layers, 64 and 1000: 12.0 / 15.0, 300 and 130,000: 38 /
+// 58, but 1000 and 1000 24.7 / 15.1, 20,000 and 100,000 1358 / 1253.
+static bool tiles32(size_t n_src, size_t n_trg, size_t spg, bool dl) {
+  if (spg > 0) return (!dl && spg <= 100) || (spg <= 64 && n_src * n_trg <= 2000000);
+  if (!dl) return n_src <= 512 || n_trg >= 20000;
+  return n_src <= 128 || (n_src <= 512 && n_trg >= (n_src > FF_TILE ? 24000 : 65536));
 }
 // Workgroups of a launch over n_trg targets.
 static dim3 split_grid(const Split &s, long n_trg) {
@@ -557,11 +672,18 @@ static int launch_pairs64(dim3 grid, hipStream_t st, const double *spos, const d
       (unsigned)sp.nsplit, eps2, SL ? csl : cdl, SL ? cdl / csl : 1.0, part);
   return launch_status();
 }
+// (rec null: through LDS tiles)
 template <bool SL, bool DL, bool GUARD>
 static int launch_pairs32(dim3 grid, hipStream_t st, const double *spos, const double *sld,
                           const double *dld, long n_src, long spg, unsigned ntile,
                           const double *tpos, long n_trg, long tpg, const Split &sp, double eps2,
                           double csl, double cdl, double *part, float *rec) {
+  if (!rec) {
+    k_tiles_f32c<SL, DL, GUARD><<<grid, FF_BLOCK, 0, st>>>(
+        spos, sld, dld, n_src, tpg > 0 ? spg : 0, tpg > 0 ? n_src / spg : 0, tpos, n_trg, tpg,
+        sp.nsplit, (float)eps2, SL ? csl : cdl, (float)(SL ? cdl / csl : 1.0), part);
+    return launch_status();
+  }
   k_pack_pairs32<SL, DL><<<cdiv(n_src, 256), 256, 0, st>>>(spos, sld, dld, n_src,
                                                            tpg > 0 ? spg : 0, rec);
   V3D_CHECK(launch_status());
@@ -599,16 +721,20 @@ static int far_eval(const double *spos, const double *sld, const double *dld,
     if (per_slice > part_cap) return VES3D_INVALID_PARAMETER;
     max_slices = std::min(max_slices, (long)(part_cap / per_slice));
   }
+  const size_t rec_n = 3 + (sld ? 3 : 0) + (dld ? 6 : 0);
+  const bool tiles = F32 && tiles32(n_src, n_trg, grouped ? spg : 0, dld != nullptr);
+  const bool per_xcd = !F32 && n_src * rec_n * sizeof(double) > (4u << 20);  // an L2
   const unsigned ntile = (unsigned)((sp + FF_TILE - 1) / FF_TILE);
-  const Split split = F32 ? choose_split((long)n_trg, n_groups * ntile, std::min(sp, (long)FF_TILE),
-                                         max_slices)
-                          : choose_split((long)n_trg, n_groups, sp, max_slices);
+  const Split split = tiles ? tile_split((long)n_trg, grouped ? n_groups : ntile, max_slices)
+                      : F32 ? choose_split((long)n_trg, n_groups * ntile,
+                                           std::min(sp, (long)FF_TILE), max_slices)
+                            : choose_split((long)n_trg, n_groups, sp, max_slices, per_xcd);
   double *part =
       part_fixed ? part_fixed : (double *)workspace(kWsFarPartial, split.nsplit * per_slice);
   if (!part) return VES3D_MEMORY_ERROR;
-  const size_t rec_n = 3 + (sld ? 3 : 0) + (dld ? 6 : 0);
-  float *rec = F32 ? (float *)workspace(kWsFarRecords, n_src * rec_n * sizeof(float)) : nullptr;
-  if (F32 && !rec) return VES3D_MEMORY_ERROR;
+  const bool packs = F32 && !tiles;
+  float *rec = packs ? (float *)workspace(kWsFarRecords, n_src * rec_n * sizeof(float)) : nullptr;
+  if (packs && !rec) return VES3D_MEMORY_ERROR;
   const dim3 grid = split_grid(split, (long)n_trg);
 #define V3D_PAIRS(SL, DL, G)                                                                     \
   V3D_CHECK(F32 ? (launch_pairs32<SL, DL, G>(grid, st, spos, sld, dld, (long)n_src, sp, ntile,   \
