@@ -191,6 +191,43 @@ def test_gpu_network_bf16_vs_oracle(hip, nin, w, B):
     pc.close()
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("nin,w,B", [(1152, 512, 4099), (320, 1024, 6145), (1152, 256, 8193)])
+def test_gpu_network_bf16_large_products(hip, nin, w, B):
+    """Products on 64 x 64 tiles against those of parts of the batch, on small
+    ones: the operands are the same bfloat16 values, the FP32 sums in another
+    order.  Rows of the output to 2e-3, the gradients (the parts' weighted by
+    their rows) to 5e-3, as above for a rounding tie; the loss to 1e-5."""
+    import torch
+    from ves3d_amd.implicit import LearnedPC
+    rng = np.random.default_rng(5)
+    pc = LearnedPC(nin, w, capacity=0, seed=3)
+    P = _params(nin, w, rng, scale=1.0 / np.sqrt(nin))
+    P[2] *= np.sqrt(nin / w)
+    P[4] *= np.sqrt(nin / w)
+    pc.set_params(torch.from_numpy(np.concatenate([p.reshape(-1) for p in P]).astype(np.float32))
+                  .cuda())
+    pc.set_activations("bf16")
+    Z, T = (torch.from_numpy(rng.standard_normal((B, nin)).astype(np.float32)).cuda()
+            for _ in range(2))
+    Y = pc.forward(Z)
+    loss, g = pc.loss_grad(Z, T)
+    ref, total, mean = torch.zeros_like(g, dtype=torch.float64), 0.0, 700
+    rows = []
+    for r0 in range(0, B, mean):
+        z, t = Z[r0:r0 + mean].contiguous(), T[r0:r0 + mean].contiguous()
+        rows.append(pc.forward(z))
+        lo, gr = pc.loss_grad(z, t)
+        ref += gr.double() * (z.shape[0] / B)
+        total += lo * z.shape[0] / B
+    err = lambda a, b: float((a - b).abs().max() / b.abs().max())
+    assert err(Y, torch.cat(rows)) < 2e-3
+    assert abs(loss - total) < 1e-5 * total
+    for off, size, _ in pc.layout():
+        assert err(g[off:off + size].double(), ref[off:off + size]) < 5e-3
+    pc.close()
+
+
 def test_stored_network_files():
     """The committed network: FP32 parameters of the p = 16, width 256
     layout, finite, and a record of the 200 plain-solve steps it was trained

@@ -88,6 +88,53 @@ def test_inner_precond_inverts_local_operator(hip):
     st.close()
 
 
+def test_precond_learned_large_products(hip):
+    """The odd part on 6656 vesicles, whose products take the 64 x 64 tiles,
+    against slices of 52, which take the small ones: every vesicle's row is its
+    own, the operands are the same bfloat16 values and the FP32 sums run in
+    another order: 2e-3 of the largest, as for a rounding tie above."""
+    nv, part, p, w = 6656, 52, 8, 1024
+    nc = p * (p + 2)
+    nin = 4 * nc
+    base = _ellipsoids(part, p, 0.1, seed=6)
+    shift = 40.0 * np.stack(np.meshgrid(*[np.arange(6)] * 3), -1).reshape(-1, 3)[:nv // part]
+    X = (base[None] + shift[:, None, :, None]).reshape(nv, 3, -1)
+    rng = np.random.default_rng(8)
+    flat = np.concatenate([rng.standard_normal((w, nin)).ravel() / np.sqrt(nin),
+                           0.1 * rng.standard_normal(w),
+                           rng.standard_normal((w, w)).ravel() / np.sqrt(w),
+                           0.1 * rng.standard_normal(w),
+                           rng.standard_normal((nin, w)).ravel() / np.sqrt(w),
+                           0.1 * rng.standard_normal(nin)]).astype(np.float32)
+    pc = I.LearnedPC(nin, w)
+    pc.set_params(torch.from_numpy(flat).cuda())
+    pc.set_activations("bf16")
+    U, S = rng.standard_normal((nv, 3 * nc)), rng.standard_normal((nv, nc))
+    off = np.cumsum([0] + [p + 1 - (j + 1) // 2 for j in range(2 * p)])
+    order_major = lambda r: np.concatenate([r[:, a:b].ravel() for a, b in zip(off, off[1:])])
+
+    def functions(y, n):
+        return np.concatenate([y[n * a:n * b].reshape(n, b - a) for a, b in zip(off, off[1:])], 1)
+
+    def apply(v0, n):
+        st = I.Stepper(n, p, dt=1e-3, shear_rate=1.0, precision=0, precond=2, near=False)
+        I.attach(st, pc, collect=False)
+        st.set_state(cu(X[v0:v0 + n]))
+        st.prepare()
+        x = np.concatenate([order_major(U[v0:v0 + n].reshape(3 * n, nc)),
+                            order_major(S[v0:v0 + n])])
+        y = st.precond_learned(cu(x)).cpu().numpy()
+        st.close()
+        return np.concatenate([functions(y[:3 * n * nc], 3 * n).reshape(n, -1),
+                               functions(y[3 * n * nc:], n)], 1)
+
+    print("learned precond nv=%d p=%d width=%d" % (nv, p, w), flush=True)
+    whole = apply(0, nv)
+    for v0 in (0, 64 * part, nv - part):
+        assert rel(whole[v0:v0 + part], apply(v0, part)) < 2e-3
+    pc.close()
+
+
 def test_precond_learned_vs_oracle(hip):
     nv, p = 3, 6
     X = _ellipsoids(nv, p, 0.1, seed=32)

@@ -188,6 +188,63 @@ struct GemmEpi {
   int ldt = 0;
 };
 
+// The epilogue of the 32 x 32 tile at (m0, n0): four consecutive columns of one
+// row per thread, value(h, row, column) the tile's sums (h = 1: row M + m).
+template <GemmOut OUT, typename V>
+__device__ __forceinline__ void finish_tile(int M, int N, int m0, int n0, const GemmEpi &e,
+                                            __bf16 (&sh)[32][34], long tile, V value) {
+  constexpr int NS = OUT == kOutOdd ? 2 : 1;
+  const int tid = threadIdx.x, tr = tid >> 3, tc = (tid & 7) * 4;
+  const int m = m0 + tr, n = n0 + tc;
+  const bool row = m < M;
+  const long o = (long)m * N + n;
+  double d2 = 0;
+  bf16x4 hv = {};
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    float v[NS];
+#pragma unroll
+    for (int h = 0; h < NS; ++h) v[h] = value(h, tr, tc + u);
+    if (!row || n + u >= N) continue;
+    if constexpr (OUT == kOutStore) {
+      e.C[o + u] = v[0];
+    } else if constexpr (OUT == kOutBias) {
+      e.C[o + u] = v[0] + e.bias[n + u];
+    } else if constexpr (OUT == kOutGelu) {
+      const float a = v[0] + e.bias[n + u];
+      if (e.C) e.C[o + u] = a;
+      hv[u] = (__bf16)gelu_f(a);
+    } else if constexpr (OUT == kOutGeluOdd) {
+      e.H[o + u] = (__bf16)gelu_f(v[0] + e.bias[n + u]);
+      e.H[(long)M * N + o + u] = (__bf16)gelu_f(-v[0] + e.bias[n + u]);
+    } else if constexpr (OUT == kOutOdd) {
+      e.C[o + u] = 0.5f * ((v[0] + e.bias[n + u]) - (v[NS - 1] + e.bias[n + u]));
+    } else if constexpr (OUT == kOutLoss) {
+      const float d = v[0] + e.bias[n + u] - e.T[o + u];
+      e.C[o + u] = d * e.invn;
+      hv[u] = (__bf16)(d * e.invn);
+      d2 += (double)d * d;
+    } else {
+      const float g = v[0] * gelu_g(e.P[o + u]);
+      e.C[o + u] = g;
+      hv[u] = (__bf16)g;
+    }
+  }
+  if constexpr (OUT == kOutGelu || OUT == kOutLoss || OUT == kOutBack) {
+    if (e.H && row && n < N) *(bf16x4 *)(e.H + o) = hv;  // N is a multiple of 8
+    if (e.HT) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) sh[tr][tc + u] = hv[u];
+      __syncthreads();
+      store_transposed(sh, m0, n0, N, e.ldt, e.HT);
+    }
+  }
+  if constexpr (OUT == kOutLoss) {
+    d2 = block_sum(d2);
+    if (tid == 0) e.part[tile] = d2;
+  }
+}
+
 // A workgroup computes a 32 x 32 tile; its four waves take every fourth slab
 // of 32 k and add their sums through LDS in wave order.  The operands go
 // straight from memory to the MFMA registers: lane l supplies row l % 16 of
@@ -256,58 +313,82 @@ __global__ __launch_bounds__(256) void k_gemm_bf16(int M, int N, int K,
 #pragma unroll
         for (int r = 0; r < 4; ++r) red[w][h][16 * i + 4 * lg + r][16 * j + li] = acc[h][i][j][r];
   __syncthreads();
-  // four consecutive columns of one row per thread
-  const int tr = tid >> 3, tc = (tid & 7) * 4;
-  const int m = m0 + tr, n = n0 + tc;
-  const bool row = m < M;
-  const long o = (long)m * N + n;
-  double d2 = 0;
-  bf16x4 hv = {};
-#pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    float v[NS];
+  finish_tile<OUT>(M, N, m0, n0, e, sh, (long)blockIdx.y * gridDim.x + blockIdx.x,
+                   [&](int h, int r, int c) {
+                     return ((red[0][h][r][c] + red[1][h][r][c]) + red[2][h][r][c]) +
+                            red[3][h][r][c];
+                   });
+}
+
+// The same for large products: a 64 x 64 tile, each wave 32 x 32 of it over all
+// of K, slabs of 32 k staged through LDS, so that an operand's row is read once
+// per 64 columns.  Bound: the operands' reads; the form above reads twice as much
+// (forward pass, 1152-1024-1024-1152, batch 4096: 103 us here, 208 there).
+// Workgroups reach the XCDs in turn: an XCD's take the column tiles of one row
+// tile one after the other, which then finds its A rows in that L2.
+template <GemmOut OUT>
+__global__ __launch_bounds__(256) void k_gemm_bf16_lds(int M, int N, int K,
+                                                       const __bf16 *__restrict__ A, long lda,
+                                                       const __bf16 *__restrict__ B, long ldb,
+                                                       const GemmEpi e) {
+  constexpr int NS = OUT == kOutOdd ? 2 : 1, kPitch = 40;
+  __shared__ __attribute__((aligned(16))) __bf16 As[NS][64][kPitch];
+  __shared__ __attribute__((aligned(16))) __bf16 Bs[64][kPitch];
+  __shared__ float sums[NS][64][65];
+  __shared__ __bf16 sh[32][34];
+  const int nt = (N + 63) / 64;
+  const long q = blockIdx.x / 8, m_tile = q / nt * 8 + blockIdx.x % 8;
+  if (m_tile >= (M + 63) / 64) return;
+  const int m0 = (int)m_tile * 64, n0 = (int)(q % nt) * 64;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int li = lane & 15, lg = lane >> 4, wm = (w >> 1) * 32, wn = (w & 1) * 32;
+  const int sr = tid >> 2, sk = (tid & 3) * 8;  // the vector that this thread stages
+  f32x4 acc[NS][2][2] = {};
+  for (int k0 = 0; k0 < K; k0 += 32) {
+    const bool in = k0 + sk < K;
 #pragma unroll
     for (int h = 0; h < NS; ++h)
-      v[h] = ((red[0][h][tr][tc + u] + red[1][h][tr][tc + u]) + red[2][h][tr][tc + u]) +
-             red[3][h][tr][tc + u];
-    if (!row || n + u >= N) continue;
-    if constexpr (OUT == kOutStore) {
-      e.C[o + u] = v[0];
-    } else if constexpr (OUT == kOutBias) {
-      e.C[o + u] = v[0] + e.bias[n + u];
-    } else if constexpr (OUT == kOutGelu) {
-      const float a = v[0] + e.bias[n + u];
-      if (e.C) e.C[o + u] = a;
-      hv[u] = (__bf16)gelu_f(a);
-    } else if constexpr (OUT == kOutGeluOdd) {
-      e.H[o + u] = (__bf16)gelu_f(v[0] + e.bias[n + u]);
-      e.H[(long)M * N + o + u] = (__bf16)gelu_f(-v[0] + e.bias[n + u]);
-    } else if constexpr (OUT == kOutOdd) {
-      e.C[o + u] = 0.5f * ((v[0] + e.bias[n + u]) - (v[NS - 1] + e.bias[n + u]));
-    } else if constexpr (OUT == kOutLoss) {
-      const float d = v[0] + e.bias[n + u] - e.T[o + u];
-      e.C[o + u] = d * e.invn;
-      hv[u] = (__bf16)(d * e.invn);
-      d2 += (double)d * d;
-    } else {
-      const float g = v[0] * gelu_g(e.P[o + u]);
-      e.C[o + u] = g;
-      hv[u] = (__bf16)g;
-    }
-  }
-  if constexpr (OUT == kOutGelu || OUT == kOutLoss || OUT == kOutBack) {
-    if (e.H && row && n < N) *(bf16x4 *)(e.H + o) = hv;  // N is a multiple of 8
-    if (e.HT) {
+      *(bf16x8 *)&As[h][sr][sk] =
+          in && m0 + sr < M
+              ? *(const bf16x8 *)(A + (m0 + sr + (long)h * M) * lda + k0 + sk)
+              : bf16x8{};
+    *(bf16x8 *)&Bs[sr][sk] =
+        in && n0 + sr < N ? *(const bf16x8 *)(B + (n0 + sr) * ldb + k0 + sk) : bf16x8{};
+    __syncthreads();
+    bf16x8 b[2];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) sh[tr][tc + u] = hv[u];
-      __syncthreads();
-      store_transposed(sh, m0, n0, N, e.ldt, e.HT);
+    for (int j = 0; j < 2; ++j) b[j] = *(const bf16x8 *)&Bs[wn + 16 * j + li][8 * lg];
+#pragma unroll
+    for (int h = 0; h < NS; ++h)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const bf16x8 a = *(const bf16x8 *)&As[h][wm + 16 * i + li][8 * lg];
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          acc[h][i][j] =
+              __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[j], acc[h][i][j], 0, 0, 0);
+      }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int h = 0; h < NS; ++h)
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          sums[h][wm + 16 * i + 4 * lg + r][wn + 16 * j + li] = acc[h][i][j][r];
+  __syncthreads();
+  const int mt32 = (M + 31) / 32;
+  for (int i = 0; i < 2; ++i)
+    for (int j = 0; j < 2; ++j) {
+      const int m = m0 + 32 * i, n = n0 + 32 * j;
+      if (m >= M || n >= N) continue;
+      finish_tile<OUT>(M, N, m, n, e, sh, (long)(n / 32) * mt32 + m / 32,
+                       [&](int h, int r, int c) { return sums[h][32 * i + r][32 * j + c]; });
+      __syncthreads();  // sh is read
     }
-  }
-  if constexpr (OUT == kOutLoss) {
-    d2 = block_sum(d2);
-    if (tid == 0) e.part[(long)blockIdx.y * gridDim.x + blockIdx.x] = d2;
-  }
 }
 
 template <GemmOut OUT>
@@ -318,6 +399,17 @@ int gemm_bf16(long M, int N, long K, const __bf16 *A, long lda, const __bf16 *B,
   if (((uintptr_t)A | (uintptr_t)B) & 15) return VES3D_INVALID_PARAMETER;
   const unsigned gy = cdiv(N, 32);
   if (M > 0x7fffff00L || gy > 65535) return VES3D_INVALID_PARAMETER;
+  // The LDS form where its tiles give every CU two workgroups and the operands'
+  // reads bound the product: forward pass 1152-512-512-1152, batch 4096 (512 tiles,
+  // 2.4e9 multiplications) 102 / 72 us, 2000 (256 tiles) 56 / 62; the weight
+  // gradients' few tiles (a quarter of these or less) take twice the time in it.
+  const long mt = cdiv(M, 64), nt = cdiv(N, 64);
+  if (mt * nt >= 512 && M * N * K >= 2000000000L) {
+    const long groups = (mt + 7) / 8 * 8 * nt;
+    if (groups > 0x7fffffffL) return VES3D_INVALID_PARAMETER;
+    k_gemm_bf16_lds<OUT><<<(unsigned)groups, 256, 0, st>>>((int)M, N, (int)K, A, lda, B, ldb, e);
+    return launch_status();
+  }
   k_gemm_bf16<OUT><<<dim3(cdiv(M, 32), gy), 256, 0, st>>>((int)M, N, (int)K, A, lda, B, ldb, e);
   return launch_status();
 }
