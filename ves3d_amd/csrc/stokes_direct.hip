@@ -184,8 +184,8 @@ __device__ __forceinline__ unsigned order_key(float x) { return __float_as_uint(
 constexpr int FF_RUN = 32;
 
 // n consecutive FP64 sources (positions p, densities f, (g, n) at q) at one
-// target, U at a time.  A lane with a bias keeps its sums (spans: the wave may
-// have such lanes).
+// target, U at a time.  A lane with a bias keeps its sums (spans: the wave has
+// such lanes).
 template <int U, bool SL, bool DL, bool GUARD>
 __device__ __forceinline__ void add_sources64(double tx, double ty, double tz, double bias,
                                               bool spans, int n, const double *__restrict__ p,
@@ -334,7 +334,6 @@ __global__ __launch_bounds__(FF_BLOCK) void k_pairs_f64(
   const double tx = tpos[3 * w.tc], ty = tpos[3 * w.tc + 1], tz = tpos[3 * w.tc + 2];
   double S[3] = {0, 0, 0};
   Slice k = slice_of(map, slice);
-  const bool spans = tpg > 0 && w.own < 0;
   constexpr int U = DL ? 2 : 4;
   while (k.u < k.u1) {
     // the slice's parts of group k.g, in one run
@@ -342,6 +341,7 @@ __global__ __launch_bounds__(FF_BLOCK) void k_pairs_f64(
     const long g = k.g, r0 = k.j * plen, n = min(take * plen, spg - r0), s0 = g * spg + r0;
     if (g != w.own) {  // wave-uniform skip
       const double bias = w.group == g ? kOwnGroupBias64 : 0.0;
+      const bool spans = __any(w.group == g);
       const double *__restrict__ p = spos + 3 * s0;
       const double *__restrict__ f = SL ? sld + 3 * s0 : p;
       const double *__restrict__ q = DL ? dld + 6 * s0 : p;
@@ -595,9 +595,10 @@ static int sum_slices(const double *part, int nsplit, long n, double *out, hipSt
 // per XCD, where there are sources for 8 (300 sources to 1,000,000 targets in
 // FP64: 251 us in two, 290 in eight); with shared targets they do on demand
 // (per_xcd), for sources past an L2 (both layers from 100,000 points, 9.6 MB, to
-// 10,000 in FP64: 1063 us, 1514 in 53 slices; not for fewer, 31,200 points in 100
-// groups, double layer, 846 -> 903 us).  Parts of groups even out the slices (about
-// eight units each) unless there are many groups per slice.
+// 10,000 in FP64: 1063 us, 1514 in 53 slices), if the last slice is filled too (48
+// groups of 1202 sources, 5.5 MB: 1058 us in 36 slices, 1206 in 36 of 40).  Parts of
+// groups even out the slices (about eight units each) unless there are many groups
+// per slice.
 // Measured: the far field of two vesicles (624 targets, 2404 sources) 10 us,
 // 348 us with whole groups per slice; 2400 points to themselves 14.5 us with
 // the sum, 22.7 us in slices of 256 sources.
@@ -612,19 +613,29 @@ static Split choose_split(long n_trg, long n_groups, long spg, long max_slices =
   const long w16 = (16 * 1024 + waves - 1) / waves, w32 = 2 * w16;
   long want = total / 128 >= w16 ? std::min(w32, total / 128) : std::min(w16, total / FF_PART);
   if (share == 1) want = total / 128 >= 8 ? std::max(8L, (want + 7) / 8 * 8) : total / 128;
-  else if (per_xcd && want >= 32) want = (want + 31) / 32 * 32;
   want = std::max(1L, std::min(want, max_slices * share));
   const long finest = (spg + FF_PART - 1) / FF_PART;
-  const long nsub = n_groups >= 8 * want ? 1 : std::min((8 * want + n_groups - 1) / n_groups, finest);
-  const long units = n_groups * nsub;
+  // units of `want` slices, about eight each
+  auto parts = [&](long want) {
+    return n_groups >= 8 * want ? 1 : std::min((8 * want + n_groups - 1) / n_groups, finest);
+  };
+  long nsub = parts(want), units = n_groups * nsub;
   long per = std::max(1L, units / want);
-  // (eight units a slice and more: rounded up leaves no slice short by much)
-  const bool xcds = per_xcd && share > 1 && want % 32 == 0 && units >= 8 * want;
-  if (xcds) per = (units + want - 1) / want;
   if ((units + per - 1) / per > max_slices * share) per = (units + want - 1) / want;
+  if (per_xcd && share > 1 && want >= 8 * share) {
+    // a multiple of 8 workgroup slices, if the units fill the last one too (an
+    // XCD with a slice less than the others waits for them)
+    const long w = std::min((want + 8 * share - 1) / (8 * share), max_slices / 8) * 8 * share;
+    const long s = parts(w), u = n_groups * s, p = (u + w - 1) / w;
+    if (w > 0 && u >= 8 * w && (u + p - 1) / p > w - share) {
+      nsub = s;
+      units = u;
+      per = p;
+    }
+  }
   const long slices = (units + per - 1) / per;
   Split s;
-  s.nsplit = (int)(((xcds ? want : slices) + share - 1) / share);
+  s.nsplit = (int)((slices + share - 1) / share);
   s.map = SliceMap{(unsigned)units, (unsigned)per, (unsigned)nsub, share};
   return s;
 }
