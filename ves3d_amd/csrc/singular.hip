@@ -1444,7 +1444,8 @@ int ves3d_hip_pole_kernel_shape(int p0, int p1, int *rows_host, int *threads_hos
   if (p0 < 1 || p1 < 1 || p0 > 128 || p1 > 255) return VES3D_INVALID_PARAMETER;
   const PoleShape ps =
       g_pole_fused.load(std::memory_order_relaxed) ? pole_fused_shape(p0, p1) : PoleShape();
-  if (rows_host) *rows_host = ps.kern ? 2 : 0;  // a latitude and its mirror
+  // a latitude and its mirror, or two pairs of them
+  if (rows_host) *rows_host = ps.kern ? 2 * pole_pairs(p1) : 0;
   if (threads_host) *threads_host = ps.kern ? kPtThreads : 0;
   if (workgroups_host) *workgroups_host = ps.blocks;
   return VES3D_SUCCESS;
