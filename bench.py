@@ -835,8 +835,8 @@ def main():
                     help="precision of the learned form: 1 FP32 singular operator + FP32-"
                          "compensated far field, 2 FP64 singular operator + FP32-compensated far field")
     ap.add_argument("--far-kernel", default="scalar", choices=sorted(FAR_KINDS),
-                    help="far field between vesicles: sources through the scalar cache (scalar2: "
-                         "two targets per lane in FP32) or LDS tiles")
+                    help="one-level far field between vesicles: the source levels' kernel (scalar, "
+                         "scalar2) or the all-pairs entry points' (lds)")
     ap.add_argument("--far-coarse", type=float, default=3.0,
                     help="learned form: two-level far field, p-grid sources for waves of "
                          "targets beyond this many vesicle radii (0: upsampled sources "

@@ -35,15 +35,33 @@ def _case(nv, p, seed, volfrac=0.05):
     return W.suspension(shapes, volfrac, seed=seed)
 
 
-@pytest.fixture(params=[1, 0, 2], ids=["far-scalar", "far-lds", "far-scalar2"])
+@pytest.fixture(params=[1, 0], ids=["far-levels", "far-pairs"])
 def far_kernel(request, hip):
-    """The kernels of the far field between vesicles (scalar-cache source
-    records; LDS-staged source tiles; scalar-cache records with two targets
-    per lane in the FP32 form)."""
+    """The kernels of the one-level far field between vesicles: those of the
+    source levels, and those of the all-pairs entry points."""
     from ves3d_amd import call
     call("ves3d_hip_set_far_kernel", request.param)
     yield request.param
     call("ves3d_hip_set_far_kernel", 1)
+
+
+@pytest.mark.parametrize("precision", [0, 2])
+def test_far_kernel_alias(hip, precision):
+    """Kind 2 of the far kernel is kind 1: the same bits."""
+    from ves3d_amd import call
+    X = _case(3, 8, seed=5)
+    y = {}
+    try:
+        for kind in (1, 2):
+            call("ves3d_hip_set_far_kernel", kind)
+            st = I.Stepper(3, 8, precision=precision)
+            st.set_state(cu(X))
+            st.prepare()
+            y[kind] = st.matvec(torch.ones(st.n, dtype=torch.float64, device="cuda"))
+            st.close()
+    finally:
+        call("ves3d_hip_set_far_kernel", 1)
+    assert torch.equal(y[1], y[2])
 
 
 @pytest.mark.parametrize("nv,p", [(2, 6), (3, 8)])

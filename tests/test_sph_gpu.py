@@ -88,44 +88,13 @@ def test_one_kernel_transforms(hip, p0, p1, N, dt, tol):
             out[tile] = [x.double() for x in synth + [a, t]]
     finally:
         call("ves3d_hip_set_gemm_tile", -1)
-    scale = max(float(x.abs().max()) for x in out[0][:4])
+    # each output to its own size; but the longitude derivative of order 1 at 0 and
+    # pi is zero up to the table's rounding of sin pi, and is held to a hundredth of
+    # the values, whose sums it shares
+    values = float(out[0][3].abs().max())
     for k, (x, y) in enumerate(zip(out[-1], out[0])):
-        err = float((x - y).abs().max()) / (scale if k < 4 else float(y.abs().max()))
+        err = float((x - y).abs().max()) / max(float(y.abs().max()), 0.01 * values if k == 1 else 0)
         assert err < tol, (k, err)
-
-
-@pytest.mark.parametrize("p0,p1,N", [(6, 6, 700), (8, 16, 300), (16, 32, 90), (24, 12, 200)])
-@pytest.mark.parametrize("dt,tol", [(torch.float64, 1e-12), (torch.float32, 1e-5)])
-def test_transforms_over_their_input(hip, p0, p1, N, dt, tol):
-    """Outputs that lie over the input, at its start and beside it: a transform
-    has read its input before it writes (every value; with derivatives only the
-    last output, the latitude derivative, may lie over the coefficients)."""
-    nc, ng = lambda p: p * (p + 2), lambda p: 2 * p * (p + 1)
-    S = torch.from_numpy(RNG.standard_normal((N, nc(p0)))).to("cuda", dt)
-    grid = lambda: torch.zeros((N, ng(p1)), dtype=dt, device="cuda")
-    X, Xt, Xp = grid(), grid(), grid()
-    G.shc2grid(S, N, p0, p1, X, Xt, Xp)
-    A, T = (torch.zeros((N, nc(p0)), dtype=dt, device="cuda") for _ in range(2))
-    G.grid2shc(Xt, N, p1, p0, A)
-    G.shc2grid_transpose(Xt, N, p1, p0, T)
-    err = lambda a, b: float((a - b).abs().max() / b.abs().max())
-    for shift in (0, 7, N * nc(p0) // 2):
-        def over(src, n_out):
-            buf = torch.zeros(src.numel() + n_out + 2 * shift, dtype=dt, device="cuda")
-            i = buf[shift:shift + src.numel()]
-            i.copy_(src.reshape(-1))
-            return i, buf[2 * shift:2 * shift + n_out]
-        i, o = over(S, N * ng(p1))
-        G.shc2grid(i, N, p0, p1, o)
-        assert err(o.reshape(N, -1), X) < tol
-        i, o = over(S, N * ng(p1))
-        t, x = grid(), grid()
-        G.shc2grid(i, N, p0, p1, x, t, o)
-        assert err(o.reshape(N, -1), Xp) < tol and err(x, X) < tol and err(t, Xt) < tol
-        for fn, ref in ((G.grid2shc, A), (G.shc2grid_transpose, T)):
-            i, o = over(Xt, N * nc(p0))
-            fn(i, N, p1, p0, o)
-            assert err(o.reshape(N, -1), ref) < tol
 
 
 @pytest.mark.parametrize("p0,p1,N", [
@@ -405,9 +374,9 @@ def test_self_apply_in_place(hip, p, nv, dt):
 
 @pytest.mark.parametrize("p0", [16, 8])
 def test_singular_build_fused_pole_stage(hip, p0):
-    """The FP64 build's fused pole kernel + transposed synthesis (the default
-    where p1 = 2 p0, p0 <= 16) against the separate kernel and grouped GEMMs,
-    SL and DL.  Asserts that the fused stage applies on this device."""
+    """The FP64 build's fused pole kernel, transposed synthesis and rotation (the
+    default where p1 is even, 12 to 32 and at least 2 p0) against the separate
+    kernels, SL and DL.  Asserts that the fused stage applies on this device."""
     import ctypes
     from ves3d_amd import call
     nv, p1, dt, tol = 3, 2 * p0, torch.float64, 1e-12
@@ -442,8 +411,8 @@ def test_singular_operator_block_symmetry(hip, p0, fused, dt):
     """The built SL and DL operators' 3 x 3 blocks of Ncoef x Ncoef satisfy
     B_ab = B_ba exactly (block (a, b) holds the rows of the symmetric tensor
     component c(a, b)), which the step's self apply relies on to read only
-    the blocks a <= b.  Fused FP64 build, separate FP64 build, and the FP32
-    build (p0 = 12 takes the separate path whatever the setting)."""
+    the blocks a <= b.  Fused FP64 build (two instances), separate FP64 build,
+    and the FP32 build."""
     from ves3d_amd import call
     nv = 2
     nc = p0 * (p0 + 2)

@@ -1,8 +1,8 @@
 // sht.hpp -- the SphericalHarmonics transforms on the GPU
-// (SHC2Grid, Grid2SHC, SHC2GridTranspose, SHC2Pole; src/SphericalHarmonics.cc:3-360)
-// expressed as two grouped GEMM launches each (Legendre stage per order,
-// Fourier stage as one dense product), with all re-layouts folded into the
-// operand strides.
+// (SHC2Grid, Grid2SHC, SHC2GridTranspose, SHC2Pole; src/SphericalHarmonics.cc:3-360):
+// one kernel each (sht_fused.hip) or two grouped GEMM launches (Legendre stage
+// per order, Fourier stage as one dense product, all re-layouts folded into the
+// operand strides), chosen by orders, type and number of functions.
 #pragma once
 #include "gemm.hpp"
 #include "sh_tables.hpp"
