@@ -97,6 +97,40 @@ def test_one_kernel_transforms(hip, p0, p1, N, dt, tol):
         assert err < tol, (k, err)
 
 
+@pytest.mark.parametrize("p0,p1,N", [(6, 6, 700), (8, 16, 300), (16, 32, 90), (24, 12, 200)])
+@pytest.mark.parametrize("dt,tol", [(torch.float64, 1e-12), (torch.float32, 1e-5)])
+def test_transforms_over_their_input(hip, p0, p1, N, dt, tol):
+    """Outputs that lie over the input, at its start and beside it: a transform
+    has read its input before it writes (every value; with derivatives only the
+    last output, the latitude derivative, may lie over the coefficients)."""
+    nc, ng = lambda p: p * (p + 2), lambda p: 2 * p * (p + 1)
+    S = torch.from_numpy(RNG.standard_normal((N, nc(p0)))).to("cuda", dt)
+    grid = lambda: torch.zeros((N, ng(p1)), dtype=dt, device="cuda")
+    X, Xt, Xp = grid(), grid(), grid()
+    G.shc2grid(S, N, p0, p1, X, Xt, Xp)
+    A, T = (torch.zeros((N, nc(p0)), dtype=dt, device="cuda") for _ in range(2))
+    G.grid2shc(Xt, N, p1, p0, A)
+    G.shc2grid_transpose(Xt, N, p1, p0, T)
+    err = lambda a, b: float((a - b).abs().max() / b.abs().max())
+    for shift in (0, 7, N * nc(p0) // 2):
+        def over(src, n_out):
+            buf = torch.zeros(src.numel() + n_out + 2 * shift, dtype=dt, device="cuda")
+            i = buf[shift:shift + src.numel()]
+            i.copy_(src.reshape(-1))
+            return i, buf[2 * shift:2 * shift + n_out]
+        i, o = over(S, N * ng(p1))
+        G.shc2grid(i, N, p0, p1, o)
+        assert err(o.reshape(N, -1), X) < tol
+        i, o = over(S, N * ng(p1))
+        t, x = grid(), grid()
+        G.shc2grid(i, N, p0, p1, x, t, o)
+        assert err(o.reshape(N, -1), Xp) < tol and err(x, X) < tol and err(t, Xt) < tol
+        for fn, ref in ((G.grid2shc, A), (G.shc2grid_transpose, T)):
+            i, o = over(Xt, N * nc(p0))
+            fn(i, N, p1, p0, o)
+            assert err(o.reshape(N, -1), ref) < tol
+
+
 @pytest.mark.parametrize("p0,p1,N", [
     (4, 4, 4095), (4, 4, 4096), (12, 12, 6143), (12, 12, 6144), (30, 20, 2047), (30, 20, 2048),
     (32, 32, 1279), (32, 32, 1280), (32, 32, 3071), (32, 32, 3072), (24, 12, 6143),
