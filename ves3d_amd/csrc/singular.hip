@@ -1115,11 +1115,14 @@ int singular_build(const double *X0, long Nv, int p0, int p1, T *SL, T *DL, hipS
   const bool fused = ps.kern != nullptr;
   // The FP32 form's transforms stay grouped GEMMs: the pole kernel subtracts
   // FP32 positions and raises the difference to r^-5, so that another order of
-  // their sums moves the operators by far more than it rounds (2.7e-4 between
-  // the two at order 24, 40 vesicles), and the one-kernel forms' came out
-  // further from 64 bits (8.9e-6 -> 1.1e-5 there).  The price: one-kernel
-  // transforms took 0.7 of the time for a few vesicles (order 16, two: 196 ->
-  // 148 us), 0.94 for 30 at order 24, 1.1 for 300 at order 10.
+  // their sums moves the operators by far more than it rounds (2.6e-4 between
+  // the two at order 24, 40 vesicles).  With the one-kernel forms the distance to
+  // the FP64 build went either way: the single layer's up at orders 12, 20 and 24
+  // (3.3e-6, 5.0e-6, 6.8e-6 -> 3.5e-6, 5.6e-6, 7.4e-6) and down at 6, 8 and 16
+  // (1.3e-6, 1.8e-6, 3.0e-6 -> 1.1e-6, 1.7e-6, 2.8e-6), the double layer's by 0.90
+  // to 1.05.  The price: one-kernel transforms took 0.7 of the time for a few
+  // vesicles (order 16, two: 196 -> 148 us), 0.94 for 30 at order 24, 1.1 for 300
+  // at order 10.
   const ShtForm form = std::is_same<T, float>::value ? ShtForm::kGrouped : ShtForm::kAuto;
   const long per = singular_elems_per_ves(p0, p1, fused);
   const long budget = (6L << 30) / (long)sizeof(T);
